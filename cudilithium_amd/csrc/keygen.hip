@@ -133,8 +133,8 @@ template <class P, int G>
 struct KgShared {
     ZetaLds zt;
     int32_t x[4][NTT_XBUF];
-    int32_t shat[G][P::L][N];
-    int32_t acc[G][P::K][N];
+    int32_t shat[G][P::L][LDS_ROW];
+    int32_t acc[G][P::K][LDS_ROW];
 };
 
 template <class P, int G>
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void kg_main_kernel(KeygenArgs a) {
     const size_t item0 = (size_t)blockIdx.x * G;
     const int wave = threadIdx.x >> 6;
     zeta_lds_load(sh.zt);
-    for (int j = threadIdx.x; j < G * P::K * N; j += blockDim.x) (&sh.acc[0][0][0])[j] = 0;
+    for (int j = threadIdx.x; j < G * P::K * LDS_ROW; j += blockDim.x) (&sh.acc[0][0][0])[j] = 0;
     __syncthreads();
 
     // NTT(s1) for the G keys

@@ -58,21 +58,41 @@ __device__ __forceinline__ uint32_t block_bits(const Lane64 (&s)[25]) {
     return v;
 }
 
+// The first four blocks hold 4 x 56 = 224 < N candidates, so only the later
+// ones test for the end of the polynomial; a candidate is rejected with
+// probability 1 - q / 2^23 = 0.001, so the fifth block nearly always ends it
+// after about 32 of its 56 candidates, and the wave leaves as soon as every
+// lane is done (tested every eight candidates).
 template <class Sink>
 __device__ __forceinline__ void uniform_poly(const uint64_t (&rho)[4], uint32_t nonce, Sink &&sink) {
     Lane64 s[25];
     const uint64_t in[5] = {rho[0], rho[1], rho[2], rho[3], (uint64_t)(nonce & 0xFFFF)};
     shake_absorb_regs<SHAKE128_RATE, SEEDBYTES + 2>(s, in);
+    constexpr int CAND = SHAKE128_RATE / 3, FREE_BLOCKS = (N - 1) / CAND;
+    static_assert(FREE_BLOCKS * CAND < N, "no end test needed in the free blocks");
     int ctr = 0;
-    do {
+#pragma unroll 1
+    for (int b = 0; b < FREE_BLOCKS; ++b) {
         keccak_f1600(s);
-        static_for<0, SHAKE128_RATE / 3>([&](auto c) {
-            constexpr int C = decltype(c)::value;
-            const uint32_t t = block_bits<24 * C, 23>(s);
-            if (t < (uint32_t)Q && ctr < N) {
+        static_for<0, CAND>([&](auto c) {
+            const uint32_t t = block_bits<24 * decltype(c)::value, 23>(s);
+            if (t < (uint32_t)Q) {
                 sink(ctr, (int32_t)t);
                 ++ctr;
             }
+        });
+    }
+    do {
+        keccak_f1600(s);
+        static_for<0, CAND / 8>([&](auto g) {
+            if (__ballot(ctr < N) == 0ull) return;
+            static_for<0, 8>([&](auto c) {
+                const uint32_t t = block_bits<24 * (8 * decltype(g)::value + decltype(c)::value), 23>(s);
+                if (t < (uint32_t)Q && ctr < N) {
+                    sink(ctr, (int32_t)t);
+                    ++ctr;
+                }
+            });
         });
     } while (ctr < N);
 }

@@ -113,8 +113,8 @@ template <class P, bool RES, int G>
 struct VfShared {
     ZetaLds zt;
     int32_t x[4][NTT_XBUF];
-    int32_t zhat[G][P::L][N];
-    int32_t acc[RES ? 1 : G][P::K][N];
+    int32_t zhat[G][P::L][LDS_ROW];
+    int32_t acc[RES ? 1 : G][P::K][LDS_ROW];
     int32_t chat[G][N];
     int32_t fail[G];
 };
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) void vf_main_kernel(VerifyArgs a) {
     const int wave = threadIdx.x >> 6;
     zeta_lds_load(sh.zt);
     if constexpr (!RES)
-        for (int j = threadIdx.x; j < G * P::K * N; j += blockDim.x) (&sh.acc[0][0][0])[j] = 0;
+        for (int j = threadIdx.x; j < G * P::K * LDS_ROW; j += blockDim.x) (&sh.acc[0][0][0])[j] = 0;
     if (threadIdx.x < G) {
         const size_t item = item0 + threadIdx.x;
         sh.fail[threadIdx.x] =
