@@ -26,6 +26,13 @@ __device__ __forceinline__ int32_t mont_mul_tw(int32_t b, int32_t z, int32_t zq)
     return __mulhi(b, z) - __mulhi(t, Q);
 }
 
+// 64-bit sum of products to its Montgomery-reduced value x * 2^-32 mod q:
+// |result| <= |x| / 2^32 + q / 2.
+__device__ __forceinline__ int32_t mont_reduce(int64_t x) {
+    const int32_t t = (int32_t)((uint32_t)x * QINV);
+    return (int32_t)(x >> 32) - __mulhi(t, Q);
+}
+
 // reduce.cuh:42-48: r == a (mod q), -6283009 <= r <= 6283007.
 __device__ __forceinline__ int32_t reduce32(int32_t a) {
     int32_t t = (a + (1 << 22)) >> 23;

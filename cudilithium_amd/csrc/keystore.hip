@@ -5,8 +5,8 @@
 // t0 on every signature (sign.cu:306-403).  For keys that stay resident
 // these depend only on the key, so they are computed once here:
 //   ks_expand  lane per A entry   A[k][l] = RejUniform(SHAKE128(rho||l||k))
-//   ks_prep    wave per poly      s1^, s2^, t0^ (with the secret key) and
-//                                 t1^ = NTT(t1 << d) from the public key
+//   ks_prep    wave per poly      s2, s1, t0 limbs as int8 (with the secret
+//                                 key) and t1^ = NTT(t1 << d) from the public key
 //   ks_tr      lane per key       tr = SHAKE256(pk)[0:32], flags
 // rho is read from the public key (its first 32 bytes equal the secret
 // key's), so verify-only keys expand without a secret key.
@@ -56,12 +56,15 @@ __global__ __launch_bounds__(64 * KS_WAVES) void ks_prep_kernel(SignArgs a, int 
         const int p = (int)(t % NP);
         if (p < NS) {
             if (with_sk) {
-                stage_prep<P>(a, i, p, x[w], zt);
+                if (lane_id() < N / 8)
+                    stage_prep<P>(a.sk + i * a.sk_pitch,
+                                  reinterpret_cast<int8_t *>(a.rows + i * a.row_pitch + KY::S8), p, lane_id());
             } else {
-                // a verify-only key holds no secret: its s1^ / s2^ / t0^ rows are
-                // cleared so that nothing of a row's previous key survives
+                // a verify-only key holds no secret: its s8 area (and the rest of
+                // the space up to t1^) is cleared so that nothing of a row's
+                // previous key survives
                 const int32_t zero[4] = {0, 0, 0, 0};
-                wave_store_D(reinterpret_cast<int32_t *>(a.rows + i * a.row_pitch + KY::S1H) + p * N, zero);
+                wave_store_D(reinterpret_cast<int32_t *>(a.rows + i * a.row_pitch + KY::S8) + p * N, zero);
             }
             continue;
         }

@@ -52,12 +52,12 @@ struct SignLayout {
     static constexpr size_t SLOT = MU + 256;
     static constexpr size_t M = SLOT + SL::BYTES;
     static size_t ints(size_t mlen) { return M + align256(mlen); }
-    // int32 arrays after the message: A (K*L), s1hat (L), s2hat (K), t0hat (K)
+    // after the message: A (K*L int32 polynomials), then s2, s1 and t0's limbs
+    // as int8 ((L + 3K) * N bytes of the (L + 2K) * N * 4 kept for them)
     static size_t mat(size_t mlen) { return ints(mlen); }
-    static size_t s1hat(size_t mlen) { return mat(mlen) + (size_t)P::K * P::L * N * 4; }
-    static size_t s2hat(size_t mlen) { return s1hat(mlen) + (size_t)P::L * N * 4; }
-    static size_t t0hat(size_t mlen) { return s2hat(mlen) + (size_t)P::K * N * 4; }
-    static size_t row(size_t mlen) { return t0hat(mlen) + (size_t)P::K * N * 4; }
+    static size_t s8(size_t mlen) { return mat(mlen) + (size_t)P::K * P::L * N * 4; }
+    static size_t row(size_t mlen) { return s8(mlen) + (size_t)(P::L + 2 * P::K) * N * 4; }
+    static_assert((P::L + 3 * P::K) * N <= (P::L + 2 * P::K) * N * 4, "int8 polynomials fit");
     // reference formula (test_vectors.cu:81-100)
     static size_t ref_row(size_t mlen) {
         return align256(Z::SIG_BYTES) + align256(Z::SK_BYTES) + align256(SEEDBYTES) + align256(SEEDBYTES + mlen) +
@@ -104,14 +104,14 @@ struct VerifyLayout {
 };
 
 // FLAGS word of a resident key: set when the key was loaded or generated
-// with its secret key (verify-only keys hold zeros in SK, s1^, s2^, t0^)
+// with its secret key (verify-only keys hold zeros in SK and the s8 area)
 constexpr uint32_t KEY_HAS_SECRET = 1u;
 
 // One resident key of a key store: public key, secret key (absent for
 // verify-only keys), tr = H(pk), and the expanded arrays every signature and
 // verification under the key would otherwise recompute: A = ExpandA(rho)
-// (K*L polys, 5*K*L Keccak permutations), s1^, s2^, t0^ (NTT domain) and
-// t1^ = NTT(t1 * 2^d), int32 in the NTT kernels' register layout.
+// (K*L polys, 5*K*L Keccak permutations), s2, s1 and t0's limbs as int8 and
+// t1^ = NTT(t1 * 2^d); A and t1^ int32 in the NTT kernels' register layout.
 template <class P>
 struct KeyLayout {
     using Z = Sizes<P>;
@@ -121,10 +121,8 @@ struct KeyLayout {
     static constexpr size_t FLAGS = TR + SEEDBYTES;           // KEY_HAS_SECRET or 0 (verify-only)
     static constexpr size_t INTS = TR + 256;
     static constexpr size_t MAT = INTS;
-    static constexpr size_t S1H = MAT + (size_t)P::K * P::L * N * 4;
-    static constexpr size_t S2H = S1H + (size_t)P::L * N * 4;
-    static constexpr size_t T0H = S2H + (size_t)P::K * N * 4;
-    static constexpr size_t T1H = T0H + (size_t)P::K * N * 4;
+    static constexpr size_t S8 = MAT + (size_t)P::K * P::L * N * 4;
+    static constexpr size_t T1H = S8 + (size_t)(P::L + 2 * P::K) * N * 4;
     static constexpr size_t ROW = T1H + (size_t)P::K * N * 4;
     // keygen into the store uses the (not yet expanded) int area as scratch
     static_assert(KeypairLayout<P>::ROW - KeypairLayout<P>::SCRATCH <= ROW - INTS, "keygen scratch fits");

@@ -47,17 +47,16 @@ __global__ __launch_bounds__(256) void sg_expand_kernel(SignArgs a) {
     stage_expand_a<P>(a, t / KL, e / P::L, e % P::L);
 }
 
+// secret key to int8 polynomials, 8 coefficients per lane
 template <class P>
-__global__ __launch_bounds__(64 * SIGN_WAVES) void sg_prep_kernel(SignArgs a) {
-    constexpr int NP = P::L + 2 * P::K;
-    __shared__ ZetaLds zt;
-    __shared__ int32_t x[SIGN_WAVES][NTT_XBUF];
-    zeta_lds_load(zt);
-    __syncthreads();
-    const int w = threadIdx.x >> 6;
-    const size_t total = a.n * NP, stride = (size_t)gridDim.x * SIGN_WAVES;
-    for (size_t t = (size_t)blockIdx.x * SIGN_WAVES + w; t < total; t += stride)
-        stage_prep<P>(a, t / NP, (int)(t % NP), x[w], zt);
+__global__ __launch_bounds__(256) void sg_prep_kernel(SignArgs a) {
+    constexpr int PER = (P::L + 2 * P::K) * (N / 8);
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= a.n * PER) return;
+    const size_t i = t / PER;
+    const int u = (int)(t % PER);
+    int8_t *dst = reinterpret_cast<int8_t *>(a.rows + i * a.row_pitch + a.off_ints) + P::K * P::L * N * 4;
+    stage_prep<P>(a.sk + i * a.sk_pitch, dst, u / (N / 8), u % (N / 8));
 }
 
 // exec entry e = (item << 16) | nonce (api.cu:221-230)
@@ -100,15 +99,12 @@ __global__ __launch_bounds__(256) void sg_c_kernel(SignArgs a, SlotRef sr, const
 template <class P>
 __global__ __launch_bounds__(64 * SIGN_WAVES) void sg_z_kernel(SignArgs a, SlotRef sr, const uint32_t *exec,
                                                                size_t nslot, int by_item, uint8_t *done) {
-    __shared__ ZetaLds zt;
-    __shared__ int32_t x[SIGN_WAVES][NTT_XBUF];
-    zeta_lds_load(zt);
-    __syncthreads();
+    __shared__ ZScratch<P> zs[SIGN_WAVES];
     const int w = threadIdx.x >> 6;
     for (size_t s = (size_t)blockIdx.x * SIGN_WAVES + w; s < nslot; s += (size_t)gridDim.x * SIGN_WAVES) {
         const size_t item = exec[s] >> 16;
         const size_t r = by_item ? item : s;
-        const bool ok = stage_z<P>(a, item, sr.base + r * sr.pitch, sr.sig + r * sr.sig_pitch, x[w], zt);
+        const bool ok = stage_z<P>(a, item, sr.base + r * sr.pitch, sr.sig + r * sr.sig_pitch, zs[w]);
         if (lane_id() == 0) done[s] = ok ? 1 : 0;
     }
 }
@@ -158,7 +154,7 @@ int sign_key_check_impl(const SignArgs &a, uint32_t *status, hipStream_t st) {
 template <class P>
 int sign_fixed_impl(const SignArgs &a, hipStream_t st) {
     if (a.n == 0) return 0;
-    constexpr int KL = P::K * P::L, NP = P::L + 2 * P::K;
+    constexpr int KL = P::K * P::L, PREP = (P::L + 2 * P::K) * (N / 8);
     auto mu = [&](hipStream_t s) -> int {
         if (a.row_mu) return launch_sign_mu_row(P::MODE, a, s);
         // two lanes per item by default: fixed stage of 16,384 Dilithium3
@@ -173,7 +169,7 @@ int sign_fixed_impl(const SignArgs &a, hipStream_t st) {
             hipLaunchKernelGGL(sg_mu_kernel<P>, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a);
         return (int)hipGetLastError();
     };
-    if (a.key_idx) return mu(st);  // resident keys carry A, s1^, s2^, t0^ already: only mu / rhoprime
+    if (a.key_idx) return mu(st);  // resident keys carry A, s1, s2, t0 already: only mu / rhoprime
     // Batches below DIL_FIXED_FORK_MIN items run the three launches in order
     // on the caller's stream.  Off by default: for one caller the fork is
     // faster (1,024 / 4,096 items: 1.76 / 1.83 ms against 1.86 / 2.07 ms);
@@ -185,8 +181,7 @@ int sign_fixed_impl(const SignArgs &a, hipStream_t st) {
     if (a.n < (size_t)DIL_FIXED_FORK_MIN) {
         int e;
         if ((e = mu(st))) return e;
-        hipLaunchKernelGGL(sg_prep_kernel<P>, dim3(default_grid_blocks(a.n * NP, SIGN_WAVES)), dim3(64 * SIGN_WAVES),
-                           0, st, a);
+        hipLaunchKernelGGL(sg_prep_kernel<P>, dim3((unsigned)((a.n * PREP + 255) / 256)), dim3(256), 0, st, a);
         hipLaunchKernelGGL(sg_expand_kernel<P>, dim3((unsigned)((a.n * KL + 255) / 256)), dim3(256), 0, st, a);
         return (int)hipGetLastError();
     }
@@ -198,8 +193,7 @@ int sign_fixed_impl(const SignArgs &a, hipStream_t st) {
     if ((e = (int)hipStreamWaitEvent(aux->s[0], aux->fork, 0))) return e;
     if ((e = (int)hipStreamWaitEvent(aux->s[1], aux->fork, 0))) return e;
     if ((e = mu(aux->s[0]))) return e;
-    hipLaunchKernelGGL(sg_prep_kernel<P>, dim3(default_grid_blocks(a.n * NP, SIGN_WAVES)), dim3(64 * SIGN_WAVES), 0,
-                       aux->s[1], a);
+    hipLaunchKernelGGL(sg_prep_kernel<P>, dim3((unsigned)((a.n * PREP + 255) / 256)), dim3(256), 0, aux->s[1], a);
     hipLaunchKernelGGL(sg_expand_kernel<P>, dim3((unsigned)((a.n * KL + 255) / 256)), dim3(256), 0, st, a);
     if ((e = (int)hipGetLastError())) return e;
     if ((e = (int)hipEventRecord(aux->join[0], aux->s[0]))) return e;

@@ -72,7 +72,11 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
     // the w stage does not pair for L = 7)
     constexpr bool W_Y_LDS = P::L >= DIL_W_Y_LDS_MIN_L && WPE <= 2;
     constexpr bool W_PAIRS = P::L < DIL_W_Y_LDS_MIN_L || W_Y_LDS;
-    __shared__ int32_t ylds[W_Y_LDS ? PERSIST_THREADS / 64 : 1][W_Y_LDS ? 2 * P::L * N : 1];
+    union StageLds {
+        int32_t y[W_Y_LDS ? 2 * P::L * N : 1];  // w stage
+        ZScratch<P> z;                          // z stage
+    };
+    __shared__ StageLds stage_lds[PERSIST_THREADS / 64];
     __shared__ uint32_t own_item[S], own_next[S];
     __shared__ int own_done[S];
     __shared__ uint32_t slot_own[S], slot_nonce[S];
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
             if (s + u < S) {
                 if constexpr (W_PAIRS) {
                     uint8_t *const pair[2] = {slot_base(s), slot_base(s + u)};
-                    stage_w_multi<P, 2>(a, item, pair, x[wave], zt, ylds[W_Y_LDS ? wave : 0]);
+                    stage_w_multi<P, 2>(a, item, pair, x[wave], zt, stage_lds[wave].y);
                     continue;
                 } else {
                     stage_w<P>(a, item, slot_base(s + u), x[wave], zt);
@@ -227,7 +231,7 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
             const size_t item = own_item[o];
             uint8_t *dst = a.sig + item * a.sig_pitch;
             for (int s = o; s < S; s += u) {
-                if (stage_z<P>(a, item, slot_base(s), dst, x[wave], zt)) {
+                if (stage_z<P>(a, item, slot_base(s), dst, stage_lds[wave].z)) {
                     const uint8_t *src = slot_sig(s);
                     if (lane < SEEDBYTES) dst[lane] = src[lane];
                     if (lane == 0) {

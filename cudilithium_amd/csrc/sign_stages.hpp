@@ -5,12 +5,13 @@
 // Fixed part per item (api.cu:117-182):
 //   mu = SHAKE256(tr || m), rhoprime = SHAKE256(key || mu)   lane per item
 //   A = ExpandA(rho)                                         lane per entry
-//   s1^, s2^, t0^ = NTT(unpack(sk))                          wave per poly
+//   s2 | s1 and the limbs of t0 as int8 (unpack of sk)        lane per 8 coefficients
 // One attempt (item, nonce) in a "slot" (sign.cu:463-1196):
 //   y    lane per (slot, l)   raw ExpandMask squeeze of rhoprime || L*nonce+l
 //   w    wave per slot        NTT(y), A y^, INTT, caddq -> w; pack w1
 //   c    lane per slot        c~ = SHAKE256(mu || w1), c = SampleInBall(c~)
-//   z    wave per slot        z = y + INTT(c^ s1^) and the three norm checks,
+//   z    wave per slot        c s2, c s1, c t0 on the matrix cores
+//                             (ringmul.hpp), the norm checks, z = y + c s1,
 //                             MakeHint, pack z and h
 #pragma once
 
@@ -19,6 +20,7 @@
 #include "layout.hpp"
 #include "pipelines.hpp"
 #include "poly.hpp"
+#include "ringmul.hpp"
 #include "sample.hpp"
 
 namespace dil {
@@ -31,11 +33,11 @@ struct SignArgs {
     MsgRef m;
     uint8_t *rows;  // SignLayout rows (item state)
     size_t row_pitch;
-    size_t off_ints;  // byte offset of the int32 arrays (A, s1^, s2^, t0^) in a row
+    size_t off_ints;  // byte offset of the expanded arrays (A, then s2 | s1 | t0 limbs as int8) in a row
     size_t n;
     // Resident keys (optional): when key_idx is set, item i signs with key
     // k = min(key_idx[i], nkeys - 1); its secret key is sk + k * sk_pitch and
-    // its expanded arrays (A, s1^, s2^, t0^) sit at key_ints + k * key_pitch
+    // its expanded arrays (A, s2, s1, t0) sit at key_ints + k * key_pitch
     // instead of in the item's row.  (Out-of-range indices are clamped so
     // that no access leaves the store.)
     const uint32_t *key_idx;
@@ -70,14 +72,15 @@ struct ItemView {
     using Z = Sizes<P>;
     using SLy = SignLayout<P>;
     uint8_t *row;
-    const int32_t *mat, *s1h, *s2h, *t0h;
+    const int32_t *mat;
+    const int8_t *s8;  // s2 (K polynomials) | s1 (L)
+    const int8_t *t8;  // t0's low limbs (K) | high limbs (K)
     __device__ ItemView(const SignArgs &a, size_t item) {
         row = a.rows + item * a.row_pitch;
         mat = a.key_idx ? reinterpret_cast<const int32_t *>(a.key_ints + sk_index(a, item) * a.key_pitch)
                         : reinterpret_cast<const int32_t *>(row + a.off_ints);
-        s1h = mat + P::K * P::L * N;
-        s2h = s1h + P::L * N;
-        t0h = s2h + P::K * N;
+        s8 = reinterpret_cast<const int8_t *>(mat + P::K * P::L * N);
+        t8 = s8 + (P::K + P::L) * N;
     }
 };
 
@@ -192,25 +195,43 @@ __device__ __forceinline__ void stage_expand_a(const SignArgs &a, size_t i, int 
     });
 }
 
-// poly p of the item: s1[0..L), s2[0..K), t0[0..K) -> NTT domain (layout D)
+// Coefficients 8c .. 8c + 7 (c < 32) of poly p of the item's secret key as
+// int8, for the products with the challenge: p < L: s1[p], p < L + K: s2,
+// else t0, whose 13-bit coefficients become a low limb in [-64, 64) and a
+// high limb, t0 = lo + 128 hi.  dst: the item's s8 area (ItemView).
 template <class P>
-__device__ __forceinline__ void stage_prep(const SignArgs &a, size_t i, int p, int32_t *x, const ZetaLds &zt) {
+__device__ __forceinline__ void stage_prep(const uint8_t *sk, int8_t *dst, int p, int c) {
     using Z = Sizes<P>;
-    const uint8_t *sk = a.sk + i * a.sk_pitch;
-    int32_t *dst = reinterpret_cast<int32_t *>(a.rows + i * a.row_pitch + a.off_ints) + (P::K * P::L + p) * N;
-    int32_t v[4];
-    uint32_t f[4];
+    uint32_t lo[2] = {0, 0}, hi[2] = {0, 0};
     if (p < P::L + P::K) {
-        wave_fields_A<Z::ETA_BITS>(f, sk + Z::SK_S1 + p * Z::POLYETA_BYTES);
+        const uint8_t *src = sk + Z::SK_S1 + p * Z::POLYETA_BYTES + c * Z::ETA_BITS;
+        uint32_t v;
+        if constexpr (Z::ETA_BITS == 4)
+            v = load_any<uint32_t>(src);
+        else
+            v = load_any<uint16_t>(src) | (uint32_t)src[2] << 16;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = P::ETA - (int32_t)f[r];
+        for (int j = 0; j < 8; ++j) {
+            const int32_t x = P::ETA - (int32_t)((v >> (j * Z::ETA_BITS)) & ((1u << Z::ETA_BITS) - 1u));
+            lo[j >> 2] |= ((uint32_t)x & 0xFFu) << (8 * (j & 3));
+        }
+        const int row = p < P::L ? P::K + p : p - P::L;
+        *reinterpret_cast<uint2 *>(dst + row * N + 8 * c) = make_uint2(lo[0], lo[1]);
     } else {
-        wave_fields_A<13>(f, sk + Z::SK_T0 + (p - P::L - P::K) * POLYT0_BYTES);
+        const int k = p - P::L - P::K;
+        const uint8_t *src = sk + Z::SK_T0 + k * POLYT0_BYTES + c * 13;
+        const uint64_t a = load_any<uint64_t>(src), b = load_any<uint64_t>(src + 5);  // bits 0.., 40..
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (1 << (D - 1)) - (int32_t)f[r];
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t f = (uint32_t)(j < 4 ? a >> (13 * j) : b >> (13 * j - 40)) & 0x1FFFu;
+            const int32_t x = (1 << (D - 1)) - (int32_t)f, h = (x + 64) >> 7;
+            lo[j >> 2] |= ((uint32_t)(x - 128 * h) & 0xFFu) << (8 * (j & 3));
+            hi[j >> 2] |= ((uint32_t)h & 0xFFu) << (8 * (j & 3));
+        }
+        int8_t *t8 = dst + (P::K + P::L) * N;
+        *reinterpret_cast<uint2 *>(t8 + k * N + 8 * c) = make_uint2(lo[0], lo[1]);
+        *reinterpret_cast<uint2 *>(t8 + (P::K + k) * N + 8 * c) = make_uint2(hi[0], hi[1]);
     }
-    ntt_wave(v, x, zt);
-    wave_store_D(dst, v);
 }
 
 // ------------------------------------------------------------- attempt part
@@ -242,6 +263,21 @@ __device__ __forceinline__ void load_y_A(int32_t (&v)[4], const uint8_t *slot, i
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = P::GAMMA1 - (int32_t)f[r];
 }
+
+template <class P>
+__device__ __forceinline__ void load_y_D(int32_t (&v)[4], const uint8_t *slot, int l) {
+    using Z = Sizes<P>;
+    uint32_t f[4];
+    wave_fields_D<Z::Z_BITS>(f, slot + SlotLayout<P>::YRAW + l * Z::YRAW_BYTES);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = P::GAMMA1 - (int32_t)f[r];
+}
+
+// One coefficient's decomposition in a word of the slot's w area: high bits
+// above bit 20, low bits (|w0| <= gamma2 < 2^19) below.
+__device__ __forceinline__ uint32_t pack_w(int32_t w1, int32_t w0) { return (uint32_t)w1 << 20 | ((uint32_t)w0 & 0xFFFFFu); }
+__device__ __forceinline__ int32_t packed_w0(uint32_t p) { return (int32_t)(p << 12) >> 12; }
+__device__ __forceinline__ uint32_t packed_w1(uint32_t p) { return p >> 20; }
 
 // w for M attempts of the same item (slots[0..M)) in one wave: every A row
 // is loaded once for all M products, and the M transforms give the wave
@@ -282,6 +318,10 @@ __device__ __forceinline__ void stage_w_multi(const SignArgs &a, size_t item, ui
             }
         }
     for (int k = 0; k < P::K; ++k) {
+        // the L products of a coefficient are summed in 64 bits (one
+        // v_mad_i64_i32 each) and reduced once; |sum| < 7 q 2^26.1 < 2^53, so
+        // the reduced sum is below q / 2 + 2^21 and the INTT cannot overflow
+        int64_t sum[M][4];
         int32_t acc[M][4];
         int32_t ac[P::L][4];
 #pragma unroll
@@ -295,31 +335,31 @@ __device__ __forceinline__ void stage_w_multi(const SignArgs &a, size_t item, ui
 #pragma unroll
         for (int j = 0; j < M; ++j) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[j][r] = 0;
+            for (int r = 0; r < 4; ++r) sum[j][r] = 0;
 #pragma unroll
             for (int l = 0; l < P::L; ++l) {
                 if constexpr (Y_LDS) {
                     int32_t yv[4];
                     wave_load_D(yv, ylds + (j * P::L + l) * N);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[j][r] += mont_mul(ac[l][r], yv[r]);
+                    for (int r = 0; r < 4; ++r) sum[j][r] += (int64_t)ac[l][r] * yv[r];
                 } else {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[j][r] += mont_mul(ac[l][r], yh[j][l][r]);
+                    for (int r = 0; r < 4; ++r) sum[j][r] += (int64_t)ac[l][r] * yh[j][l][r];
                 }
             }
         }
 #pragma unroll
         for (int j = 0; j < M; ++j) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[j][r] = reduce32(acc[j][r]);
+            for (int r = 0; r < 4; ++r) acc[j][r] = mont_reduce(sum[j][r]);
             intt_wave(acc[j], x, zt);
             int32_t w1[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                acc[j][r] = caddq(acc[j][r]);
                 int32_t w0;
-                w1[r] = decompose<P>(acc[j][r], w0);
+                w1[r] = decompose<P>(caddq(acc[j][r]), w0);
+                acc[j][r] = (int32_t)pack_w(w1[r], w0);
             }
             wave_store_A(reinterpret_cast<int32_t *>(slots[j] + SL::W) + k * N, acc[j]);
             layout_A_to_D(w1, x);
@@ -391,103 +431,105 @@ __device__ __forceinline__ void stage_c_pair(const SignArgs &a, size_t item, uin
         challenge<P::TAU>(ct, reinterpret_cast<uint32_t *>(slot + SL::CP), h == 0);
 }
 
+// One wave's LDS area in the z stage: the challenge's operand table and the
+// rows c s2 (K) | c s1 (L); the rows c t0 (low limbs K, high limbs K) take
+// the place of c s1 once z is written.
+template <class P>
+struct ZScratch {
+    static constexpr int ROWS = P::K + (P::L > 2 * P::K ? P::L : 2 * P::K);
+    uint32_t toep[TOEP_WORDS];
+    uint16_t rows[ROWS * RING_ROW];
+};
+
 // Returns true (wave-uniform) when the attempt passes every check; then
 // sig_out holds the complete signature.  An attempt is accepted iff all of
-// ||r0|| < gamma2 - beta, ||c t0|| < gamma2, #hints <= omega and
-// ||z|| < gamma1 - beta hold (sign.cu:986-1196), so the order of the checks
-// does not change any result; the r0 check runs first because it rejects
-// most often (about 2/3 of Dilithium3 attempts), then c t0 and the hints,
-// then z.  Fields of a rejected attempt's sig_out are left partly written.
+// ||r0|| < gamma2 - beta, ||z|| < gamma1 - beta, ||c t0|| < gamma2 and
+// #hints <= omega hold (sign.cu:986-1196), so the order of the checks does
+// not change any result: c s2 and c s1 come from one set of matrix products,
+// r0 is checked first because it rejects most often (about 2/3 of Dilithium3
+// attempts), then z, and only the remaining fifth computes c t0 and the
+// hints.  All values are exact integers below q / 2, where the reference's
+// representatives mod q agree with them.  Fields of a rejected attempt's
+// sig_out are left partly written.
 template <class P>
-__device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t *slot, uint8_t *sig_out, int32_t *x,
-                                        const ZetaLds &zt) {
+__device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t *slot, uint8_t *sig_out,
+                                        ZScratch<P> &zs) {
     using Z = Sizes<P>;
     using SL = SlotLayout<P>;
     const ItemView<P> it(a, item);
     const int lane = lane_id();
-    int32_t ch[4];
-    wave_load_challenge_A(ch, reinterpret_cast<const uint32_t *>(slot + SL::CP));
-    ntt_wave(ch, x, zt);
+    const uint4 *wbase = reinterpret_cast<const uint4 *>(slot + SL::W) + lane;  // layout D
+    uint4 w[P::K];
+#pragma unroll
+    for (int k = 0; k < P::K; ++k) w[k] = wbase[k * (N / 4)];
+    wave_toeplitz(zs.toep, reinterpret_cast<const uint32_t *>(slot + SL::CP));
+    wave_ring_mul<P::K + P::L>(zs.rows, zs.toep, it.s8);
+    wave_lds_sync();
 
-    uint8_t *h = sig_out + Z::SIG_H;
-    int pos = 0;
-    // operands of row k + 1 are loaded while row k is transformed (prefetch)
-    const int32_t *wbase = reinterpret_cast<const int32_t *>(slot + SL::W);
-    int32_t nr0[4], nct0[4], nw[4];
-    wave_load_D(nr0, it.s2h);
-    wave_load_D(nct0, it.t0h);
-    wave_load_A(nw, wbase);
+    // r0 = w0 - c s2
+#pragma unroll
     for (int k = 0; k < P::K; ++k) {
-        int32_t r0[4], ct0[4], w[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            r0[r] = nr0[r];
-            ct0[r] = nct0[r];
-            w[r] = nw[r];
-        }
-        if (k + 1 < P::K) {
-            wave_load_D(nr0, it.s2h + (k + 1) * N);
-            wave_load_D(nct0, it.t0h + (k + 1) * N);
-            wave_load_A(nw, wbase + (k + 1) * N);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            r0[r] = mont_mul(ch[r], r0[r]);
-            ct0[r] = mont_mul(ch[r], ct0[r]);
-        }
-        intt_wave(r0, x, zt);
-        int32_t w1[4];
+        int32_t cs[4];
+        wave_ring_row(cs, zs.rows + k * RING_ROW);
+        const uint32_t wp[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
         bool big = false;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            int32_t w0;
-            w1[r] = decompose<P>(w[r], w0);
-            r0[r] = reduce32(w0 - r0[r]);
-            big |= exceeds(r0[r], P::GAMMA2 - P::BETA);
-        }
+        for (int r = 0; r < 4; ++r) big |= abs(packed_w0(wp[r]) - cs[r]) >= P::GAMMA2 - P::BETA;
         if (wave_any(big)) return false;
-        intt_wave(ct0, x, zt);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            ct0[r] = reduce32(ct0[r]);
-            big |= exceeds(ct0[r], P::GAMMA2);
-        }
-        if (wave_any(big)) return false;
-        // MakeHint in ascending coefficient order j = 64 r + lane
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int hb = make_hint<P>(r0[r] + ct0[r], w1[r]);
-            const uint64_t m = __ballot(hb);
-            const int cnt = __popcll(m);
-            if (pos + cnt > P::OMEGA) return false;
-            if (hb) {
-                const int idx = pos + __popcll(m & ((1ull << lane) - 1ull));
-                h[idx] = (uint8_t)(64 * r + lane);
-            }
-            pos += cnt;
-        }
-        if (lane == 0) h[P::OMEGA + k] = (uint8_t)pos;
     }
 
+    // z = y + c s1
+    int32_t y[P::L][4];
+#pragma unroll
+    for (int l = 0; l < P::L; ++l) load_y_D<P>(y[l], slot, l);
+#pragma unroll
     for (int l = 0; l < P::L; ++l) {
-        int32_t zl[4], s[4], y[4];
-        wave_load_D(s, it.s1h + l * N);
-        load_y_A<P>(y, slot, l);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) zl[r] = mont_mul(ch[r], s[r]);
-        intt_wave(zl, x, zt);
+        int32_t cs[4];
+        wave_ring_row(cs, zs.rows + (P::K + l) * RING_ROW);
         bool big = false;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            zl[r] = reduce32(zl[r] + y[r]);
-            big |= exceeds(zl[r], P::GAMMA1 - P::BETA);
-        }
-        if (wave_any(big)) return false;
-        layout_A_to_D(zl, x);
         uint32_t f[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) f[r] = (uint32_t)(P::GAMMA1 - zl[r]);
+        for (int r = 0; r < 4; ++r) {
+            const int32_t z = y[l][r] + cs[r];
+            big |= abs(z) >= P::GAMMA1 - P::BETA;
+            f[r] = (uint32_t)(P::GAMMA1 - z);
+        }
+        if (wave_any(big)) return false;
         wave_pack_D<Z::Z_BITS>(sig_out + Z::SIG_Z + l * Z::POLYZ_BYTES, f);
+    }
+
+    // c t0, the hints in ascending coefficient order j = 4 lane + r
+    wave_lds_sync();
+    wave_ring_mul<2 * P::K>(zs.rows + P::K * RING_ROW, zs.toep, it.t8);
+    wave_lds_sync();
+    uint8_t *h = sig_out + Z::SIG_H;
+    int pos = 0;
+#pragma unroll 1
+    for (int k = 0; k < P::K; ++k) {
+        int32_t cs[4], lo[4], hi[4];
+        wave_ring_row(cs, zs.rows + k * RING_ROW);
+        wave_ring_row(lo, zs.rows + (P::K + k) * RING_ROW);
+        wave_ring_row(hi, zs.rows + (2 * P::K + k) * RING_ROW);
+        const uint4 wk = wbase[k * (N / 4)];
+        const uint32_t wp[4] = {wk.x, wk.y, wk.z, wk.w};
+        bool big = false;
+        int hb[4], before = 0, cnt = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int32_t ct0 = lo[r] + 128 * hi[r];
+            big |= abs(ct0) >= P::GAMMA2;
+            hb[r] = make_hint<P>(packed_w0(wp[r]) - cs[r] + ct0, (int32_t)packed_w1(wp[r]));
+            const uint64_t m = __ballot(hb[r]);
+            before += __popcll(m & ((1ull << lane) - 1ull));  // hints of lower lanes
+            cnt += __popcll(m);
+        }
+        if (wave_any(big) || pos + cnt > P::OMEGA) return false;
+        int idx = pos + before;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (hb[r]) h[idx++] = (uint8_t)(4 * lane + r);
+        pos += cnt;
+        if (lane == 0) h[P::OMEGA + k] = (uint8_t)pos;
     }
     for (int j = pos + lane; j < P::OMEGA; j += 64) h[j] = 0;
     return true;
