@@ -367,22 +367,18 @@ static int sign_dropin(int mode, int engine, uint8_t *sig, size_t sig_pitch, siz
         } else {
             // Attempt slots. Up to exec_threshold items: the temp rows. Larger
             // batches: slot s keeps its state in sign-pool row s (its slot area,
-            // otherwise unused here) and its candidate signature in the temp pool
-            // read as one array of SIG_STRIDE entries, so the same pools give up
-            // to `batch` slots (a card-filling batch at the reference's default
-            // exec_threshold of 2048). Results do not depend on the slot count.
-            // The first word of d_copy_lut is the work-queue head.
-            if ((e = launch_sign_fixed(mode, a, st))) return e;
-            constexpr size_t SIG_STRIDE = align256(Z::SIG_BYTES);
-            SlotRef slots = temp_slots;
-            size_t nslots = exec_threshold;
-            if (batch > exec_threshold) {
-                nslots = std::min(batch, exec_threshold * temp_pitch / SIG_STRIDE);
-                slots = SlotRef{d_sign_pool + SLy::SLOT, sign_pitch, d_temp_pool, SIG_STRIDE};
-            }
+            // otherwise unused here), so the same pools give `batch` slots (a
+            // card-filling batch at the reference's default exec_threshold of
+            // 2048). Results do not depend on the slot count. The first words of
+            // d_copy_lut are the call's control words; the lists lie behind the
+            // int8 key polynomials of the sign-pool rows.
+            const bool own = batch > exec_threshold;
             uint32_t *ctl = reinterpret_cast<uint32_t *>(lut->d_copy_lut);
-            e = launch_sign_persistent(mode, a, slots, nslots, default_slots_per_block(nslots), 0, 0, 0, ctl, nullptr,
-                                       st);
+            constexpr size_t KEY8 = (size_t)(P::L + 3 * P::K) * N;
+            static_assert(KEY8 + CHAIN_CHUNK_BYTES <= (size_t)(P::L + 2 * P::K) * N * 4, "a row holds a list chunk");
+            const ChunkRef lists{d_sign_pool + SLy::s8(mlen) + KEY8, sign_pitch};
+            e = sign_call(mode, a, own ? item_slots : temp_slots, own ? batch : exec_threshold, lists, PersistTiling{},
+                          ctl, nullptr, st, nullptr);
             if (e == -3) return DIL_ERANGE;
             if (e) return e;
             // like the reference's call, return once the rejection loop is done
@@ -605,6 +601,7 @@ int dil_verify_device(int mode, int32_t *d_ret, const uint8_t *d_sig, size_t sig
 struct dil_sign_ctx {
     int mode = 0;
     size_t max_batch = 0, nslots = 0;
+    size_t round_slots = 0;   // slots allocated: nslots, or more for small batches
     uint8_t *rows = nullptr;  // SignLayout rows (messages stay external)
     size_t row_pitch = 0;
     uint8_t *slots = nullptr;  // TempLayout rows = attempt slots
@@ -683,19 +680,19 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
         if (engine == DIL_ENGINE_PERSTAGE) {
             // the per-stage scheduler launches the fixed part itself; the
             // status word is cleared here (the persistent launch clears it)
-            if ((e = launch_zero_ctl(c->d_head, st))) return e;
+            if ((e = launch_zero_ctl(c->d_head, nullptr, st))) return e;
             if (e3 && (e = (int)hipEventRecord(e3[1], st))) return e;
             const SlotRef items{c->rows + SignLayout<P>::SLOT, c->row_pitch, d_sig, sig_pitch};
             e = sign_perstage(c->mode, a, items, slots, c->nslots, c->sign_lut.data(), c->h_exec, c->d_exec,
                               c->h_done, c->d_done, c->h_copy, c->d_copy, st);
         } else {
-            if ((e = launch_sign_fixed(c->mode, a, st))) return e;
-            if (e3 && (e = (int)hipEventRecord(e3[1], st))) return e;
-            const int spb = c->slots_per_block ? c->slots_per_block : default_slots_per_block(c->nslots);
             unsigned long long *ph =
                 c->profile ? reinterpret_cast<unsigned long long *>(c->d_head + 16) : nullptr;
-            e = launch_sign_persistent(c->mode, a, slots, c->nslots, spb, c->occupancy, c->blocks, c->claim, c->d_head,
-                                       ph, st);
+            const ChunkRef lists{reinterpret_cast<uint8_t *>(c->d_copy), sign_lists_chunk_bytes()};
+            // a tiling is for the slots the caller asked for
+            const PersistTiling tiling{c->nslots, c->slots_per_block, c->blocks, c->claim};
+            e = sign_call(c->mode, a, slots, c->round_slots, lists, tiling, c->d_head, ph, st,
+                          e3 ? e3[1] : nullptr);
             if (e == -3) return DIL_ERANGE;
         }
         if (e) return e;
@@ -709,12 +706,21 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
 }
 
 
-static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots, bool resident_only) {
+// Attempt slots of a context for small batches: enough that each item gets 16
+// consecutive nonces per round (a round's latency is the same for one or for
+// thousands of attempts), at most 8,192 (about 130 MB).
+static size_t round_slots_for(size_t max_batch, size_t nslots) {
+    return std::max({nslots, 2 * max_batch, std::min<size_t>(16 * max_batch, 8192)});
+}
+
+static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots, size_t round_slots,
+                      bool resident_only) {
     if (!out || !valid_mode(mode) || max_batch == 0 || nslots == 0) return DIL_EINVAL;
     dil_sign_ctx *c = new dil_sign_ctx();
     c->mode = mode;
     c->max_batch = max_batch;
     c->nslots = nslots;
+    c->round_slots = round_slots;
     c->resident_only = resident_only;
     c->row_pitch = resident_only
                        ? with_params(mode, [](auto p) { return align256(SignLayout<decltype(p)>::ints(0)); })
@@ -725,11 +731,13 @@ static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nsl
         if (r != hipSuccess && e == hipSuccess) e = r;
     };
     chk(hipMalloc((void **)&c->rows, c->row_pitch * max_batch));
-    chk(hipMalloc((void **)&c->slots, c->slot_pitch * nslots));
+    chk(hipMalloc((void **)&c->slots, c->slot_pitch * round_slots));
     chk(hipMalloc((void **)&c->d_head, 256));
     chk(hipMalloc((void **)&c->d_exec, 4 * nslots));
     chk(hipMalloc((void **)&c->d_done, nslots));
-    chk(hipMalloc((void **)&c->d_copy, 16 * nslots));
+    // the per-stage engine's copy table, or the rounds' lists
+    chk(hipMalloc((void **)&c->d_copy,
+                  std::max(16 * nslots, sign_lists_chunks(max_batch) * sign_lists_chunk_bytes())));
     chk(hipHostMalloc((void **)&c->h_exec, 4 * nslots, hipHostMallocDefault));
     chk(hipHostMalloc((void **)&c->h_done, nslots, hipHostMallocDefault));
     chk(hipHostMalloc((void **)&c->h_copy, 16 * nslots, hipHostMallocDefault));
@@ -740,6 +748,10 @@ static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nsl
     }
     *out = c;
     return 0;
+}
+
+int sign_ctx_create_resident_exact(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots) {
+    return ctx_create(out, mode, max_batch, nslots, nslots, true);
 }
 
 extern "C" {
@@ -762,11 +774,11 @@ int dil_sign_ctx_destroy(dil_sign_ctx *c) {
 }
 
 int dil_sign_ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots) {
-    return ctx_create(out, mode, max_batch, nslots, false);
+    return ctx_create(out, mode, max_batch, nslots, round_slots_for(max_batch, nslots), false);
 }
 
 int dil_sign_ctx_create_resident(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots) {
-    return ctx_create(out, mode, max_batch, nslots, true);
+    return ctx_create(out, mode, max_batch, nslots, round_slots_for(max_batch, nslots), true);
 }
 
 int dil_sign_ctx_set_tiling(dil_sign_ctx *c, int slots_per_block, int occupancy, int blocks) {

@@ -34,6 +34,7 @@ struct SlotLayout {
     using Z = Sizes<P>;
     static constexpr size_t W1PK = 0;                                 // K * POLYW1_BYTES
     static constexpr size_t CP = align256(Z::W1PK_BYTES);             // challenge masks (64 B)
+    static constexpr size_t CT = CP + 64;                             // c~ (32 B) in the signing rounds
     static constexpr size_t FLAG = CP + 256;                          // int32 flags
     static constexpr size_t YRAW = FLAG + 256;                        // L * 680 bytes
     static constexpr size_t W = YRAW + align256((size_t)P::L * Z::YRAW_BYTES);  // int32 K x 256
@@ -49,6 +50,9 @@ struct SignLayout {
     static constexpr size_t MU = SK + align256(Z::SK_BYTES);  // mu (64) | rhoprime (64) | attempts (4)
     static constexpr size_t RHOPRIME = MU + CRHBYTES;
     static constexpr size_t ATTEMPTS = MU + 2 * CRHBYTES;
+    // control block of a chain of signing rounds (sign_rounds.hip), in the
+    // chain's first row
+    static constexpr size_t CHAIN = MU + 136;
     static constexpr size_t SLOT = MU + 256;
     static constexpr size_t M = SLOT + SL::BYTES;
     static size_t ints(size_t mlen) { return M + align256(mlen); }

@@ -83,6 +83,7 @@ struct SignLutEntry {
 
 struct SignArgs;
 struct SlotRef;
+struct Chain;
 
 int launch_keygen(int mode, const KeygenArgs &a, hipStream_t st);
 // Expands keys [0, n) of a key store (KeyLayout rows from `keys`): tr, A and
@@ -90,10 +91,11 @@ int launch_keygen(int mode, const KeygenArgs &a, hipStream_t st);
 int launch_key_expand(int mode, uint8_t *keys, size_t key_pitch, size_t n, int with_sk, hipStream_t st);
 // ev: null, or four events recorded around vf_prep / vf_main / vf_final
 int launch_verify(int mode, const VerifyArgs &a, hipStream_t st, hipEvent_t *ev = nullptr);
-int launch_sign_fixed(int mode, const SignArgs &a, hipStream_t st);
-// mu / rhoprime (signing) and tr / mu (verification) with one sponge per
-// 16-lane row instead of one lane: for batches of long messages
-int launch_sign_mu_row(int mode, const SignArgs &a, hipStream_t st);
+// The fixed part of signing (mu, rhoprime, ExpandA, the int8 secret key) for
+// the chain's items; starts its list when it has one.
+int launch_sign_fixed(int mode, const SignArgs &a, const Chain &ch, hipStream_t st);
+// tr / mu of verification with one sponge per 16-lane row instead of one
+// lane: for batches of long messages
 int launch_verify_mu_row(int mode, const VerifyArgs &a, hipStream_t st);
 int launch_sign_round(int mode, const SignArgs &a, const SlotRef &sr, const uint32_t *d_exec, size_t nslot,
                       int by_item, uint8_t *d_done, hipStream_t st);
@@ -105,17 +107,42 @@ constexpr uint32_t SIGN_STATUS_NO_SECRET = 2u;  // an item's resident key has no
 // Resident keys: zeroes the signatures of items whose key has no secret key
 // and sets SIGN_STATUS_NO_SECRET in *status (no-op without key indices).
 int launch_sign_key_check(int mode, const SignArgs &a, uint32_t *status, hipStream_t st);
-// Clears the control words d_head[0..2] (a kernel, so graph capture records
-// no memset node).
-int launch_zero_ctl(uint32_t *d_head, hipStream_t st);
+// Clears the control words ctl[0..2], and the phase sums when given (a
+// kernel, so graph capture records no memset node).
+int launch_zero_ctl(uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st);
+// A whole signing call, over nslots attempt slots: device-driven rounds
+// (sign_rounds.hip), or for large batches the persistent kernel.
+// lists: sign_lists_chunks(n) chunks of sign_lists_chunk_bytes() scratch
+// bytes (8-aligned), lists.pitch apart.  phase_sums: null, or the persistent
+// kernel runs and fills them.  fixed_done: null, or an event recorded after
+// the fixed stage.
+struct ChunkRef {
+    uint8_t *base;
+    size_t pitch;
+};
+struct PersistTiling {  // 0: automatic
+    size_t nslots;      // of the slots, those the persistent kernel uses
+    int slots_per_block, blocks, claim;
+};
+size_t sign_lists_chunks(size_t n);
+size_t sign_lists_chunk_bytes();
+int sign_call(int mode, const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRef &lists,
+              const PersistTiling &tiling, uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st,
+              hipEvent_t fixed_done);
 int sign_perstage(int mode, const SignArgs &a, const SlotRef &item_slots, const SlotRef &temp_slots, size_t thr,
                   SignLutEntry *sign_lut, uint32_t *h_exec, uint32_t *d_exec, uint8_t *h_done, uint8_t *d_done,
                   uint64_t *h_copy, uint64_t *d_copy, hipStream_t st);
-// Rejection loop of the persistent engine over nslots slots (the fixed part
-// must have been launched first).  blocks <= 0: nslots / slots_per_block.
-int launch_sign_persistent(int mode, const SignArgs &a, const SlotRef &sr, size_t nslots, int slots_per_block,
-                           int occupancy, int blocks, int claim, uint32_t *d_head, unsigned long long *phase_sums,
-                           hipStream_t st);
+// The persistent kernel over nslots slots (the fixed part must have been
+// launched and ctl cleared first): the items left in the chain's list.
+// blocks <= 0: nslots / slots_per_block.
+int launch_sign_persistent(int mode, const SignArgs &a, const SlotRef &sr, const Chain &chain, size_t nslots,
+                           int slots_per_block, int blocks, int claim, uint32_t *ctl,
+                           unsigned long long *phase_sums, hipStream_t st);
 int default_slots_per_block(size_t nslots);
 
 }  // namespace dil
+
+// dil_sign_ctx_create_resident with exactly nslots attempt slots, for callers
+// that budget the context's memory (the server)
+struct dil_sign_ctx;
+int sign_ctx_create_resident_exact(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t nslots);

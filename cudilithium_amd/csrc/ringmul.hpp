@@ -35,14 +35,16 @@ constexpr int RING_ROW = N + 16;
 // bit b of a nibble to byte b
 __device__ __forceinline__ uint32_t nibble_bytes(uint32_t nib) { return (nib * 0x00204081u) & 0x01010101u; }
 
-// Fills T from the challenge masks (nz[8] | neg[8]; neg is a subset of nz).
-__device__ __forceinline__ void wave_toeplitz(uint32_t *T, const uint32_t *masks) {
+// Fills T from the challenge masks nz[8] | neg[8] (neg is a subset of nz):
+// lane l passes words w = toeplitz_word(l) of both.
+__device__ __forceinline__ int toeplitz_word(int l) { return 7 - (l >> 3); }
+__device__ __forceinline__ void wave_toeplitz(uint32_t *T, uint32_t nz_word, uint32_t neg_word) {
     const int l = lane_id();
     // word l holds x = 4l .. 4l + 3, i.e. c[255 - 4l] downwards: nibble l of
     // the bit-reversed masks
-    const int w = 7 - (l >> 3), sh = 4 * (l & 7);
-    const uint32_t nz = nibble_bytes((__brev(masks[w]) >> sh) & 15u);
-    const uint32_t ng = nibble_bytes((__brev(masks[8 + w]) >> sh) & 15u);
+    const int sh = 4 * (l & 7);
+    const uint32_t nz = nibble_bytes((__brev(nz_word) >> sh) & 15u);
+    const uint32_t ng = nibble_bytes((__brev(neg_word) >> sh) & 15u);
     wave_lds_sync();
     T[l] = nz + ng * 0xFEu;              // 0x01 or, negative, 0xFF
     T[64 + l] = nz + (nz ^ ng) * 0xFEu;  // the negated half, x >= 256
@@ -57,56 +59,48 @@ __device__ __forceinline__ void wave_toeplitz(uint32_t *T, const uint32_t *masks
     wave_lds_sync();
 }
 
-// rows[n] = c * s8[n] for n < NCOL: s8 holds int8 polynomials of N bytes
-// each (16-byte aligned), rows int16 rows of RING_ROW.
-//
-// Row tile a (coefficients 16a .. 16a + 15) and step b (j = 64b ..) need, in
-// lane (m, g) = (lane & 15, lane >> 4), the 16 bytes C~[16a + m - 64b - 16g - t],
-// t < 16: Rv from x = 16 (15 - (a - 4b) + g) + (15 - m), which depends on
-// q = a - 4b only, so 28 operands serve all 64 products.
-template <int NCOL>
-__device__ __forceinline__ void wave_ring_mul(uint16_t *rows, const uint32_t *T, const int8_t *s8) {
-    static_assert(NCOL <= 16, "one column tile");
-    const int l = lane_id(), n = l & 15, g = l >> 4;
-    const int8_t *src = s8 + min(n, NCOL - 1) * N + 16 * g;
-    v4i B[4];
+// The right-hand operands of wave_ring_mul: lane (n, g) = (lane & 15,
+// lane >> 4) holds bytes 64b + 16g .. + 15 of its column's polynomial, a
+// 16-byte aligned int8 polynomial of N bytes at `poly`.
+__device__ __forceinline__ void wave_ring_load(v4i (&B)[4], const int8_t *poly) {
+    const int8_t *src = poly + 16 * (lane_id() >> 4);
 #pragma unroll
     for (int b = 0; b < 4; ++b) B[b] = *reinterpret_cast<const v4i *>(src + 64 * b);
+}
+
+// rows[n] = c * (column n) for n < NCOL, int16 rows of RING_ROW.
+//
+// Row tile a (coefficients 16a .. 16a + 15) and step b (j = 64b ..) need, in
+// lane (m, g), the 16 bytes C~[16a + m - 64b - 16g - t], t < 16: Rv from
+// x = 16 (15 - (a - 4b) + g) + (15 - m).  They are read from the table for
+// each product (half the LDS bandwidth) rather than held: 64 registers fewer
+// let one or two more waves run on each SIMD.
+template <int NCOL>
+__device__ __forceinline__ void wave_ring_mul(uint16_t *rows, const uint32_t *T, const v4i (&B)[4]) {
+    static_assert(NCOL <= 16, "one column tile");
+    const int l = lane_id(), n = l & 15, g = l >> 4;
     const uint32_t *tl = T + ((15 - n) & 3) * TOEP_STRIDE + ((15 - n) >> 2) + 4 * (15 + g);
-    auto operand = [&](int q) -> v4i {
-        const uint32_t *p = tl - 4 * q;
-        return v4i{(int)p[0], (int)p[1], (int)p[2], (int)p[3]};
-    };
-    // op[i][b]: operand of q = 4A + i - 4b; the step to the next four tiles
-    // shifts b by one and loads four new ones
-    v4i op[4][4];
-#pragma unroll
-    for (int b = 0; b < 3; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) op[i][b] = operand(i - 4 * (b + 1));
     uint16_t *dst = rows + n * RING_ROW + 4 * g;
-#pragma unroll
-    for (int A = 0; A < 4; ++A) {
+#pragma unroll 1
+    for (int A = 0; A < 4; ++A, tl -= 16, dst += 64) {
         v4i acc[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int b = 3; b > 0; --b) op[i][b] = op[i][b - 1];
-            op[i][0] = operand(4 * A + i);
-            acc[i] = v4i{0, 0, 0, 0};
-        }
+        for (int i = 0; i < 4; ++i) acc[i] = v4i{0, 0, 0, 0};
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[i][b], B[b], acc[i], 0, 0, 0);
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t *p = tl - 4 * (i - 4 * b);
+                const v4i op{(int)p[0], (int)p[1], (int)p[2], (int)p[3]};
+                acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op, B[b], acc[i], 0, 0, 0);
+            }
         if (n < NCOL) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 // low halves of two results per word
                 const uint32_t lo = __builtin_amdgcn_perm((uint32_t)acc[i][1], (uint32_t)acc[i][0], 0x05040100u);
                 const uint32_t hi = __builtin_amdgcn_perm((uint32_t)acc[i][3], (uint32_t)acc[i][2], 0x05040100u);
-                *reinterpret_cast<uint2 *>(dst + 16 * (4 * A + i)) = make_uint2(lo, hi);
+                *reinterpret_cast<uint2 *>(dst + 16 * i) = make_uint2(lo, hi);
             }
         }
     }

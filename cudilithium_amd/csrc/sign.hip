@@ -19,46 +19,6 @@ namespace dil {
 
 constexpr int SIGN_WAVES = 4;
 
-// One lane absorbs a whole message serially, so the batch waits for its
-// longest message; the wave asks for the highest issue priority on its SIMD
-// (s_setprio, a per-wave hint) so that other kernels' waves sharing the SIMD
-// do not stretch that serial chain.
-template <class P>
-__global__ __launch_bounds__(256) void sg_mu_kernel(SignArgs a) {
-    __builtin_amdgcn_s_setprio(3);
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < a.n) stage_mu<P>(a, i);
-}
-
-// two lanes per item: 128 items per workgroup
-template <class P>
-__global__ __launch_bounds__(256) void sg_mu_pair_kernel(SignArgs a) {
-    __builtin_amdgcn_s_setprio(3);
-    const size_t i = (size_t)blockIdx.x * 128 + (threadIdx.x >> 1);
-    if (i < a.n) stage_mu_pair<P>(a, i, threadIdx.x & 1);  // both lanes of a pair take the same branch
-}
-
-template <class P>
-__global__ __launch_bounds__(256) void sg_expand_kernel(SignArgs a) {
-    constexpr int KL = P::K * P::L;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.n * KL) return;
-    const int e = (int)(t % KL);
-    stage_expand_a<P>(a, t / KL, e / P::L, e % P::L);
-}
-
-// secret key to int8 polynomials, 8 coefficients per lane
-template <class P>
-__global__ __launch_bounds__(256) void sg_prep_kernel(SignArgs a) {
-    constexpr int PER = (P::L + 2 * P::K) * (N / 8);
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.n * PER) return;
-    const size_t i = t / PER;
-    const int u = (int)(t % PER);
-    int8_t *dst = reinterpret_cast<int8_t *>(a.rows + i * a.row_pitch + a.off_ints) + P::K * P::L * N * 4;
-    stage_prep<P>(a.sk + i * a.sk_pitch, dst, u / (N / 8), u % (N / 8));
-}
-
 // exec entry e = (item << 16) | nonce (api.cu:221-230)
 template <class P>
 __global__ __launch_bounds__(256) void sg_y_kernel(SignArgs a, SlotRef sr, const uint32_t *exec, size_t nslot,
@@ -145,63 +105,6 @@ int sign_key_check_impl(const SignArgs &a, uint32_t *status, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-// The three fixed-stage launches are independent: mu/rhoprime (two lanes per
-// item, latency-bound on long messages), ExpandA (one lane per matrix entry,
-// throughput-bound) and the s1/s2/t0 NTTs run as a fork/join over the
-// caller's stream and two auxiliary streams of this device, so the idle
-// lanes of one fill with the others' waves.  Event fork/join is also what a
-// HIP graph capture records as parallel branches.
-template <class P>
-int sign_fixed_impl(const SignArgs &a, hipStream_t st) {
-    if (a.n == 0) return 0;
-    constexpr int KL = P::K * P::L, PREP = (P::L + 2 * P::K) * (N / 8);
-    auto mu = [&](hipStream_t s) -> int {
-        if (a.row_mu) return launch_sign_mu_row(P::MODE, a, s);
-        // two lanes per item by default: fixed stage of 16,384 Dilithium3
-        // items 0.77 -> 0.53 ms when launched call by call; inside a graph,
-        // where ExpandA and the transforms bound it, the step is unchanged
-#ifndef DIL_MU_PAIR
-#define DIL_MU_PAIR 1
-#endif
-        if (DIL_MU_PAIR)
-            hipLaunchKernelGGL(sg_mu_pair_kernel<P>, dim3((unsigned)((a.n + 127) / 128)), dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL(sg_mu_kernel<P>, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a);
-        return (int)hipGetLastError();
-    };
-    if (a.key_idx) return mu(st);  // resident keys carry A, s1, s2, t0 already: only mu / rhoprime
-    // Batches below DIL_FIXED_FORK_MIN items run the three launches in order
-    // on the caller's stream.  Off by default: for one caller the fork is
-    // faster (1,024 / 4,096 items: 1.76 / 1.83 ms against 1.86 / 2.07 ms);
-    // with ten concurrent callers the serial form was faster (4.6 against
-    // 5.0 ms per round of 1,000-item calls).
-#ifndef DIL_FIXED_FORK_MIN
-#define DIL_FIXED_FORK_MIN 0
-#endif
-    if (a.n < (size_t)DIL_FIXED_FORK_MIN) {
-        int e;
-        if ((e = mu(st))) return e;
-        hipLaunchKernelGGL(sg_prep_kernel<P>, dim3((unsigned)((a.n * PREP + 255) / 256)), dim3(256), 0, st, a);
-        hipLaunchKernelGGL(sg_expand_kernel<P>, dim3((unsigned)((a.n * KL + 255) / 256)), dim3(256), 0, st, a);
-        return (int)hipGetLastError();
-    }
-    AuxStreams *aux = aux_streams(st);
-    if (!aux) return (int)hipErrorOutOfMemory;
-    std::lock_guard<std::mutex> guard(aux->lock);
-    int e;
-    if ((e = (int)hipEventRecord(aux->fork, st))) return e;
-    if ((e = (int)hipStreamWaitEvent(aux->s[0], aux->fork, 0))) return e;
-    if ((e = (int)hipStreamWaitEvent(aux->s[1], aux->fork, 0))) return e;
-    if ((e = mu(aux->s[0]))) return e;
-    hipLaunchKernelGGL(sg_prep_kernel<P>, dim3((unsigned)((a.n * PREP + 255) / 256)), dim3(256), 0, aux->s[1], a);
-    hipLaunchKernelGGL(sg_expand_kernel<P>, dim3((unsigned)((a.n * KL + 255) / 256)), dim3(256), 0, st, a);
-    if ((e = (int)hipGetLastError())) return e;
-    if ((e = (int)hipEventRecord(aux->join[0], aux->s[0]))) return e;
-    if ((e = (int)hipEventRecord(aux->join[1], aux->s[1]))) return e;
-    if ((e = (int)hipStreamWaitEvent(st, aux->join[0], 0))) return e;
-    return (int)hipStreamWaitEvent(st, aux->join[1], 0);
-}
-
 template <class P>
 int sign_round_impl(const SignArgs &a, const SlotRef &sr, const uint32_t *d_exec, size_t nslot, int by_item,
                     uint8_t *d_done, hipStream_t st) {
@@ -231,8 +134,6 @@ int sign_copy_impl(const SignArgs &a, const SlotRef &sr, const uint64_t *d_copy,
         default: return -1;                              \
     }
 
-int launch_sign_fixed(int mode, const SignArgs &a, hipStream_t st) { DIL_DISPATCH(mode, sign_fixed_impl, a, st) }
-
 int launch_sign_key_check(int mode, const SignArgs &a, uint32_t *status, hipStream_t st) {
     DIL_DISPATCH(mode, sign_key_check_impl, a, status, st)
 }
@@ -256,7 +157,10 @@ int launch_sign_copy(int mode, const SignArgs &a, const SlotRef &sr, const uint6
 int sign_perstage(int mode, const SignArgs &a, const SlotRef &item_slots, const SlotRef &temp_slots, size_t thr,
                   SignLutEntry *sign_lut, uint32_t *h_exec, uint32_t *d_exec, uint8_t *h_done, uint8_t *d_done,
                   uint64_t *h_copy, uint64_t *d_copy, hipStream_t st) {
-    int e = launch_sign_fixed(mode, a, st);
+    Chain all{};
+    all.rows = a.rows;
+    all.n = (uint32_t)a.n;
+    int e = launch_sign_fixed(mode, a, all, st);
     if (e) return e;
     for (size_t i = 0; i < a.n; ++i) sign_lut[i] = SignLutEntry{0, 0};
     size_t remaining = a.n;

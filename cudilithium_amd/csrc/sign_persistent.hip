@@ -12,22 +12,21 @@ __global__ void zero_ctl_kernel(uint32_t *p, unsigned long long *phase_sums) {
         for (int w = 0; w < PERSIST_PHASES; ++w) phase_sums[w] = 0;
 }
 
-int launch_zero_ctl(uint32_t *d_head, hipStream_t st) {
-    hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(1), 0, st, d_head, nullptr);
+int launch_zero_ctl(uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st) {
+    hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(1), 0, st, ctl, phase_sums);
     return (int)hipGetLastError();
 }
 
-int launch_sign_persistent(int mode, const SignArgs &a, const SlotRef &sr, size_t nslots, int slots_per_block,
-                           int occupancy, int blocks, int claim, uint32_t *d_head, unsigned long long *phase_sums,
-                           hipStream_t st) {
+int launch_sign_persistent(int mode, const SignArgs &a, const SlotRef &sr, const Chain &chain, size_t nslots,
+                           int slots_per_block, int blocks, int claim, uint32_t *ctl,
+                           unsigned long long *phase_sums, hipStream_t st) {
     if (a.n == 0) return 0;
-    if (occupancy == 0) occupancy = 2;
     switch (mode) {
-        case 2: return launch_persistent_p<Params<2>>(a, sr, nslots, slots_per_block, occupancy, blocks, claim, d_head,
+        case 2: return launch_persistent_p<Params<2>>(a, sr, chain, nslots, slots_per_block, blocks, claim, ctl,
                                                       phase_sums, st);
-        case 3: return launch_persistent_p<Params<3>>(a, sr, nslots, slots_per_block, occupancy, blocks, claim, d_head,
+        case 3: return launch_persistent_p<Params<3>>(a, sr, chain, nslots, slots_per_block, blocks, claim, ctl,
                                                       phase_sums, st);
-        case 5: return launch_persistent_p<Params<5>>(a, sr, nslots, slots_per_block, occupancy, blocks, claim, d_head,
+        case 5: return launch_persistent_p<Params<5>>(a, sr, chain, nslots, slots_per_block, blocks, claim, ctl,
                                                       phase_sums, st);
         default: return -1;
     }

@@ -51,27 +51,23 @@ constexpr int PERSIST_PHASES = 6;
 #define DIL_KECCAK_PRIO 2
 #endif
 constexpr int KECCAK_PRIO = DIL_KECCAK_PRIO;
-// claim argument of the guided kernel: items per workgroup (low 16 bits) and
-// the number of workgroups resident at once (high 16 bits); guided claims
-// are built for the 2-waves-per-SIMD register budget only
-constexpr int CLAIM_GUIDED_FLAG = 0x10000;  // DIL_CLAIM_GUIDED of the header
+// waves per SIMD the register allocation must allow (256 VGPRs).  Three or
+// four (w unpaired, no spills) measured slower: 16,384 Dilithium3 items 2.85 /
+// 3.05 against 2.82 ms.
+constexpr int PERSIST_WPE = 2;
 
-// WPE: waves per SIMD the register allocation must allow (512 / WPE VGPRs)
 // claim: at most this many items owned per workgroup (1..S); below S every
 // owned item gets at least S / claim slots (nonces) per round, which trades
 // speculative attempts for fewer rounds on small batches
-// GUIDED: guided claims (a separate instantiation, so that the scalar code
-// for it does not change the register allocation of the plain kernel)
-template <class P, int S, int WPE, bool GUIDED>
-__global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void sg_persistent_kernel(
-    SignArgs a, SlotRef sr, uint32_t *head, int claim, unsigned long long *phase_sums) {
+// the items are those left in the chain's list, claimed through its head
+template <class P, int S>
+__global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu(PERSIST_WPE))) void
+sg_persistent_kernel(SignArgs a, SlotRef sr, Chain chain, uint32_t *ctl, int claim, unsigned long long *phase_sums) {
     __shared__ ZetaLds zt;
     __shared__ int32_t x[PERSIST_THREADS / 64][NTT_XBUF];
     // L = 7: the paired w stage's transformed y vectors (56 KiB per workgroup,
-    // which leaves room for two workgroups per CU: with more waves per SIMD
-    // the w stage does not pair for L = 7)
-    constexpr bool W_Y_LDS = P::L >= DIL_W_Y_LDS_MIN_L && WPE <= 2;
-    constexpr bool W_PAIRS = P::L < DIL_W_Y_LDS_MIN_L || W_Y_LDS;
+    // which leaves room for two workgroups per CU)
+    constexpr bool W_Y_LDS = P::L >= DIL_W_Y_LDS_MIN_L;
     union StageLds {
         int32_t y[W_Y_LDS ? 2 * P::L * N : 1];  // w stage
         ZScratch<P> z;                          // z stage
@@ -86,7 +82,7 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
     constexpr int NW = PERSIST_THREADS / 64;
     const size_t slot0 = (size_t)blockIdx.x * S;
     auto slot_base = [&](int s) { return sr.base + (slot0 + s) * sr.pitch; };
-    auto slot_sig = [&](int s) { return sr.sig + (slot0 + s) * sr.sig_pitch; };
+    auto slot_ct = [&](int s) { return slot_base(s) + SlotLayout<P>::CT; };  // c~ until the attempt passes
     zeta_lds_load(zt);
     if (tid == 0) {
         n_own = 0;
@@ -114,39 +110,24 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
         if (round == PERSIST_MAX_ROUNDS) {
             // no correct run gets here (each round succeeds per item with
             // probability >= 1/5); stop instead of spinning and report it
-            if (tid == 0) atomicOr(head + 1, SIGN_STATUS_ROUND_CAP);
+            if (tid == 0) atomicOr(ctl + 1, SIGN_STATUS_ROUND_CAP);
             break;
         }
         if (tid == 0) {
-            const int claim_items = GUIDED ? claim & 0xFFFF : claim;
-            int cap = claim_items > 0 && claim_items < S ? claim_items : S;
-            if constexpr (GUIDED) {
-                // guided claims: once fewer than cap items per resident
-                // workgroup are left in the queue, own at most remaining /
-                // resident workgroups of them (rounded up), so that the last
-                // items spread over all workgroups (each then gets more slots
-                // per round) instead of holding a few workgroups while the
-                // others exit
-                const uint32_t resident = (uint32_t)claim >> 16;  // >= 1: the launch passes it
-                if (!queue_empty) {
-                    const uint32_t h0 = __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    const size_t rem = (size_t)h0 < a.n ? a.n - h0 : 0;
-                    if (rem < (size_t)cap * resident) {
-                        int per = 1;
-                        while ((size_t)per * resident < rem) ++per;
-                        cap = per;
-                    }
-                }
-            }
+            const int cap = claim > 0 && claim < S ? claim : S;
             int u = n_own;
             if (u < cap && !queue_empty) {
-                const uint32_t start = atomicAdd(head, (uint32_t)(cap - u));
-                for (int j = 0; j < cap - u && (size_t)start + j < a.n; ++j) {
-                    own_item[n_own] = start + j;
-                    own_next[n_own] = 0;
+                ChainCtl *const cc = chain_ctl<P>(chain);
+                const size_t end = cc->left;
+                const uint32_t list = cc->cur;
+                const uint32_t start = atomicAdd(&cc->head, (uint32_t)(cap - u));
+                for (int j = 0; j < cap - u && (size_t)start + j < end; ++j) {
+                    const uint2 e = *chain_entry(chain, list, start + j);
+                    own_item[n_own] = e.x;
+                    own_next[n_own] = e.y;
                     ++n_own;
                 }
-                if ((size_t)start + (cap - u) >= a.n) queue_empty = 1;
+                if ((size_t)start + (cap - u) >= end) queue_empty = 1;
             }
             u = n_own;
             for (int s = 0; s < S && u > 0; ++s) {
@@ -169,7 +150,7 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
         mark(0);
         const int u = n_own;
         if (u == 0) break;
-        if (tid == 0) atomicAdd(head + 2, (uint32_t)S);  // attempts executed (incl. speculative)
+        if (tid == 0) atomicAdd(ctl + 2, (uint32_t)S);  // attempts executed (incl. speculative)
 
         // the Keccak stages (y, c) run few serial permutation chains that the
         // whole workgroup then waits for; their waves get issue priority over
@@ -199,13 +180,9 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
             const int s = w_unit[t];
             const size_t item = own_item[slot_own[s]];
             if (s + u < S) {
-                if constexpr (W_PAIRS) {
-                    uint8_t *const pair[2] = {slot_base(s), slot_base(s + u)};
-                    stage_w_multi<P, 2>(a, item, pair, x[wave], zt, stage_lds[wave].y);
-                    continue;
-                } else {
-                    stage_w<P>(a, item, slot_base(s + u), x[wave], zt);
-                }
+                uint8_t *const pair[2] = {slot_base(s), slot_base(s + u)};
+                stage_w_multi<P, 2>(a, item, pair, x[wave], zt, stage_lds[wave].y);
+                continue;
             }
             stage_w<P>(a, item, slot_base(s), x[wave], zt);
         }
@@ -215,7 +192,7 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
         // two lanes per slot (keccak_f1600_pair): S slots on 2 S lanes
         for (int t = tid; t < 2 * S; t += PERSIST_THREADS) {
             const int s = t >> 1;
-            stage_c_pair<P>(a, own_item[slot_own[s]], slot_base(s), slot_sig(s), (uint32_t)(t & 1));
+            stage_c_pair<P>(a, own_item[slot_own[s]], slot_base(s), slot_ct(s), (uint32_t)(t & 1));
         }
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
@@ -232,7 +209,7 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
             uint8_t *dst = a.sig + item * a.sig_pitch;
             for (int s = o; s < S; s += u) {
                 if (stage_z<P>(a, item, slot_base(s), dst, stage_lds[wave].z)) {
-                    const uint8_t *src = slot_sig(s);
+                    const uint8_t *src = slot_ct(s);
                     if (lane < SEEDBYTES) dst[lane] = src[lane];
                     if (lane == 0) {
                         own_done[o] = 1;
@@ -268,55 +245,33 @@ __global__ __launch_bounds__(PERSIST_THREADS) __attribute__((amdgpu_waves_per_eu
 // than a memset so that the sequence can be captured in a HIP graph
 __global__ void zero_ctl_kernel(uint32_t *p, unsigned long long *phase_sums);
 
-template <class P, int S, int WPE>
-static int launch_persistent_s(const SignArgs &a, const SlotRef &sr, size_t nslots, int blocks, int claim,
-                               uint32_t *d_head, unsigned long long *phase_sums, hipStream_t st) {
+template <class P, int S>
+static int launch_persistent_s(const SignArgs &a, const SlotRef &sr, const Chain &chain, size_t nslots, int blocks,
+                               int claim, uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st) {
     int nb = (int)(nslots / S);
     if (blocks > 0 && blocks < nb) nb = blocks;
     if (nb < 1) return -3;
-    hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(1), 0, st, d_head, phase_sums);
-    // claim: items per workgroup (low 16 bits) | workgroups resident at once
-    // (high 16 bits: the register budget allows WPE waves per SIMD)
-    if ((claim & CLAIM_GUIDED_FLAG) && WPE == 2) {
-        const int resident = std::max(1, std::min(nb, device_cu_count() * 4 * WPE / (PERSIST_THREADS / 64)));
-        const int claim_arg = (claim & 0xFFFF) | (std::min(resident, 0xFFFF) << 16);
-        hipLaunchKernelGGL((sg_persistent_kernel<P, S, WPE, WPE == 2>), dim3(nb), dim3(PERSIST_THREADS), 0, st, a,
-                           sr, d_head, claim_arg, phase_sums);
-    } else {
-        hipLaunchKernelGGL((sg_persistent_kernel<P, S, WPE, false>), dim3(nb), dim3(PERSIST_THREADS), 0, st, a, sr,
-                           d_head, claim & 0xFFFF, phase_sums);
-    }
+    hipLaunchKernelGGL((sg_persistent_kernel<P, S>), dim3(nb), dim3(PERSIST_THREADS), 0, st, a, sr, chain, ctl,
+                       claim & 0xFFFF, phase_sums);
     return (int)hipGetLastError();
 }
 
-// Defined once per mode (sign_persistent_<mode>.hip).  occupancy: waves per
-// SIMD the kernel's register allocation allows (2, 3 or 4).
+// Defined once per mode (sign_persistent_<mode>.hip).
 template <class P>
-int launch_persistent_p(const SignArgs &a, const SlotRef &sr, size_t nslots, int slots_per_block, int occupancy,
-                        int blocks, int claim, uint32_t *d_head, unsigned long long *phase_sums, hipStream_t st);
-
-template <class P, int WPE>
-static int launch_persistent_w(const SignArgs &a, const SlotRef &sr, size_t nslots, int slots_per_block, int blocks,
-                               int claim, uint32_t *d_head, unsigned long long *ph, hipStream_t st) {
-    switch (slots_per_block) {
-        case 1: return launch_persistent_s<P, 1, WPE>(a, sr, nslots, blocks, claim, d_head, ph, st);
-        case 8: return launch_persistent_s<P, 8, WPE>(a, sr, nslots, blocks, claim, d_head, ph, st);
-        case 16: return launch_persistent_s<P, 16, WPE>(a, sr, nslots, blocks, claim, d_head, ph, st);
-        case 32: return launch_persistent_s<P, 32, WPE>(a, sr, nslots, blocks, claim, d_head, ph, st);
-        default: return -1;
-    }
-}
+int launch_persistent_p(const SignArgs &a, const SlotRef &sr, const Chain &chain, size_t nslots, int slots_per_block,
+                        int blocks, int claim, uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st);
 
 #define DIL_DEFINE_PERSISTENT_LAUNCHER(MODE)                                                                       \
     template <>                                                                                                  \
-    int launch_persistent_p<Params<MODE>>(const SignArgs &a, const SlotRef &sr, size_t nslots,                    \
-                                          int slots_per_block, int occupancy, int blocks, int claim,              \
-                                          uint32_t *d_head, unsigned long long *ph, hipStream_t st) {            \
+    int launch_persistent_p<Params<MODE>>(const SignArgs &a, const SlotRef &sr, const Chain &chain, size_t nslots, \
+                                          int slots_per_block, int blocks, int claim, uint32_t *ctl,             \
+                                          unsigned long long *ph, hipStream_t st) {                              \
         using P = Params<MODE>;                                                                                  \
-        switch (occupancy) {                                                                                     \
-            case 2: return launch_persistent_w<P, 2>(a, sr, nslots, slots_per_block, blocks, claim, d_head, ph, st); \
-            case 3: return launch_persistent_w<P, 3>(a, sr, nslots, slots_per_block, blocks, claim, d_head, ph, st); \
-            case 4: return launch_persistent_w<P, 4>(a, sr, nslots, slots_per_block, blocks, claim, d_head, ph, st); \
+        switch (slots_per_block) {                                                                               \
+            case 1: return launch_persistent_s<P, 1>(a, sr, chain, nslots, blocks, claim, ctl, ph, st);          \
+            case 8: return launch_persistent_s<P, 8>(a, sr, chain, nslots, blocks, claim, ctl, ph, st);          \
+            case 16: return launch_persistent_s<P, 16>(a, sr, chain, nslots, blocks, claim, ctl, ph, st);        \
+            case 32: return launch_persistent_s<P, 32>(a, sr, chain, nslots, blocks, claim, ctl, ph, st);        \
             default: return -1;                                                                                  \
         }                                                                                                        \
     }

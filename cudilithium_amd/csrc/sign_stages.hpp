@@ -59,6 +59,41 @@ __device__ __forceinline__ size_t sk_index(const SignArgs &a, size_t i) {
     return k < a.nkeys ? k : a.nkeys - 1;
 }
 
+// Control block of one chain of signing rounds (SignLayout::CHAIN of the
+// chain's first row).
+struct ChainCtl {
+    uint32_t left;   // items without a signature: entries of list `cur`
+    uint32_t count;  // entries [0, count) take part in the current round
+    uint32_t m;      // attempts (consecutive nonces) per item of the round
+    uint32_t cur;    // which of the two lists
+    uint32_t head;   // the finishing persistent kernel's queue head
+};
+static_assert(sizeof(ChainCtl) <= 256 - 136, "control block fits the row's mu area");
+
+// One chain of rounds.  The items without a signature are a list of entries
+// {item, next nonce}; two lists alternate.  They lie in chunks of 512 entries
+// (8 KiB: both lists) `chunk_pitch` bytes apart, so that a caller's pool rows
+// can hold them.
+constexpr uint32_t CHAIN_CHUNK = 512;
+constexpr size_t CHAIN_CHUNK_BYTES = CHAIN_CHUNK * 2 * sizeof(uint2);
+struct Chain {
+    uint8_t *rows;  // row of the chain's first item
+    uint8_t *lists;
+    size_t chunk_pitch;
+    uint32_t first, n;
+    uint32_t nslots;  // attempt slots of the chain
+    uint32_t target;  // attempts a round aims at when fewer items are left
+};
+
+template <class P>
+__device__ __forceinline__ ChainCtl *chain_ctl(const Chain &ch) {
+    return reinterpret_cast<ChainCtl *>(ch.rows + SignLayout<P>::CHAIN);
+}
+__device__ __forceinline__ uint2 *chain_entry(const Chain &ch, uint32_t list, uint32_t e) {
+    return reinterpret_cast<uint2 *>(ch.lists + (e / CHAIN_CHUNK) * ch.chunk_pitch) + list * CHAIN_CHUNK +
+           e % CHAIN_CHUNK;
+}
+
 // Scratch and signature destination of attempt slots.
 struct SlotRef {
     uint8_t *base;  // SlotLayout of slot s at base + s * pitch
@@ -432,11 +467,12 @@ __device__ __forceinline__ void stage_c_pair(const SignArgs &a, size_t item, uin
 }
 
 // One wave's LDS area in the z stage: the challenge's operand table and the
-// rows c s2 (K) | c s1 (L); the rows c t0 (low limbs K, high limbs K) take
-// the place of c s1 once z is written.
+// rows c s2 (K) | c s1 (L); once z is written, the rows c t0 of half of the
+// K polynomials at a time (low limbs K / 2, high limbs K / 2) take the place
+// of c s1.
 template <class P>
 struct ZScratch {
-    static constexpr int ROWS = P::K + (P::L > 2 * P::K ? P::L : 2 * P::K);
+    static constexpr int ROWS = P::K + (P::L > P::K ? P::L : P::K);
     uint32_t toep[TOEP_WORDS];
     uint16_t rows[ROWS * RING_ROW];
 };
@@ -451,19 +487,25 @@ struct ZScratch {
 // hints.  All values are exact integers below q / 2, where the reference's
 // representatives mod q agree with them.  Fields of a rejected attempt's
 // sig_out are left partly written.
-template <class P>
+// WRITE false: the checks only.
+template <class P, bool WRITE = true>
 __device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t *slot, uint8_t *sig_out,
                                         ZScratch<P> &zs) {
     using Z = Sizes<P>;
     using SL = SlotLayout<P>;
     const ItemView<P> it(a, item);
     const int lane = lane_id();
+    // every load that the first check needs is issued before the first use
+    const uint32_t *masks = reinterpret_cast<const uint32_t *>(slot + SL::CP) + toeplitz_word(lane);
+    const uint32_t nzw = masks[0], ngw = masks[8];
+    v4i B[4];
+    wave_ring_load(B, it.s8 + min(lane & 15, P::K + P::L - 1) * N);
     const uint4 *wbase = reinterpret_cast<const uint4 *>(slot + SL::W) + lane;  // layout D
     uint4 w[P::K];
 #pragma unroll
     for (int k = 0; k < P::K; ++k) w[k] = wbase[k * (N / 4)];
-    wave_toeplitz(zs.toep, reinterpret_cast<const uint32_t *>(slot + SL::CP));
-    wave_ring_mul<P::K + P::L>(zs.rows, zs.toep, it.s8);
+    wave_toeplitz(zs.toep, nzw, ngw);
+    wave_ring_mul<P::K + P::L>(zs.rows, zs.toep, B);
     wave_lds_sync();
 
     // r0 = w0 - c s2
@@ -495,43 +537,52 @@ __device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t 
             f[r] = (uint32_t)(P::GAMMA1 - z);
         }
         if (wave_any(big)) return false;
-        wave_pack_D<Z::Z_BITS>(sig_out + Z::SIG_Z + l * Z::POLYZ_BYTES, f);
+        if constexpr (WRITE) wave_pack_D<Z::Z_BITS>(sig_out + Z::SIG_Z + l * Z::POLYZ_BYTES, f);
     }
 
-    // c t0, the hints in ascending coefficient order j = 4 lane + r
-    wave_lds_sync();
-    wave_ring_mul<2 * P::K>(zs.rows + P::K * RING_ROW, zs.toep, it.t8);
-    wave_lds_sync();
+    // c t0 in two halves of K / 2 polynomials; the hints in ascending
+    // coefficient order j = 4 lane + r
     uint8_t *h = sig_out + Z::SIG_H;
     int pos = 0;
 #pragma unroll 1
-    for (int k = 0; k < P::K; ++k) {
-        int32_t cs[4], lo[4], hi[4];
-        wave_ring_row(cs, zs.rows + k * RING_ROW);
-        wave_ring_row(lo, zs.rows + (P::K + k) * RING_ROW);
-        wave_ring_row(hi, zs.rows + (2 * P::K + k) * RING_ROW);
-        const uint4 wk = wbase[k * (N / 4)];
-        const uint32_t wp[4] = {wk.x, wk.y, wk.z, wk.w};
-        bool big = false;
-        int hb[4], before = 0, cnt = 0;
+    for (int k0 = 0; k0 < P::K; k0 += P::K / 2) {
+        const int col = min(lane & 15, P::K - 1);  // low limbs, then high limbs
+        wave_ring_load(B, it.t8 + (col < P::K / 2 ? k0 + col : P::K / 2 + k0 + col) * N);
+        wave_lds_sync();  // the rows are read by now
+        wave_ring_mul<P::K>(zs.rows + P::K * RING_ROW, zs.toep, B);
+        wave_lds_sync();
+#pragma unroll 1
+        for (int k = k0; k < k0 + P::K / 2; ++k) {
+            int32_t cs[4], lo[4], hi[4];
+            wave_ring_row(cs, zs.rows + k * RING_ROW);
+            wave_ring_row(lo, zs.rows + (P::K + k - k0) * RING_ROW);
+            wave_ring_row(hi, zs.rows + (P::K + P::K / 2 + k - k0) * RING_ROW);
+            const uint4 wk = wbase[k * (N / 4)];
+            const uint32_t wp[4] = {wk.x, wk.y, wk.z, wk.w};
+            bool big = false;
+            int hb[4], before = 0, cnt = 0;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int32_t ct0 = lo[r] + 128 * hi[r];
-            big |= abs(ct0) >= P::GAMMA2;
-            hb[r] = make_hint<P>(packed_w0(wp[r]) - cs[r] + ct0, (int32_t)packed_w1(wp[r]));
-            const uint64_t m = __ballot(hb[r]);
-            before += __popcll(m & ((1ull << lane) - 1ull));  // hints of lower lanes
-            cnt += __popcll(m);
+            for (int r = 0; r < 4; ++r) {
+                const int32_t ct0 = lo[r] + 128 * hi[r];
+                big |= abs(ct0) >= P::GAMMA2;
+                hb[r] = make_hint<P>(packed_w0(wp[r]) - cs[r] + ct0, (int32_t)packed_w1(wp[r]));
+                const uint64_t m = __ballot(hb[r]);
+                before += __popcll(m & ((1ull << lane) - 1ull));  // hints of lower lanes
+                cnt += __popcll(m);
+            }
+            if (wave_any(big) || pos + cnt > P::OMEGA) return false;
+            int idx = pos + before;
+            pos += cnt;
+            if constexpr (WRITE) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (hb[r]) h[idx++] = (uint8_t)(4 * lane + r);
+                if (lane == 0) h[P::OMEGA + k] = (uint8_t)pos;
+            }
         }
-        if (wave_any(big) || pos + cnt > P::OMEGA) return false;
-        int idx = pos + before;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (hb[r]) h[idx++] = (uint8_t)(4 * lane + r);
-        pos += cnt;
-        if (lane == 0) h[P::OMEGA + k] = (uint8_t)pos;
     }
-    for (int j = pos + lane; j < P::OMEGA; j += 64) h[j] = 0;
+    if constexpr (WRITE)
+        for (int j = pos + lane; j < P::OMEGA; j += 64) h[j] = 0;
     return true;
 }
 
