@@ -5,15 +5,14 @@
 //   kg_seed   lane per key     seed (explicit or SHAKE128(le64(ctr))), then
 //                              rho | rhoprime | key = SHAKE256(seed)
 //   kg_eta    lane per s-poly  ExpandS into int8 scratch, pack eta into sk
-//   kg_main   G keys per workgroup: NTT(s1) into LDS, then one lane per
-//             ExpandA entry (G*K*L sponges) folds each accepted coefficient
-//             straight into t^[k][ctr] += mont(a, s1^[l][ctr]) with LDS
-//             atomics -- A is never stored; the sum is exact int32 so the
-//             accumulation order does not matter.  Then INTT, + s2, caddq,
-//             Power2Round and packing of t1 / t0, one wavefront per row.
-//   kg_tr     lane per key     tr = SHAKE256(pk)[0:32]
+//   kg_main   one wave per FoldCfg<P>::IPW keys: NTT(s1), A s1^ straight from
+//             the sponges (fold.hpp), then per row INTT, + s2, caddq,
+//             Power2Round and packing of t1 / t0
+//   kg_tr     tr = SHAKE256(pk)[0:32], a 16-lane row or a lane pair per key
 #include <hip/hip_runtime.h>
 
+#include "fold.hpp"
+#include "hash_row.hpp"
 #include "internal.hpp"
 #include "layout.hpp"
 #include "pipelines.hpp"
@@ -21,15 +20,6 @@
 #include "sample.hpp"
 
 namespace dil {
-
-__device__ __forceinline__ void store_le64(uint8_t *p, uint64_t v) {
-    if (((uintptr_t)p & 7) == 0) {
-        *reinterpret_cast<uint64_t *>(p) = v;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) p[i] = (uint8_t)(v >> (8 * i));
-    }
-}
 
 template <class P>
 __global__ __launch_bounds__(256) void kg_seed_kernel(KeygenArgs a) {
@@ -55,12 +45,12 @@ __global__ __launch_bounds__(256) void kg_seed_kernel(KeygenArgs a) {
     uint8_t *rp = a.scratch + i * a.scratch_pitch + KeypairLayout<P>::RHOPRIME - KeypairLayout<P>::SCRATCH;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-        store_le64(pk + 8 * w, out[w]);
-        store_le64(sk + 8 * w, out[w]);
-        store_le64(sk + SEEDBYTES + 8 * w, out[12 + w]);
+        store_any<uint64_t>(pk + 8 * w, out[w]);
+        store_any<uint64_t>(sk + 8 * w, out[w]);
+        store_any<uint64_t>(sk + SEEDBYTES + 8 * w, out[12 + w]);
     }
 #pragma unroll
-    for (int w = 0; w < 8; ++w) store_le64(rp + 8 * w, out[4 + w]);
+    for (int w = 0; w < 8; ++w) store_any<uint64_t>(rp + 8 * w, out[4 + w]);
 }
 
 template <class P>
@@ -122,79 +112,65 @@ __global__ __launch_bounds__(256) void kg_eta_kernel(KeygenArgs a) {
     });
 }
 
-// keys per workgroup of kg_main: the compiled default, and the values a
-// tiling may choose (those whose LDS fits in 160 KiB)
+// one wave per workgroup: waves of the fold need no barriers
 template <class P>
-struct KgMainCfg {
-    static constexpr int G = P::MODE == 2 ? 16 : (P::MODE == 3 ? 8 : 4);
-};
-
-template <class P, int G>
 struct KgShared {
     ZetaLds zt;
-    int32_t x[4][NTT_XBUF];
-    int32_t shat[G][P::L][LDS_ROW];
-    int32_t acc[G][P::K][LDS_ROW];
+    FoldLds<P> f;  // its windows double as the transforms' exchange buffer
+    __device__ int32_t *x() {
+        static_assert(sizeof(f.win) >= NTT_XBUF * 4, "the windows hold an exchange buffer");
+        return &f.win[0][0];
+    }
 };
 
-template <class P, int G>
-__global__ __launch_bounds__(256) void kg_main_kernel(KeygenArgs a) {
+template <class P>
+__global__ __launch_bounds__(64) void kg_main_kernel(KeygenArgs a) {
     using Z = Sizes<P>;
     using KL = KeypairLayout<P>;
-    extern __shared__ __align__(16) uint8_t smem_raw[];
-    KgShared<P, G> &sh = *reinterpret_cast<KgShared<P, G> *>(smem_raw);
-    const size_t item0 = (size_t)blockIdx.x * G;
-    const int wave = threadIdx.x >> 6;
+    constexpr int IPW = FoldCfg<P>::IPW;
+    __shared__ __align__(16) KgShared<P> sh;
+    const size_t item0 = (size_t)blockIdx.x * IPW;
+    const int lane = lane_id(), count = (int)min((size_t)IPW, a.n - item0);
+    auto s8_of = [&](int i) {
+        return reinterpret_cast<const int8_t *>(a.scratch + (item0 + i) * a.scratch_pitch + KL::S8 - KL::SCRATCH);
+    };
     zeta_lds_load(sh.zt);
-    for (int j = threadIdx.x; j < G * P::K * LDS_ROW; j += blockDim.x) (&sh.acc[0][0][0])[j] = 0;
-    __syncthreads();
 
-    // NTT(s1) for the G keys
-    for (int t = wave; t < G * P::L; t += 4) {
-        const int g = t / P::L, l = t % P::L;
-        if (item0 + g >= a.n) continue;
-        const int8_t *s8 = reinterpret_cast<const int8_t *>(a.scratch + (item0 + g) * a.scratch_pitch + KL::S8 -
-                                                            KL::SCRATCH);
+#pragma unroll 1
+    for (int t = 0; t < count * P::L; ++t) {
+        const int i = t / P::L, l = t % P::L;
         int32_t v[4];
-        wave_load_i8_A(v, s8 + l * N);
-        ntt_wave(v, sh.x[wave], sh.zt);
-        wave_store_D(sh.shat[g][l], v);
+        wave_load_i8_A(v, s8_of(i) + l * N);
+        ntt_wave(v, sh.x(), sh.zt);
+        wave_store_D(sh.f.row[i * P::K + l], v);
     }
-    __syncthreads();
 
-    // ExpandA: one sponge per (key, k, l), accepted coefficients folded into t^
-    for (int t = threadIdx.x; t < G * P::K * P::L; t += blockDim.x) {
-        const int g = t / (P::K * P::L), kl = t % (P::K * P::L);
-        const int k = kl / P::L, l = kl % P::L;
-        if (item0 + g >= a.n) continue;
-        const uint8_t *pk = a.pk + (item0 + g) * a.pk_pitch;
+    {
+        const int i = lane / (P::K * P::L);
+        const bool run = i < count;
+        const uint8_t *pk = a.pk + (item0 + (run ? i : 0)) * a.pk_pitch;
         uint64_t rho[4];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) rho[w] = load_le64(pk + 8 * w);
-        int32_t *acc = sh.acc[g][k];
-        const int32_t *s1 = sh.shat[g][l];
-        uniform_poly(rho, (uint32_t)((k << 8) | l), [&](int ctr, int32_t v) { atomicAdd(&acc[ctr], mont_mul(v, s1[ctr])); });
+        for (int w = 0; w < 4; ++w) rho[w] = load_any<uint64_t>(pk + 8 * w);
+        expand_fold<P>(sh.f, rho, run);
     }
-    __syncthreads();
 
     // t = INTT(reduce32(t^)) + s2, caddq, Power2Round, pack (keypair.cu:251-301)
-    for (int t = wave; t < G * P::K; t += 4) {
-        const int g = t / P::K, k = t % P::K;
-        const size_t item = item0 + g;
-        if (item >= a.n) continue;
+#pragma unroll 1
+    for (int t = 0; t < count * P::K; ++t) {
+        const int i = t / P::K, k = t % P::K;
+        const size_t item = item0 + i;
         int32_t v[4];
-        wave_load_D(v, sh.acc[g][k]);
+        wave_load_D(v, sh.f.row[t]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = reduce32(v[r]);
-        intt_wave(v, sh.x[wave], sh.zt);
-        const int8_t *s2 = reinterpret_cast<const int8_t *>(a.scratch + item * a.scratch_pitch + KL::S8 - KL::SCRATCH) +
-                           (P::L + k) * N;
+        intt_wave(v, sh.x(), sh.zt);
         int32_t s2v[4], t1[4], t0[4];
-        wave_load_i8_A(s2v, s2);
+        wave_load_i8_A(s2v, s8_of(i) + (P::L + k) * N);
 #pragma unroll
         for (int r = 0; r < 4; ++r) t1[r] = power2round(caddq(v[r] + s2v[r]), t0[r]);
-        layout_A_to_D(t1, sh.x[wave]);
-        layout_A_to_D(t0, sh.x[wave]);
+        layout_A_to_D(t1, sh.x());
+        layout_A_to_D(t0, sh.x());
         uint32_t f1[4], f0[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -206,21 +182,24 @@ __global__ __launch_bounds__(256) void kg_main_kernel(KeygenArgs a) {
     }
 }
 
+// tr = SHAKE256(pk)[0:32] with one 16-lane row per key: for batches whose
+// rows all find a place on the card, where the serial absorb of the public
+// key (10 / 15 / 20 permutations) is the latency
 template <class P>
-__global__ __launch_bounds__(256) void kg_tr_kernel(KeygenArgs a) {
+__global__ __launch_bounds__(256) void kg_tr_row_kernel(KeygenArgs a) {
     using Z = Sizes<P>;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n) return;
+    __shared__ uint32_t lds[4 * 4 * ROW_LDS_WORDS];
+    const RowLane r = row_lane_setup(lds, (threadIdx.x >> 6) * 4 * ROW_LDS_WORDS);
+    const size_t i = (size_t)blockIdx.x * ROW_ITEMS_PER_BLOCK + (threadIdx.x >> 4);
+    if (i >= a.n) return;  // whole rows
     const uint8_t *pk = a.pk + i * a.pk_pitch;
-    Lane64 s[25];
-    shake_absorb<SHAKE256_RATE>(s, [&](uint32_t w, uint32_t nb) {
-        return nb == 8 ? load_le64(pk + 8 * w) : load_le_partial(pk + 8 * w, nb);
-    }, (uint32_t)Z::PK_BYTES);
-    uint64_t tr[4];
-    squeeze_words<4>(s, tr);
-    uint8_t *sk = a.sk + i * a.sk_pitch + Z::SK_TR;
+    uint32_t s[5];
+    shake_row<SHAKE256_RATE>(s, r, lds, (uint32_t)Z::PK_BYTES,
+                             [&](uint32_t w) { return load_half_bytes(pk, 8 * w + 4 * r.h, Z::PK_BYTES); });
+    uint8_t *tr = a.sk + i * a.sk_pitch + Z::SK_TR;
+    if (r.active && r.y == 0)
 #pragma unroll
-    for (int w = 0; w < 4; ++w) store_le64(sk + 8 * w, tr[w]);
+        for (int x = 0; x < 4; ++x) store_any<uint32_t>(tr + 8 * x + 4 * r.h, s[x]);
 }
 
 // tr = SHAKE256(pk)[0:32] with two lanes per key (keccak_f1600_pair): the
@@ -235,39 +214,20 @@ __global__ __launch_bounds__(256) void kg_tr_pair_kernel(KeygenArgs a) {
     uint32_t s[25];
     shake_pair<SHAKE256_RATE>(s, h, (uint32_t)Z::PK_BYTES,
                               [&](uint32_t w) { return load_half_bytes(pk, 8 * w + 4 * h, Z::PK_BYTES); });
-    uint8_t *sk = a.sk + i * a.sk_pitch + Z::SK_TR;
-    const bool al = (reinterpret_cast<uintptr_t>(sk) & 3) == 0;
+    uint8_t *tr = a.sk + i * a.sk_pitch + Z::SK_TR;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        uint8_t *q = sk + 8 * w + 4 * h;
-        if (al) {
-            *reinterpret_cast<uint32_t *>(q) = s[w];
-        } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b) q[b] = (uint8_t)(s[w] >> (8 * b));
-        }
-    }
+    for (int w = 0; w < 4; ++w) store_any<uint32_t>(tr + 8 * w + 4 * h, s[w]);
 }
 
+// Keys-per-workgroup values that the tiling setter accepts (a wave's keys are
+// fixed now; recorded tilings keep loading).
 template <class P, int G>
 constexpr bool kg_fits() {
-    return sizeof(KgShared<P, G>) <= 160 * 1024;
+    return G * (P::L + P::K) * N * 4 + 8 * 1024 <= 160 * 1024;
 }
 
-template <class P, int G>
-static int launch_kg_main(const KeygenArgs &a, hipStream_t st) {
-    if constexpr (!kg_fits<P, G>()) {
-        return -1;
-    } else {
-        const size_t smem = sizeof(KgShared<P, G>);
-        // set once per kernel: a host call, not a stream operation
-        static const hipError_t attr = hipFuncSetAttribute((const void *)kg_main_kernel<P, G>,
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (attr != hipSuccess) return (int)attr;
-        hipLaunchKernelGGL((kg_main_kernel<P, G>), dim3((unsigned)((a.n + G - 1) / G)), dim3(256), smem, st, a);
-        return 0;
-    }
-}
+// 4,096 rows are one wave per SIMD
+constexpr size_t KEYGEN_ROW_MAX = 4096;
 
 template <class P>
 static int keygen_impl(const KeygenArgs &a, hipStream_t st) {
@@ -276,22 +236,13 @@ static int keygen_impl(const KeygenArgs &a, hipStream_t st) {
     const unsigned b1 = (unsigned)((a.n + 255) / 256);
     hipLaunchKernelGGL(kg_seed_kernel<P>, dim3(b1), dim3(256), 0, st, a);
     hipLaunchKernelGGL(kg_eta_kernel<P>, dim3((unsigned)((a.n * NP + 255) / 256)), dim3(256), 0, st, a);
-    int e;
-    switch (tiling_get(TILE_KEYGEN_ITEMS, P::MODE, a.n)) {
-        case 2: e = launch_kg_main<P, 2>(a, st); break;
-        case 4: e = launch_kg_main<P, 4>(a, st); break;
-        case 8: e = launch_kg_main<P, 8>(a, st); break;
-        case 16: e = launch_kg_main<P, 16>(a, st); break;
-        default: e = launch_kg_main<P, KgMainCfg<P>::G>(a, st); break;
-    }
-    if (e) return e;
-#ifndef DIL_KG_TR_PAIR
-#define DIL_KG_TR_PAIR 1  // 16,384 keys: 1-1.5 % faster keygen than one lane per key
-#endif
-    if (DIL_KG_TR_PAIR)
-        hipLaunchKernelGGL(kg_tr_pair_kernel<P>, dim3((unsigned)((a.n + 127) / 128)), dim3(256), 0, st, a);
+    constexpr int IPW = FoldCfg<P>::IPW;
+    hipLaunchKernelGGL(kg_main_kernel<P>, dim3((unsigned)((a.n + IPW - 1) / IPW)), dim3(64), 0, st, a);
+    if (a.n <= KEYGEN_ROW_MAX)
+        hipLaunchKernelGGL(kg_tr_row_kernel<P>, dim3((unsigned)((a.n + ROW_ITEMS_PER_BLOCK - 1) / ROW_ITEMS_PER_BLOCK)),
+                           dim3(256), 0, st, a);
     else
-        hipLaunchKernelGGL(kg_tr_kernel<P>, dim3(b1), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(kg_tr_pair_kernel<P>, dim3((unsigned)((a.n + 127) / 128)), dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }
 

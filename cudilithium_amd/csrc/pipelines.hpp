@@ -54,25 +54,10 @@ struct VerifyArgs {
     const uint8_t *keys;
     size_t key_pitch;
     uint32_t nkeys;
-    // Long messages: tr and mu are computed before vf_prep with one sponge
-    // per 16-lane row (vf_mu_row_kernel) and vf_prep skips them.
+    // Long messages: tr and mu with one sponge per 16-lane row whatever the
+    // batch size.
     int row_mu;
-    // Otherwise, fork_mu: tr and mu are computed with two lanes per item on
-    // an auxiliary stream beside vf_prep / vf_main (only vf_final needs mu);
-    // 0 keeps them in vf_prep on the caller's stream (no auxiliary streams).
-    int fork_mu;
 };
-// fork_mu of the verification entry points for a batch of n items: on for
-// card-filling batches (65,536 Dilithium5 items 4.85 -> 4.78 ms, 10,000
-// Dilithium2 items 1.33 -> 1.26 ms per call); off below 8,192 items, where
-// the extra streams cost concurrent callers more than the overlap gives
-// (serving saturation -30 %, ten 1,000-item callers -10 %).  The entry point
-// that allocates nothing keeps 0: it creates no auxiliary streams.
-#ifndef DIL_VERIFY_FORK_MU
-#define DIL_VERIFY_FORK_MU 1
-#endif
-constexpr size_t VERIFY_FORK_MIN_ITEMS = 8192;
-inline int verify_fork_mu(size_t n) { return DIL_VERIFY_FORK_MU && n >= VERIFY_FORK_MIN_ITEMS ? 1 : 0; }
 
 // Host-side per-item state of the per-stage scheduler, laid out as the
 // reference's sign_lut_element (api.cuh:31-34).
@@ -94,9 +79,6 @@ int launch_verify(int mode, const VerifyArgs &a, hipStream_t st, hipEvent_t *ev 
 // The fixed part of signing (mu, rhoprime, ExpandA, the int8 secret key) for
 // the chain's items; starts its list when it has one.
 int launch_sign_fixed(int mode, const SignArgs &a, const Chain &ch, hipStream_t st);
-// tr / mu of verification with one sponge per 16-lane row instead of one
-// lane: for batches of long messages
-int launch_verify_mu_row(int mode, const VerifyArgs &a, hipStream_t st);
 int launch_sign_round(int mode, const SignArgs &a, const SlotRef &sr, const uint32_t *d_exec, size_t nslot,
                       int by_item, uint8_t *d_done, hipStream_t st);
 int launch_sign_copy(int mode, const SignArgs &a, const SlotRef &sr, const uint64_t *d_copy, size_t ncopy,
