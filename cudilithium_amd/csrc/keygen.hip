@@ -4,7 +4,7 @@
 // Four launches, each with the lane mapping its work wants:
 //   kg_seed   lane per key     seed (explicit or SHAKE128(le64(ctr))), then
 //                              rho | rhoprime | key = SHAKE256(seed)
-//   kg_eta    lane per s-poly  ExpandS into int8 scratch, pack eta into sk
+//   kg_eta    lane per s-poly  ExpandS, packed into sk
 //   kg_main   one wave per FoldCfg<P>::IPW keys: NTT(s1), A s1^ straight from
 //             the sponges (fold.hpp), then per row INTT, + s2, caddq,
 //             Power2Round and packing of t1 / t0
@@ -53,63 +53,68 @@ __global__ __launch_bounds__(256) void kg_seed_kernel(KeygenArgs a) {
     for (int w = 0; w < 8; ++w) store_any<uint64_t>(rp + 8 * w, out[4 + w]);
 }
 
+// ExpandS, lane per polynomial (keypair.cu:80-130), one wave per workgroup.
+// Each lane writes every nibble to the next free byte of its LDS row and moves
+// on only past an accepted one, so a nibble costs a field extract, a byte
+// store, a compare and an add, with no branch.  The accepted nibbles are then
+// packed a row at a time by the whole wave: eta - s is the nibble itself
+// (eta 4) or the nibble mod 5 (eta 2).  16,384 Dilithium3 keys: 178 us when
+// each lane branched per nibble and stored its own row, 96 us now.
+constexpr int ETA_ROW = N + 4;  // bytes; an odd number of words apart
 template <class P>
-__global__ __launch_bounds__(256) void kg_eta_kernel(KeygenArgs a) {
+__global__ __launch_bounds__(64) void kg_eta_kernel(KeygenArgs a) {
     using Z = Sizes<P>;
-    constexpr int NP = P::L + P::K;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.n * NP) return;
-    const size_t i = t / NP;
-    const int p = (int)(t % NP);
-    uint8_t *scr = a.scratch + i * a.scratch_pitch;
-    const uint8_t *rp = scr + KeypairLayout<P>::RHOPRIME - KeypairLayout<P>::SCRATCH;
-    int8_t *s8 = reinterpret_cast<int8_t *>(scr + KeypairLayout<P>::S8 - KeypairLayout<P>::SCRATCH) + p * N;
-    uint64_t seed[8];
+    constexpr uint32_t NP = P::L + P::K, BOUND = P::ETA == 2 ? 15 : 9;
+    __shared__ __align__(16) uint8_t rows[64 * ETA_ROW];
+    const size_t t0 = (size_t)blockIdx.x * 64, total = a.n * NP;
+    const int lane = lane_id();
+    {
+        const size_t t = min(t0 + lane, total - 1);
+        const uint8_t *rp = a.scratch + t / NP * a.scratch_pitch + KeypairLayout<P>::RHOPRIME - KeypairLayout<P>::SCRATCH;
+        Lane64 s[25];
+        uint64_t in[9];
 #pragma unroll
-    for (int w = 0; w < 8; ++w) seed[w] = *reinterpret_cast<const uint64_t *>(rp + 8 * w);
-    // The coefficients arrive in order: they are collected into 16-byte
-    // stores of the int8 copy (kg_main reads it) and into
-    // the packed eta - s bit stream of the secret key (keypair.cu:116-130),
-    // written a 32-bit word at a time (bytes when the row is not 4-aligned).
-    // Lanes write different rows, so one store per coefficient made every
-    // store instruction touch 64 cache lines for a single byte each.
-    uint8_t *dst = a.sk + i * a.sk_pitch + Z::SK_S1 + p * Z::POLYETA_BYTES;
-    const bool dst4 = (reinterpret_cast<uintptr_t>(dst) & 3) == 0;
-    const bool s8_16 = (reinterpret_cast<uintptr_t>(s8) & 15) == 0;  // else 8-aligned (work pitch % 8 == 0)
-    uint32_t cur = 0, w0 = 0, w1 = 0, w2 = 0;  // int8 bytes: the current word and the last three
-    uint64_t bits = 0;
-    int nbits = 0, nout = 0;
-    // nonce l for s1[l], L + k for s2[k] (keypair.cu:84-89, 202-207)
-    eta_poly<P::ETA>(seed, (uint32_t)p, [&](int ctr, int32_t v) {
-        cur = (cur >> 8) | ((uint32_t)(uint8_t)(int8_t)v << 24);
-        if ((ctr & 3) == 3) {
-            if ((ctr & 15) == 15) {
-                if (s8_16) {
-                    reinterpret_cast<uint4 *>(s8)[ctr >> 4] = make_uint4(w0, w1, w2, cur);
-                } else {
-                    reinterpret_cast<uint2 *>(s8)[2 * (ctr >> 4)] = make_uint2(w0, w1);
-                    reinterpret_cast<uint2 *>(s8)[2 * (ctr >> 4) + 1] = make_uint2(w2, cur);
+        for (int w = 0; w < 8; ++w) in[w] = load_any<uint64_t>(rp + 8 * w);
+        in[8] = t % NP;  // nonce l for s1[l], L + k for s2[k] (keypair.cu:84-89, 202-207)
+        shake_absorb_regs<SHAKE256_RATE, CRHBYTES + 2>(s, in);
+        uint8_t *row = rows + lane * ETA_ROW;
+        uint32_t ctr = 0;
+#pragma unroll 1
+        while (__ballot(ctr < N)) {
+            keccak_f1600(s);
+            static_for<0, 2 * (SHAKE256_RATE / 8)>([&](auto h) {
+                if (__ballot(ctr < N) == 0ull) return;
+                const uint32_t w = half_word<decltype(h)::value>(s);
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    const uint32_t v = (w >> (4 * b)) & 15u;
+                    row[min(ctr, (uint32_t)N)] = (uint8_t)v;
+                    ctr += v < BOUND;
                 }
-            }
-            w0 = w1;
-            w1 = w2;
-            w2 = cur;
+            });
         }
-        bits |= (uint64_t)(uint32_t)(P::ETA - v) << nbits;
-        nbits += Z::ETA_BITS;
-        if (nbits >= 32) {
-            const uint32_t word = (uint32_t)bits;
-            if (dst4) {
-                reinterpret_cast<uint32_t *>(dst)[nout] = word;
-            } else {
-#pragma unroll
-                for (int b = 0; b < 4; ++b) dst[4 * nout + b] = (uint8_t)(word >> (8 * b));
+    }
+    wave_lds_sync();
+    const int count = (int)min((size_t)64, total - t0);
+#pragma unroll 4
+    for (int r = 0; r < count; ++r) {
+        const size_t t = t0 + r;
+        uint8_t *dst = a.sk + t / NP * a.sk_pitch + Z::SK_S1 + t % NP * Z::POLYETA_BYTES;
+        const uint32_t d = reinterpret_cast<const uint32_t *>(rows + r * ETA_ROW)[lane];
+        if constexpr (P::ETA == 4) {
+            const uint32_t x = d | d >> 4;
+            store_any<uint16_t>(dst + 2 * lane, (uint16_t)((x & 0xFFu) | (x >> 8 & 0xFF00u)));
+        } else {
+            // per byte: minus 5 for v >= 5 and again for v >= 10
+            const uint32_t m = d - 5u * ((d + 0x7B7B7B7Bu >> 7 & 0x01010101u) + (d + 0x76767676u >> 7 & 0x01010101u));
+            const uint32_t f = (m & 7u) | (m >> 5 & 7u << 3) | (m >> 10 & 7u << 6) | (m >> 15 & 7u << 9);
+            const uint32_t v = f | pair_other(f) << 12;
+            if ((lane & 1) == 0) {
+                store_any<uint16_t>(dst + 3 * (lane >> 1), (uint16_t)v);
+                dst[3 * (lane >> 1) + 2] = (uint8_t)(v >> 16);
             }
-            ++nout;
-            bits >>= 32;
-            nbits -= 32;
         }
-    });
+    }
 }
 
 // one wave per workgroup: waves of the fold need no barriers
@@ -126,13 +131,16 @@ struct KgShared {
 template <class P>
 __global__ __launch_bounds__(64) void kg_main_kernel(KeygenArgs a) {
     using Z = Sizes<P>;
-    using KL = KeypairLayout<P>;
     constexpr int IPW = FoldCfg<P>::IPW;
     __shared__ __align__(16) KgShared<P> sh;
     const size_t item0 = (size_t)blockIdx.x * IPW;
     const int lane = lane_id(), count = (int)min((size_t)IPW, a.n - item0);
-    auto s8_of = [&](int i) {
-        return reinterpret_cast<const int8_t *>(a.scratch + (item0 + i) * a.scratch_pitch + KL::S8 - KL::SCRATCH);
+    // polynomial p of s1 | s2, packed in the secret key as eta - s
+    auto load_s = [&](int32_t (&v)[4], int i, int p) {
+        uint32_t f[4];
+        wave_fields_A<Z::ETA_BITS>(f, a.sk + (item0 + i) * a.sk_pitch + Z::SK_S1 + p * Z::POLYETA_BYTES);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = P::ETA - (int32_t)f[r];
     };
     zeta_lds_load(sh.zt);
 
@@ -140,7 +148,7 @@ __global__ __launch_bounds__(64) void kg_main_kernel(KeygenArgs a) {
     for (int t = 0; t < count * P::L; ++t) {
         const int i = t / P::L, l = t % P::L;
         int32_t v[4];
-        wave_load_i8_A(v, s8_of(i) + l * N);
+        load_s(v, i, l);
         ntt_wave(v, sh.x(), sh.zt);
         wave_store_D(sh.f.row[i * P::K + l], v);
     }
@@ -166,7 +174,7 @@ __global__ __launch_bounds__(64) void kg_main_kernel(KeygenArgs a) {
         for (int r = 0; r < 4; ++r) v[r] = reduce32(v[r]);
         intt_wave(v, sh.x(), sh.zt);
         int32_t s2v[4], t1[4], t0[4];
-        wave_load_i8_A(s2v, s8_of(i) + (P::L + k) * N);
+        load_s(s2v, i, P::L + k);
 #pragma unroll
         for (int r = 0; r < 4; ++r) t1[r] = power2round(caddq(v[r] + s2v[r]), t0[r]);
         layout_A_to_D(t1, sh.x());
@@ -235,7 +243,7 @@ static int keygen_impl(const KeygenArgs &a, hipStream_t st) {
     constexpr int NP = P::L + P::K;
     const unsigned b1 = (unsigned)((a.n + 255) / 256);
     hipLaunchKernelGGL(kg_seed_kernel<P>, dim3(b1), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(kg_eta_kernel<P>, dim3((unsigned)((a.n * NP + 255) / 256)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(kg_eta_kernel<P>, dim3((unsigned)((a.n * NP + 63) / 64)), dim3(64), 0, st, a);
     constexpr int IPW = FoldCfg<P>::IPW;
     hipLaunchKernelGGL(kg_main_kernel<P>, dim3((unsigned)((a.n + IPW - 1) / IPW)), dim3(64), 0, st, a);
     if (a.n <= KEYGEN_ROW_MAX)

@@ -18,11 +18,9 @@ struct KeypairLayout {
     static constexpr size_t PK = 0;
     static constexpr size_t SK = align256(Z::PK_BYTES);
     static constexpr size_t SCRATCH = SK + align256(Z::SK_BYTES);
-    // scratch: rhoprime (64 B) then s1 | s2 as int8 polynomials
+    // scratch: rhoprime (64 B); the rest of the reference's K polynomials is unused
     static constexpr size_t RHOPRIME = SCRATCH;
-    static constexpr size_t S8 = SCRATCH + 64;
     static constexpr size_t ROW = SCRATCH + (size_t)P::K * N * 4;
-    static_assert(64 + (P::L + P::K) * N <= P::K * N * 4, "keypair scratch fits the reference row");
     // reference formula (test_vectors.cu:64-70)
     static constexpr size_t REF_ROW = align256(Z::PK_BYTES) + align256(Z::SK_BYTES) + (size_t)P::K * N * 4;
 };

@@ -148,12 +148,6 @@ __device__ __forceinline__ void wave_load_challenge_A(int32_t (&v)[4], const uin
     }
 }
 
-__device__ __forceinline__ void wave_load_i8_A(int32_t (&v)[4], const int8_t *p) {
-    const int l = lane_id();
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = p[64 * r + l];
-}
-
 // Wave-wide OR of a per-lane predicate.
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0ull; }
 

@@ -8,8 +8,6 @@
 //
 //   uniform_poly   ExpandA entry, SHAKE128(rho || le16(nonce)), 23-bit
 //                  candidates < q (sign.cu:98-163, keypair.cu:140-189)
-//   eta_poly       ExpandS entry, SHAKE256(rhoprime || le16(nonce)), nibbles
-//                  (keypair.cu:80-115)
 //   mask_raw       ExpandMask squeeze of 5 SHAKE256 blocks (sign.cu:463-526)
 //   challenge      SampleInBall (sign.cu:710-734, verify.cu:221-245)
 //
@@ -93,37 +91,6 @@ __device__ __forceinline__ void uniform_poly(const uint64_t (&rho)[4], uint32_t 
                     ++ctr;
                 }
             });
-        });
-    } while (ctr < N);
-}
-
-template <int ETA, class Sink>
-__device__ __forceinline__ void eta_poly(const uint64_t (&seed)[8], uint32_t nonce, Sink &&sink) {
-    Lane64 s[25];
-    const uint64_t in[9] = {seed[0], seed[1], seed[2], seed[3], seed[4],
-                            seed[5], seed[6], seed[7], (uint64_t)(nonce & 0xFFFF)};
-    shake_absorb_regs<SHAKE256_RATE, CRHBYTES + 2>(s, in);
-    int ctr = 0;
-    do {
-        keccak_f1600(s);
-        // 17 state words, 16 nibbles each, low nibble first
-        static_for<0, 2 * (SHAKE256_RATE / 8)>([&](auto h) {
-            uint32_t w = half_word<decltype(h)::value>(s);
-#pragma unroll 2
-            for (int b = 0; b < 8; ++b, w >>= 4) {
-                const uint32_t t = w & 15u;
-                if constexpr (ETA == 2) {
-                    if (t < 15u && ctr < N) {
-                        sink(ctr, 2 - (int32_t)(t - ((205u * t) >> 10) * 5u));
-                        ++ctr;
-                    }
-                } else {
-                    if (t < 9u && ctr < N) {
-                        sink(ctr, 4 - (int32_t)t);
-                        ++ctr;
-                    }
-                }
-            }
         });
     } while (ctr < N);
 }
