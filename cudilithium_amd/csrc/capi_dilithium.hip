@@ -704,11 +704,11 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
 }
 
 
-// Attempt slots of a context for small batches: enough that each item gets 16
+// Attempt slots of a context for small batches: enough that each item gets 32
 // consecutive nonces per round (a round's latency is the same for one or for
 // thousands of attempts), at most 8,192 (about 130 MB).
 static size_t round_slots_for(size_t max_batch, size_t nslots) {
-    return std::max({nslots, 2 * max_batch, std::min<size_t>(16 * max_batch, 8192)});
+    return std::max({nslots, 2 * max_batch, std::min<size_t>(32 * max_batch, 8192)});
 }
 
 static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots, size_t round_slots,

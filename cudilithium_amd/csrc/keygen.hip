@@ -106,7 +106,7 @@ __global__ __launch_bounds__(64) void kg_eta_kernel(KeygenArgs a) {
             store_any<uint16_t>(dst + 2 * lane, (uint16_t)((x & 0xFFu) | (x >> 8 & 0xFF00u)));
         } else {
             // per byte: minus 5 for v >= 5 and again for v >= 10
-            const uint32_t m = d - 5u * ((d + 0x7B7B7B7Bu >> 7 & 0x01010101u) + (d + 0x76767676u >> 7 & 0x01010101u));
+            const uint32_t m = d - 5u * ((((d + 0x7B7B7B7Bu) >> 7) & 0x01010101u) + (((d + 0x76767676u) >> 7) & 0x01010101u));
             const uint32_t f = (m & 7u) | (m >> 5 & 7u << 3) | (m >> 10 & 7u << 6) | (m >> 15 & 7u << 9);
             const uint32_t v = f | pair_other(f) << 12;
             if ((lane & 1) == 0) {

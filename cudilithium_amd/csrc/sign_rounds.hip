@@ -10,11 +10,12 @@
 //
 //   fixed  mu / rhoprime, ExpandA and the int8 secret key, one launch whose
 //          workgroups take one of the three roles
-//   y      lane (or lane pair) per mask sponge
+//   y      lane, lane pair or 16-lane row per mask sponge
 //   w      wave per attempt
-//   c      lane pair per attempt
-//   z      wave per attempt; the first in nonce order that passes is the
-//          specification's signature of its item
+//   c      lane pair or 16-lane row per attempt
+//   z      wave per attempt: the checks of r0 and z
+//   s      wave per item: the first of its attempts in nonce order that passed
+//          them and passes c t0 and the hints is the specification's signature
 //   plan   one workgroup lists the items without a signature and plans the
 //          next round (how many items, how many consecutive nonces for each),
 //          so the host issues a fixed sequence of launches and never waits.
@@ -24,9 +25,14 @@
 //
 // The sequence is as long as the expected decay of the batch needs; what is
 // left after it (rarely anything) is finished by the persistent kernel, which
-// takes its items from the same queue.  Large batches run as two chains of
-// rounds on two streams, so that the hash launches of one fill the SIMDs that
-// the other leaves idle.
+// takes its items from the same queue.  The largest batches run as two chains
+// of rounds on two streams, so that the hash launches of one fill the SIMDs
+// that the other leaves idle.
+//
+// 16,384 Dilithium3 items in one chain: fixed 401 us; the rounds' y 490, w
+// 725, c 510, z 290, s 257 and plan 60 us.  y and c are serial chains of
+// permutations in every round (c 64 us with lane pairs for any number up to
+// 32,768), w and z bound by their vector instructions and memory waits.
 //
 // The reference issues its rounds from the host with a synchronisation and
 // about eight small copies per round (api.cu:208-441).
@@ -48,15 +54,25 @@ constexpr uint32_t ROUND_MAX_M = 32;  // attempts per item and round
 // chain gives (3,001 Dilithium5 items with messages up to 4 KiB: fixed stage
 // 394 us with lane pairs, 174 us with rows).
 constexpr uint32_t FIXED_ROW_MAX = 4096;
-// Larger batches go to the persistent kernel, whose workgroups need no
-// launches between stages: 10,000 Dilithium2 items (drop-in) 2.79 ms in
-// rounds, 2.82 ms persistent; 16,384 Dilithium3 items 3.14 and 2.82 ms; 3,001
-// Dilithium5 items 1.18 and 1.43 ms; 1,000 Dilithium2 items 0.44 and 0.81 ms;
-// 17 Dilithium3 items 0.30 and 0.79 ms.
-constexpr size_t ROUNDS_MAX_ITEMS = 4096;
-// Attempts a round aims at when few items are left, and the least per item (a
-// second attempt reads the item's A from L2).
-constexpr size_t ROUND_TARGET = 8192;
+// The persistent kernel, which needs no launches between stages, runs what is
+// left after the rounds and calls with fewer slots than half their items (a
+// round then covers a small part of them).  Rounds with enough slots are
+// faster at every size: 17 Dilithium3 items 0.22 ms (persistent 0.79), 1,000
+// Dilithium2 items 0.37 (0.79), 3,001 Dilithium5 0.98 (1.17), 8,000 Dilithium5
+// 1.73 (2.43), 10,000 Dilithium2 1.29 (1.72), 16,384 Dilithium3 2.45 (2.83),
+// 40,000 Dilithium3 5.0 (5.65).
+constexpr size_t ROUNDS_MAX_ITEMS_PER_SLOT = 2;
+// Two chains from this batch on: 16,384 Dilithium3 items 2.45 ms (one chain
+// 2.60), 40,000 5.03 (5.36), 14,000 2.19 (2.29), 16,384 Dilithium5 2.87
+// (2.84); smaller ones lose as much as they gain (12,288 Dilithium2 1.46 and
+// 1.44 ms, Dilithium3 2.13 and 2.14, 10,000 Dilithium2 1.29 and 1.28).
+constexpr size_t TWO_CHAINS_MIN = 12288;
+// Attempts a round aims at when few items are left, and the least per item.
+// A second attempt reads the item's A from L2 and saves rounds: 40,000
+// Dilithium3 items 5.03 ms, 5.62 with a least of one; 16,384 2.50 and 2.71.
+// Targets of 8,192 / 16,384 attempts: 10,000 Dilithium2 items 1.41 / 1.28 ms,
+// 16,384 Dilithium3 2.69 / 2.60, 8,000 Dilithium5 1.74 / 1.73.
+constexpr size_t ROUND_TARGET = 16384;
 constexpr uint32_t ROUND_MIN_M = 2;
 
 // items and attempts per item of a round over u waiting items
@@ -131,8 +147,9 @@ __device__ __forceinline__ Attempt slot_attempt(const Chain &ch, const ChainCtl 
 // Layout of a round's hashes by their number.  A chained permutation of a
 // lone wave takes 8.6 / 5.9 / 3.5 us with one, two or sixteen lanes per
 // state, and the card runs 9.6 / 7.4 / 2.1 G permutations/s: the row form
-// while its waves have SIMDs of their own, then the pair form, then one lane.
-constexpr uint32_t Y_ROW_MAX = 4096, Y_PAIR_MAX = 32768, C_ROW_MAX = 4096;
+// while its waves are few (8,192 challenges with rows 40 us, with pairs 64),
+// then the pair form, then one lane.
+constexpr uint32_t Y_ROW_MAX = 4096, Y_PAIR_MAX = 32768, C_ROW_MAX = 8192;
 constexpr uint32_t ROW_LDS = 4 * 4 * ROW_LDS_WORDS;
 
 template <class P>
@@ -216,46 +233,46 @@ __global__ __launch_bounds__(256) void sg_rc_kernel(SignArgs a, SlotRef sr, Chai
 
 constexpr uint32_t ENTRY_DONE = 0xFFFFFFFFu;  // item of an entry whose signature is written
 
-// The attempts are latency-bound (a few dependent rounds of memory per
-// attempt, little arithmetic), so an item's attempts are checked by waves of
-// their own: W waves per item, the first attempt writing its signature as it
-// goes; if only a later one passes, it is run again to write.
+// The attempts are latency-bound (a few dependent rounds of memory each, little
+// arithmetic) and most end early, so r0 and z are checked by a wave and a
+// workgroup per attempt, which leave the CU as soon as they are decided.
 template <class P>
-__global__ __launch_bounds__(64 * ROUND_WAVES) void sg_rz_kernel(SignArgs a, SlotRef sr, Chain ch) {
+__global__ __launch_bounds__(64) void sg_rz_kernel(SignArgs a, SlotRef sr, Chain ch) {
     using SL = SlotLayout<P>;
-    __shared__ ZScratch<P> zs[ROUND_WAVES];
-    __shared__ uint32_t best[ROUND_WAVES];
+    __shared__ ZScratch<P, true> zs;
     const ChainCtl c = *chain_ctl<P>(ch);
-    const uint32_t w = threadIdx.x >> 6, lane = (uint32_t)lane_id();
-    const uint32_t W = c.m == 1 ? 1 : c.m == 2 ? 2 : 4, per = ROUND_WAVES / W, sub = w / W, j0 = w % W;
-    for (uint32_t o0 = blockIdx.x * per; o0 < c.count; o0 += gridDim.x * per) {
-        if (threadIdx.x < ROUND_WAVES) best[threadIdx.x] = c.m;
-        __syncthreads();
-        const uint32_t o = o0 + sub;
-        const bool have = o < c.count;
-        uint2 *const entry = chain_entry(ch, c.cur, have ? o : 0);
+    const uint32_t slots = c.count * c.m;
+    for (uint32_t s = blockIdx.x; s < slots; s += gridDim.x) {
+        uint8_t *slot = sr.base + s * sr.pitch;
+        const bool ok = stage_z<P, true>(a, slot_attempt(ch, c, s).item, slot, nullptr, zs);
+        if (lane_id() == 0) *reinterpret_cast<uint32_t *>(slot + SL::FLAG) = ok;
+    }
+}
+
+// Wave per item: the first of its attempts that passed the checks and also
+// passes c t0 and the hints is its signature.
+template <class P>
+__global__ __launch_bounds__(64) void sg_rs_kernel(SignArgs a, SlotRef sr, Chain ch) {
+    using SL = SlotLayout<P>;
+    __shared__ ZScratch<P> zs;
+    const ChainCtl c = *chain_ctl<P>(ch);
+    const uint32_t lane = (uint32_t)lane_id();
+    for (uint32_t o = blockIdx.x; o < c.count; o += gridDim.x) {
+        uint2 *const entry = chain_entry(ch, c.cur, o);
         const uint2 e = *entry;
+        uint8_t *const slots = sr.base + (size_t)o * c.m * sr.pitch;
+        uint32_t passed = 0;  // m <= ROUND_MAX_M <= 32
+        if (lane < c.m) passed = *reinterpret_cast<const uint32_t *>(slots + lane * sr.pitch + SL::FLAG);
+        uint64_t left = __ballot(passed != 0);
         uint8_t *dst = a.sig + (size_t)e.x * a.sig_pitch;
-        auto slot_of = [&](uint32_t j) { return sr.base + (size_t)(o * c.m + j) * sr.pitch; };
-        if (have) {
-            for (uint32_t j = j0; j < c.m && j < *(volatile uint32_t *)&best[sub]; j += W) {
-                const bool ok = j == 0 ? stage_z<P, true>(a, e.x, slot_of(j), dst, zs[w])
-                                       : stage_z<P, false>(a, e.x, slot_of(j), dst, zs[w]);
-                if (ok) {
-                    if (lane == 0) atomicMin(&best[sub], j);
-                    break;
-                }
-            }
-        }
-        __syncthreads();
-        if (have) {
-            const uint32_t j = best[sub];
-            if (j == c.m) {
-                if (j0 == 0 && lane == 0) entry->y = e.y + c.m;
-            } else if (j0 == j % W) {
-                const uint8_t *ct = slot_of(j) + SL::CT;
-                if (j) (void)stage_z<P, true>(a, e.x, slot_of(j), dst, zs[w]);
-                if (lane < SEEDBYTES) dst[lane] = ct[lane];
+        bool done = false;
+        while (left && !done) {
+            const uint32_t j = (uint32_t)__ffsll((unsigned long long)left) - 1;
+            left &= left - 1;
+            uint8_t *slot = slots + j * sr.pitch;
+            done = stage_z<P>(a, e.x, slot, dst, zs);
+            if (done) {
+                if (lane < SEEDBYTES) dst[lane] = slot[SL::CT + lane];
                 if (lane == 0) {
                     *reinterpret_cast<uint32_t *>(a.rows + (size_t)e.x * a.row_pitch + SignLayout<P>::ATTEMPTS) =
                         e.y + j + 1;
@@ -263,7 +280,7 @@ __global__ __launch_bounds__(64 * ROUND_WAVES) void sg_rz_kernel(SignArgs a, Slo
                 }
             }
         }
-        __syncthreads();  // best is read before the next items reset it
+        if (!done && lane == 0) entry->y = e.y + c.m;
     }
 }
 
@@ -276,28 +293,28 @@ __global__ __launch_bounds__(PLAN_THREADS) void sg_plan_kernel(Chain ch, uint32_
     const ChainCtl c = *cc;
     if (c.left == 0) return;  // count is 0 already
     const uint32_t t = threadIdx.x, w = t >> 6, lane = t & 63;
-    // thread t keeps the order of entries [t * per, (t + 1) * per)
-    const uint32_t per = (c.left + PLAN_THREADS - 1) / PLAN_THREADS, e0 = t * per, e1 = min(e0 + per, c.left);
-    uint32_t alive = 0;
-    for (uint32_t e = e0; e < e1; ++e) alive += chain_entry(ch, c.cur, e)->x != ENTRY_DONE;
-    uint32_t incl = alive;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t v = (uint32_t)__shfl_up((int)incl, d);
-        if (lane >= (uint32_t)d) incl += v;
-    }
-    if (lane == 63) sums[w] = incl;
+    // wave w keeps the order of its run of entries, 64 at a time
+    const uint32_t run = ((c.left + PLAN_THREADS - 1) / PLAN_THREADS) * 64, e0 = w * run, e1 = min(e0 + run, c.left);
+    auto alive = [&](uint32_t e, uint2 &v) {
+        v = e < e1 ? *chain_entry(ch, c.cur, e) : make_uint2(ENTRY_DONE, 0);
+        return v.x != ENTRY_DONE;
+    };
+    uint32_t count = 0;
+    uint2 v;
+    for (uint32_t e = e0; e < e1; e += 64) count += __popcll(__ballot(alive(e + lane, v)));
+    if (lane == 0) sums[w] = count;
     __syncthreads();
-    uint32_t before = 0, total = 0;
+    uint32_t at = 0, total = 0;
 #pragma unroll
     for (uint32_t i = 0; i < PLAN_THREADS / 64; ++i) {
-        before += i < w ? sums[i] : 0u;
+        at += i < w ? sums[i] : 0u;
         total += sums[i];
     }
-    uint32_t at = before + incl - alive;
-    for (uint32_t e = e0; e < e1; ++e) {
-        const uint2 v = *chain_entry(ch, c.cur, e);
-        if (v.x != ENTRY_DONE) *chain_entry(ch, c.cur ^ 1, at++) = v;
+    for (uint32_t e = e0; e < e1; e += 64) {
+        const bool keep = alive(e + lane, v);
+        const uint64_t mask = __ballot(keep);
+        if (keep) *chain_entry(ch, c.cur ^ 1, at + __popcll(mask & ((1ull << lane) - 1ull))) = v;
+        at += __popcll(mask);
     }
     if (t == 0) {
         ChainCtl nx{total, 0, 0, c.cur ^ 1, 0};
@@ -337,19 +354,32 @@ int launch_round(const SignArgs &a, const SlotRef &sr, const Chain &ch, double &
     const double fail = P::MODE == 2 ? 1.0 - 1.0 / 4.25 : P::MODE == 3 ? 1.0 - 1.0 / 5.1 : 1.0 - 1.0 / 3.85;
     uint32_t count, m;
     plan_round((uint32_t)std::ceil(u), ch.nslots, ch.target, count, m);
-    // grids for the expected round (every kernel strides over what there is)
-    const uint32_t slots = count * m;
+    // The count on the device differs from the expected one by a few percent, and
+    // an attempt more than a hash grid holds costs its wave a second chain of
+    // permutations (13,700 challenge hashes 62 us, 120 us with a grid for 13,600).
+    // So the grids cover the largest need within an eighth of the expectation,
+    // over every form and m that such a count selects; blocks without work exit.
+    const uint32_t lo = count - count / 8, hi = std::min(count + count / 8 + 64, ch.n);
+    const uint32_t most = std::min(ch.nslots, std::max(hi * ROUND_MIN_M, std::min(hi * ROUND_MAX_M, ch.target)));
+    const uint32_t slots = std::min(most, count * m + count * m / 8 + 64);
     auto blocks = [](uint32_t units, uint32_t per, uint32_t cap) {
         return dim3(std::max(1u, std::min((units + per - 1) / per, cap)));
     };
-    const uint32_t total = slots * P::L;
-    const uint32_t lanes = total <= Y_ROW_MAX ? 16 * total : total <= Y_PAIR_MAX ? 2 * total : total;
-    hipLaunchKernelGGL(sg_ry_kernel<P>, blocks(lanes, 256, 4096), dim3(256), 0, st, a, sr, ch);
+    auto lanes_y = [](uint32_t t) { return t <= Y_ROW_MAX ? 16 * t : t <= Y_PAIR_MAX ? 2 * t : t; };
+    auto lanes_c = [](uint32_t t) { return t <= C_ROW_MAX ? 16 * t : 2 * t; };
+    auto widest = [](auto f, uint32_t from, uint32_t to, uint32_t edge) {
+        return std::max(f(to), edge >= from && edge <= to ? f(edge) : 0u);
+    };
+    const uint32_t least = std::min(lo * ROUND_MIN_M, most);
+    uint32_t ly = widest(lanes_y, least * P::L, most * P::L, Y_ROW_MAX);
+    ly = std::max(ly, widest(lanes_y, least * P::L, most * P::L, Y_PAIR_MAX));
+    const uint32_t lc = widest(lanes_c, least, most, C_ROW_MAX);
+    const dim3 gy = blocks(ly, 256, 4096), gc = blocks(lc, 256, 4096);
+    hipLaunchKernelGGL(sg_ry_kernel<P>, gy, dim3(256), 0, st, a, sr, ch);
     hipLaunchKernelGGL(sg_rw_kernel<P>, blocks(slots, ROUND_WAVES, 8192), dim3(64 * ROUND_WAVES), 0, st, a, sr, ch);
-    hipLaunchKernelGGL(sg_rc_kernel<P>, blocks((slots <= C_ROW_MAX ? 16 : 2) * slots, 256, 4096), dim3(256), 0, st,
-                       a, sr, ch);
-    hipLaunchKernelGGL(sg_rz_kernel<P>, blocks(m == 1 ? (count + 3) / 4 : m == 2 ? (count + 1) / 2 : count, 1, 8192),
-                       dim3(64 * ROUND_WAVES), 0, st, a, sr, ch);
+    hipLaunchKernelGGL(sg_rc_kernel<P>, gc, dim3(256), 0, st, a, sr, ch);
+    hipLaunchKernelGGL(sg_rz_kernel<P>, blocks(slots, 1, 32768), dim3(64), 0, st, a, sr, ch);
+    hipLaunchKernelGGL(sg_rs_kernel<P>, blocks(hi, 1, 32768), dim3(64), 0, st, a, sr, ch);
     hipLaunchKernelGGL(sg_plan_kernel<P>, dim3(1), dim3(PLAN_THREADS), 0, st, ch, ctl);
     u = (u > count ? u - count : 0.0) + std::min(u, (double)count) * std::pow(fail, m);
     return (int)hipGetLastError();
@@ -360,9 +390,8 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
               uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st, hipEvent_t fixed_done) {
     int e = launch_zero_ctl(ctl, phase_sums, st);
     if (e) return e;
-    const bool rounds = !phase_sums && a.n <= ROUNDS_MAX_ITEMS;
-    // two chains of at least 2,048 items
-    const int nchain = rounds && a.n >= 4096 ? 2 : 1;
+    const bool rounds = !phase_sums && a.n <= ROUNDS_MAX_ITEMS_PER_SLOT * nslots;
+    const int nchain = rounds && a.n >= TWO_CHAINS_MIN ? 2 : 1;
     AuxStreams *aux = nullptr;
     std::unique_lock<std::mutex> guard;
     if (nchain == 2) {
@@ -375,7 +404,7 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
     Chain ch[2];
     SlotRef csr[2];
     hipStream_t cs[2];
-    double u[2];
+    double u[2] = {0.0, 0.0};
     size_t first = 0, slot = 0;
     for (int k = 0; k < nchain; ++k) {
         const size_t n = a.n * (k + 1) / nchain - first, ns = nslots * (k + 1) / nchain - slot;
@@ -404,7 +433,7 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
                                       st);
     }
     // the chains' rounds in turn, so that neither stream waits for the host
-    for (int r = 0; r < 48 && (u[0] > 0.05 || (nchain == 2 && u[1] > 0.05)); ++r)
+    for (int r = 0; r < 48 && (u[0] > 0.05 || u[1] > 0.05); ++r)
         for (int k = 0; k < nchain; ++k)
             if (u[k] > 0.05 && (e = launch_round<P>(a, csr[k], ch[k], u[k], ctl, cs[k]))) return e;
     for (int k = 0; k < nchain; ++k)

@@ -126,50 +126,7 @@ __device__ __forceinline__ void load_words8(uint64_t (&w)[8], const uint8_t *p) 
 
 // ---------------------------------------------------------------- fixed part
 
-template <class P>
-__device__ __forceinline__ void stage_mu(const SignArgs &a, size_t i) {
-    using Z = Sizes<P>;
-    using SLy = SignLayout<P>;
-    const uint8_t *sk = a.sk + sk_index(a, i) * a.sk_pitch;
-    uint64_t tr[4], key[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        tr[w] = load_le64(sk + Z::SK_TR + 8 * w);
-        key[w] = load_le64(sk + Z::SK_KEY + 8 * w);
-    }
-    const uint8_t *m = a.m.ptr(i);
-    const uint32_t mlen = a.m.len(i);
-    Lane64 s[25];
-    shake_absorb<SHAKE256_RATE>(s, [&](uint32_t w, uint32_t nb) -> uint64_t {
-        if (w < 4) return w == 0 ? tr[0] : (w == 1 ? tr[1] : (w == 2 ? tr[2] : tr[3]));
-        const uint8_t *p = m + 8 * (w - 4);
-        return nb == 8 ? load_le64(p) : load_le_partial(p, nb);
-    }, SEEDBYTES + mlen);
-    uint64_t in[12];
-    uint64_t mu[8];
-    squeeze_words<8>(s, mu);
-    uint64_t rp[8];
-    if (a.rnd) {
-        const uint8_t *r = a.rnd + i * a.rnd_pitch;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) rp[w] = load_le64(r + 8 * w);
-    } else {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) in[w] = key[w];
-#pragma unroll
-        for (int w = 0; w < 8; ++w) in[4 + w] = mu[w];
-        shake_absorb_regs<SHAKE256_RATE, SEEDBYTES + CRHBYTES>(s, in);
-        squeeze_words<8>(s, rp);
-    }
-    uint64_t *dst = reinterpret_cast<uint64_t *>(a.rows + i * a.row_pitch + SLy::MU);
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-        dst[w] = mu[w];
-        dst[8 + w] = rp[w];
-    }
-}
-
-// stage_mu with two lanes per item (keccak_f1600_pair): lane h of the pair
+// mu and rhoprime with two lanes per item (keccak_f1600_pair): lane h of the pair
 // holds the 32-bit halves h of the state.  A permutation takes 2/3 of the
 // one-lane form's time for 1.2 x its instructions, so the serial absorb of
 // the batch's longest message, which bounds the fixed stage, is shorter.
@@ -470,9 +427,9 @@ __device__ __forceinline__ void stage_c_pair(const SignArgs &a, size_t item, uin
 // rows c s2 (K) | c s1 (L); once z is written, the rows c t0 of half of the
 // K polynomials at a time (low limbs K / 2, high limbs K / 2) take the place
 // of c s1.
-template <class P>
+template <class P, bool CHECK_ONLY = false>
 struct ZScratch {
-    static constexpr int ROWS = P::K + (P::L > P::K ? P::L : P::K);
+    static constexpr int ROWS = P::K + (CHECK_ONLY || P::L > P::K ? P::L : P::K);
     uint32_t toep[TOEP_WORDS];
     uint16_t rows[ROWS * RING_ROW];
 };
@@ -487,10 +444,11 @@ struct ZScratch {
 // hints.  All values are exact integers below q / 2, where the reference's
 // representatives mod q agree with them.  Fields of a rejected attempt's
 // sig_out are left partly written.
-// WRITE false: the checks only.
-template <class P, bool WRITE = true>
+// CHECK_ONLY: r0 and z are checked and nothing is written; c t0 and the hints
+// (which reject about 2 % of what is left) are not looked at.
+template <class P, bool CHECK_ONLY = false>
 __device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t *slot, uint8_t *sig_out,
-                                        ZScratch<P> &zs) {
+                                        ZScratch<P, CHECK_ONLY> &zs) {
     using Z = Sizes<P>;
     using SL = SlotLayout<P>;
     const ItemView<P> it(a, item);
@@ -537,8 +495,9 @@ __device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t 
             f[r] = (uint32_t)(P::GAMMA1 - z);
         }
         if (wave_any(big)) return false;
-        if constexpr (WRITE) wave_pack_D<Z::Z_BITS>(sig_out + Z::SIG_Z + l * Z::POLYZ_BYTES, f);
+        if constexpr (!CHECK_ONLY) wave_pack_D<Z::Z_BITS>(sig_out + Z::SIG_Z + l * Z::POLYZ_BYTES, f);
     }
+    if constexpr (CHECK_ONLY) return true;
 
     // c t0 in two halves of K / 2 polynomials; the hints in ascending
     // coefficient order j = 4 lane + r
@@ -573,16 +532,13 @@ __device__ __forceinline__ bool stage_z(const SignArgs &a, size_t item, uint8_t 
             if (wave_any(big) || pos + cnt > P::OMEGA) return false;
             int idx = pos + before;
             pos += cnt;
-            if constexpr (WRITE) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (hb[r]) h[idx++] = (uint8_t)(4 * lane + r);
-                if (lane == 0) h[P::OMEGA + k] = (uint8_t)pos;
-            }
+            for (int r = 0; r < 4; ++r)
+                if (hb[r]) h[idx++] = (uint8_t)(4 * lane + r);
+            if (lane == 0) h[P::OMEGA + k] = (uint8_t)pos;
         }
     }
-    if constexpr (WRITE)
-        for (int j = pos + lane; j < P::OMEGA; j += 64) h[j] = 0;
+    for (int j = pos + lane; j < P::OMEGA; j += 64) h[j] = 0;
     return true;
 }
 

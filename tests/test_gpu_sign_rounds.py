@@ -1,6 +1,6 @@
 """Signing at the batch sizes where its launches change: one item, a few, the
-edges of a list chunk (512 entries), and the line between rounds and the
-persistent kernel; signatures and attempt counts equal the oracle's, through
+edges of a list chunk (512 entries), the line between the forms of the message
+hash and the one between one and two chains of rounds; signatures and attempt counts equal the oracle's, through
 the device entry point and through the drop-in call with few temp rows."""
 import numpy as np
 import pytest
@@ -29,6 +29,16 @@ def test_signatures_and_attempts_match_oracle(mode, n):
         assert np.array_equal(ctx.sign(msgs, sk), exp)
         assert np.array_equal(ctx.attempt_counts(n), att)
         assert ctx.executed_attempts() >= int(att.sum())
+
+
+@pytest.mark.parametrize("n", [12287, 12288, 12801])
+def test_two_chains_match_oracle(n):
+    from cudilithium_amd.api import SignContext
+    msgs, sk = _batch(2, n, n)
+    exp, att = oracle.sign_batch(2, msgs, sk)
+    ctx = SignContext(2, n)
+    assert np.array_equal(ctx.sign(msgs, sk), exp)
+    assert np.array_equal(ctx.attempt_counts(n), att)
 
 
 @pytest.mark.parametrize("n,threshold", [(1, 1), (3, 1), (600, 1), (600, 7), (600, 600), (513, 2048)])
