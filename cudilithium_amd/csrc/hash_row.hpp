@@ -1,10 +1,12 @@
-// Message hashing with one sponge per 16-lane row: the device code shared by
-// the kernels of hash_row.hip and the signing rounds' fixed stage.
+// Hashes with one sponge per 16-lane row or per wavefront, for the launches
+// whose chains of permutations are longer than the card's work beside them:
+// mu / rhoprime, the mask sponges and the challenges.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include "keccak_row.hpp"
+#include "keccak_wave.hpp"
 #include "sign_stages.hpp"
 
 namespace dil {
@@ -71,28 +73,6 @@ __device__ __forceinline__ void stage_mu_row(const SignArgs &a, size_t i, const 
         return sh.get(lds, w - 4, h);
     });
     row_store_words(t, r, reinterpret_cast<uint32_t *>(row + SLy::RHOPRIME), 8);
-}
-
-// mask_raw with one sponge per 16-lane row: 5 squeezed SHAKE256 blocks of
-// rhoprime || le16(nonce) to out; run false: the row takes part in the
-// permutations (DPP reads whole rows) and writes nothing.
-__device__ __forceinline__ void mask_raw_row(const uint32_t *rhoprime, uint32_t nonce, uint32_t *out,
-                                             const RowLane &r, uint32_t *lds, bool run) {
-    uint32_t a[5];
-#pragma unroll
-    for (int x = 0; x < 5; ++x) {
-        const uint32_t w = row_word(r, x);
-        a[x] = r.active && w < 8 && run ? rhoprime[2 * w + r.h] : 0u;
-        // 66 input bytes: le16(nonce) and the domain byte 0x1F in the low half
-        // of word 8, the final bit in the high half of word 16
-        if (r.active && w == 8 && r.h == 0) a[x] = (nonce & 0xFFFFu) | (0x1Fu << 16);
-        if (r.active && w == SHAKE256_RATE / 8 - 1 && r.h == 1) a[x] = 0x80000000u;
-    }
-#pragma unroll 1
-    for (int b = 0; b < 5; ++b) {
-        keccak_f1600_row(a, r, lds);
-        if (run) row_store_words(a, r, out + 2 * 17 * b, SHAKE256_RATE / 8);
-    }
 }
 
 // LDS words per row of challenge_row: the block, the accepted positions, the
@@ -193,6 +173,127 @@ __device__ __forceinline__ void stage_c_row(const uint32_t *mu, const uint32_t *
         if (r.active && w == SHAKE256_RATE / 8 - 1 && r.h == 1) a[x] = 0x80000000u;
     }
     challenge_row<P::TAU>(a, masks, r, lds, my, run);
+}
+
+// ------------------------------------------------- one sponge per wavefront
+
+// 8 bytes at off of a buffer of len bytes (bytes past the end zero)
+__device__ __forceinline__ uint64_t load_word_bytes(const uint8_t *p, uint32_t off, uint32_t len) {
+    if (off + 8 <= len) return load_any<uint64_t>(p + off);
+    uint64_t v = 0;
+    for (uint32_t b = 0; off + b < len; ++b) v |= (uint64_t)p[off + b] << (8 * b);
+    return v;
+}
+
+// stage_mu_row by a wave; lds: its WAVE_LDS_WORDS words at base
+template <class P>
+__device__ __forceinline__ void stage_mu_wave(const SignArgs &a, size_t i, const WaveLane &r, uint32_t *lds,
+                                              uint32_t base) {
+    using Z = Sizes<P>;
+    using SLy = SignLayout<P>;
+    const uint8_t *sk = a.sk + sk_index(a, i) * a.sk_pitch;
+    const uint8_t *m = a.m.ptr(i);
+    const uint32_t mlen = a.m.len(i);
+    uint32_t lo, hi;
+    shake_wave<SHAKE256_RATE>(lo, hi, r, lds, SEEDBYTES + mlen, [&](uint32_t w) -> uint64_t {
+        return w < 4 ? load_word_bytes(sk + Z::SK_TR, 8 * w, SEEDBYTES) : load_word_bytes(m, 8 * (w - 4), mlen);
+    });
+    uint8_t *row = a.rows + i * a.row_pitch;
+    wave_store_words(lo, hi, r, reinterpret_cast<uint32_t *>(row + SLy::MU), 8);
+    uint32_t *rhoprime = reinterpret_cast<uint32_t *>(row + SLy::RHOPRIME);
+    if (a.rnd) {
+        const uint32_t g = (uint32_t)lane_id();
+        if (g < CRHBYTES / 4) rhoprime[g] = load_half_bytes(a.rnd + i * a.rnd_pitch, 4 * g, CRHBYTES);
+        return;
+    }
+    // rhoprime = SHAKE256(key || mu): mu's words change lanes through LDS (the
+    // area of the pi exchange, free after the permutation)
+    wave_store_words(lo, hi, r, lds + base, 8);
+    wave_lds_sync();
+    shake_wave<SHAKE256_RATE>(lo, hi, r, lds, SEEDBYTES + CRHBYTES, [&](uint32_t w) -> uint64_t {
+        return w < 4 ? load_word_bytes(sk + Z::SK_KEY, 8 * w, SEEDBYTES)
+                     : *reinterpret_cast<const uint64_t *>(lds + base + 2 * (w - 4));
+    });
+    wave_store_words(lo, hi, r, rhoprime, 8);
+}
+
+// mask_raw by a wave: 5 squeezed SHAKE256 blocks of rhoprime || le16(nonce)
+__device__ __forceinline__ void mask_raw_wave(const uint32_t *rhoprime, uint32_t nonce, uint32_t *out,
+                                              const WaveLane &r, uint32_t *lds) {
+    // 66 input bytes: le16(nonce) and the domain byte 0x1F in word 8, the final
+    // bit in word 16
+    uint32_t lo = r.w < 8 ? rhoprime[2 * r.w] : 0u, hi = r.w < 8 ? rhoprime[2 * r.w + 1] : 0u;
+    if (r.w == 8) lo = (nonce & 0xFFFFu) | (0x1Fu << 16);
+    if (r.w == SHAKE256_RATE / 8 - 1) hi = 0x80000000u;
+#pragma unroll 1
+    for (int b = 0; b < 5; ++b) {
+        keccak_f1600_wave(lo, hi, r, lds);
+        wave_store_words(lo, hi, r, out + 2 * 17 * b, SHAKE256_RATE / 8);
+    }
+}
+
+// challenge_row by a wave, each lane following one sign; my: as for a row
+template <int TAU>
+__device__ __forceinline__ void challenge_wave(uint32_t lo, uint32_t hi, uint32_t *masks, const WaveLane &r,
+                                               uint32_t *lds, uint32_t *my) {
+    static_assert(TAU <= 64, "a sign per lane");
+    constexpr uint32_t BLOCK = 2 * (SHAKE256_RATE / 8);
+    const uint32_t lane = (uint32_t)lane_id();
+    uint32_t *list = my + BLOCK, *mk = list + 16;
+    uint8_t *lb = reinterpret_cast<uint8_t *>(list);
+    uint32_t n = 0, sign0 = 0, sign1 = 0;
+    for (uint32_t start = 2; n < TAU; start = 0) {
+        keccak_f1600_wave(lo, hi, r, lds);
+        wave_store_words(lo, hi, r, my, SHAKE256_RATE / 8);
+        wave_lds_sync();
+        if (start) {
+            sign0 = my[0];
+            sign1 = my[1];
+        }
+        for (uint32_t k = start; k < BLOCK && n < TAU; ++k) {
+            uint32_t v = my[k];
+#pragma unroll
+            for (int b = 0; b < 4; ++b, v >>= 8) {
+                const uint32_t byte = v & 0xFFu;
+                if (byte <= N - TAU + n && n < TAU) {
+                    if (lane == 0) lb[n] = (uint8_t)byte;
+                    ++n;
+                }
+            }
+        }
+        wave_lds_sync();  // the block is read before the next one overwrites it
+    }
+    if (lane < 16) mk[lane] = 0u;
+    wave_lds_sync();
+    uint32_t pos = 0xFFFFu;
+#pragma unroll 8
+    for (int j = 0; j < TAU; ++j) {
+        const uint32_t b = lb[j];
+        pos = pos == b ? (uint32_t)(N - TAU + j) : pos;
+        pos = lane == (uint32_t)j ? b : pos;
+    }
+    if (lane < TAU) {
+        const uint32_t bit = 1u << (pos & 31), neg = ((lane < 32 ? sign0 : sign1) >> (lane & 31)) & 1u;
+        atomicOr(&mk[pos >> 5], bit);
+        if (neg) atomicOr(&mk[8 + (pos >> 5)], bit);
+    }
+    wave_lds_sync();
+    if (lane < 16) masks[lane] = mk[lane];
+}
+
+// stage_c by a wave
+template <class P>
+__device__ __forceinline__ void stage_c_wave(const uint32_t *mu, const uint32_t *w1, uint32_t *ct, uint32_t *masks,
+                                             const WaveLane &r, uint32_t *lds, uint32_t *my) {
+    uint32_t lo, hi;
+    shake_wave<SHAKE256_RATE>(lo, hi, r, lds, Sizes<P>::CHASH_IN_BYTES, [&](uint32_t w) -> uint64_t {
+        const uint32_t *src = w < 8 ? mu + 2 * w : w1 + 2 * (w - 8);
+        return src[0] | (uint64_t)src[1] << 32;
+    });
+    wave_store_words(lo, hi, r, ct, SEEDBYTES / 8);
+    lo = r.w < 4 ? lo : (r.w == 4 ? 0x1Fu : 0u);
+    hi = r.w < 4 ? hi : (r.w == SHAKE256_RATE / 8 - 1 ? 0x80000000u : 0u);
+    challenge_wave<P::TAU>(lo, hi, masks, r, lds, my);
 }
 
 }  // namespace dil

@@ -10,9 +10,9 @@
 //
 //   fixed  mu / rhoprime, ExpandA and the int8 secret key, one launch whose
 //          workgroups take one of the three roles
-//   y      lane, lane pair or 16-lane row per mask sponge
+//   y      lane, lane pair or wave per mask sponge
 //   w      wave per attempt
-//   c      lane pair or 16-lane row per attempt
+//   c      lane pair, 16-lane row or wave per attempt
 //   z      wave per attempt: the checks of r0 and z
 //   s      wave per item: the first of its attempts in nonce order that passed
 //          them and passes c t0 and the hints is the specification's signature
@@ -54,6 +54,11 @@ constexpr uint32_t ROUND_MAX_M = 32;  // attempts per item and round
 // chain gives (3,001 Dilithium5 items with messages up to 4 KiB: fixed stage
 // 394 us with lane pairs, 174 us with rows).
 constexpr uint32_t FIXED_ROW_MAX = 4096;
+// With a wave each up to these, the second with resident keys, where nothing
+// runs beside the hashes (messages up to 4 KiB, whole call with waves / rows:
+// 1,000 Dilithium3 items 465 / 517 us, 2,000 Dilithium5 691 / 713, 3,001
+// Dilithium5 960 / 938; resident 3,000 Dilithium5 862 / 910).
+constexpr uint32_t FIXED_WAVE_MAX = 2048, FIXED_WAVE_MAX_RESIDENT = 3072;
 // The persistent kernel, which needs no launches between stages, runs what is
 // left after the rounds and calls with fewer slots than half their items (a
 // round then covers a small part of them).  Rounds with enough slots are
@@ -91,20 +96,24 @@ struct FixedGrid {
     uint32_t mu, expand, prep;  // workgroups of each role
 };
 
-template <class P, bool ROW>
+// lanes per message hash
+enum { MU_PAIR = 2, MU_ROW = 16, MU_WAVE = 64 };
+
+template <class P, int LANES>
 __global__ __launch_bounds__(256) void sg_fixed_kernel(SignArgs a, Chain ch, FixedGrid g) {
     constexpr int KL = P::K * P::L, PREP = (P::L + 2 * P::K) * (N / 8);
-    __shared__ uint32_t lds[ROW ? 4 * 4 * ROW_LDS_WORDS : 1];
+    __shared__ __align__(8) uint32_t
+        lds[LANES == MU_WAVE ? 4 * WAVE_LDS_WORDS : LANES == MU_ROW ? 4 * 4 * ROW_LDS_WORDS : 1];
     uint32_t b = blockIdx.x;
     if (b < g.mu) {
         // serial chains, which end the stage: highest issue priority
         __builtin_amdgcn_s_setprio(3);
         const uint32_t t = threadIdx.x;
-        const uint32_t i = ROW ? b * ROW_ITEMS_PER_BLOCK + (t >> 4) : b * 128 + (t >> 1);
+        const uint32_t i = b * (256 / LANES) + t / LANES;
         RowLane r;
-        if constexpr (ROW) r = row_lane_setup(lds, (t >> 6) * 4 * ROW_LDS_WORDS);
-        if (i >= ch.n) return;  // whole rows / pairs of lanes
-        if ((t & (ROW ? 15 : 1)) == 0) {
+        if constexpr (LANES == MU_ROW) r = row_lane_setup(lds, (t >> 6) * 4 * ROW_LDS_WORDS);
+        if (i >= ch.n) return;  // whole waves / rows / pairs of lanes
+        if (t % LANES == 0) {
             if (ch.lists) *chain_entry(ch, 0, i) = make_uint2(ch.first + i, 0);
             if (ch.lists && i == 0) {
                 ChainCtl c{ch.n, 0, 0, 0, 0};
@@ -112,7 +121,10 @@ __global__ __launch_bounds__(256) void sg_fixed_kernel(SignArgs a, Chain ch, Fix
                 *chain_ctl<P>(ch) = c;
             }
         }
-        if constexpr (ROW)
+        if constexpr (LANES == MU_WAVE) {
+            const uint32_t base = (t >> 6) * WAVE_LDS_WORDS;
+            stage_mu_wave<P>(a, ch.first + i, wave_lane_setup(lds, base), lds, base);
+        } else if constexpr (LANES == MU_ROW)
             stage_mu_row<P>(a, ch.first + i, r, lds, t >> 6);
         else
             stage_mu_pair<P>(a, ch.first + i, t & 1);
@@ -145,32 +157,34 @@ __device__ __forceinline__ Attempt slot_attempt(const Chain &ch, const ChainCtl 
 }
 
 // Layout of a round's hashes by their number.  A chained permutation of a
-// lone wave takes 8.6 / 5.9 / 3.5 us with one, two or sixteen lanes per
-// state, and the card runs 9.6 / 7.4 / 2.1 G permutations/s: the row form
-// while its waves are few (8,192 challenges with rows 40 us, with pairs 64),
-// then the pair form, then one lane.
-constexpr uint32_t Y_ROW_MAX = 4096, Y_PAIR_MAX = 32768, C_ROW_MAX = 8192;
+// lone wave takes 8.6 / 5.9 / 3.5 / 2.2 us with one, two, sixteen or 64 lanes
+// per state, and the card runs 9.6 / 7.4 / 2.1 / 0.9 G permutations/s: the
+// wave form while its waves are few, then rows (challenges: 8,192 take 40 us,
+// with pairs 64; there is no such range for the shorter mask chains), pairs
+// and one lane.  17 resident Dilithium3 items 151 us (157 with 2,048 for both
+// limits, 218 without the wave form), 3,001 Dilithium5 919 (938, 977).
+constexpr uint32_t Y_WAVE_MAX = 4096, Y_PAIR_MAX = 32768;
+constexpr uint32_t C_WAVE_MAX = 4096, C_ROW_MAX = 8192;
 constexpr uint32_t ROW_LDS = 4 * 4 * ROW_LDS_WORDS;
+static_assert(ROW_LDS >= 4 * WAVE_LDS_WORDS, "the row form's LDS also serves the wave form");
 
 template <class P>
 __global__ __launch_bounds__(256) void sg_ry_kernel(SignArgs a, SlotRef sr, Chain ch) {
     using SL = SlotLayout<P>;
-    __shared__ uint32_t lds[ROW_LDS];
+    __shared__ __align__(8) uint32_t lds[4 * WAVE_LDS_WORDS];
     const ChainCtl c = *chain_ctl<P>(ch);
     const uint32_t total = c.count * c.m * P::L, stride = gridDim.x * 256;
     uint32_t t = blockIdx.x * 256 + threadIdx.x;
     __builtin_amdgcn_s_setprio(2);
-    if (total <= Y_ROW_MAX) {
-        const RowLane r = row_lane_setup(lds, (threadIdx.x >> 6) * 4 * ROW_LDS_WORDS);
-        // whole waves: rows past the end run along without storing
-        for (; (t & ~63u) < 16 * total; t += stride) {
-            const bool run = t < 16 * total;
-            const uint32_t q = run ? t >> 4 : 0, s = q / P::L, l = q % P::L;
+    if (total <= Y_WAVE_MAX) {
+        const WaveLane r = wave_lane_setup(lds, (threadIdx.x >> 6) * WAVE_LDS_WORDS);
+        for (; t < 64 * total; t += stride) {
+            const uint32_t q = t >> 6, s = q / P::L, l = q % P::L;
             const Attempt at = slot_attempt(ch, c, s);
-            mask_raw_row(reinterpret_cast<const uint32_t *>(a.rows + at.item * a.row_pitch + SignLayout<P>::RHOPRIME),
-                         P::L * at.nonce + l,
-                         reinterpret_cast<uint32_t *>(sr.base + s * sr.pitch + SL::YRAW + l * Sizes<P>::YRAW_BYTES), r,
-                         lds, run);
+            mask_raw_wave(reinterpret_cast<const uint32_t *>(a.rows + at.item * a.row_pitch + SignLayout<P>::RHOPRIME),
+                          P::L * at.nonce + l,
+                          reinterpret_cast<uint32_t *>(sr.base + s * sr.pitch + SL::YRAW + l * Sizes<P>::YRAW_BYTES),
+                          r, lds);
         }
     } else if (total <= Y_PAIR_MAX) {
         for (; t < 2 * total; t += stride) {
@@ -204,13 +218,24 @@ __global__ __launch_bounds__(64 * ROUND_WAVES) void sg_rw_kernel(SignArgs a, Slo
 template <class P>
 __global__ __launch_bounds__(256) void sg_rc_kernel(SignArgs a, SlotRef sr, Chain ch) {
     using SL = SlotLayout<P>;
-    __shared__ uint32_t lds[ROW_LDS];
+    __shared__ __align__(8) uint32_t lds[ROW_LDS];
     __shared__ uint32_t chal[16 * CHALLENGE_ROW_WORDS];
     const ChainCtl c = *chain_ctl<P>(ch);
     const uint32_t slots = c.count * c.m, stride = gridDim.x * 256;
     uint32_t t = blockIdx.x * 256 + threadIdx.x;
     __builtin_amdgcn_s_setprio(2);
-    if (slots <= C_ROW_MAX) {
+    if (slots <= C_WAVE_MAX) {
+        const WaveLane r = wave_lane_setup(lds, (threadIdx.x >> 6) * WAVE_LDS_WORDS);
+        for (; t < 64 * slots; t += stride) {
+            const uint32_t s = t >> 6;
+            uint8_t *slot = sr.base + s * sr.pitch;
+            const uint8_t *row = a.rows + slot_attempt(ch, c, s).item * a.row_pitch;
+            stage_c_wave<P>(reinterpret_cast<const uint32_t *>(row + SignLayout<P>::MU),
+                            reinterpret_cast<const uint32_t *>(slot + SL::W1PK),
+                            reinterpret_cast<uint32_t *>(slot + SL::CT), reinterpret_cast<uint32_t *>(slot + SL::CP),
+                            r, lds, chal + (threadIdx.x >> 6) * CHALLENGE_ROW_WORDS);
+        }
+    } else if (slots <= C_ROW_MAX) {
         const RowLane r = row_lane_setup(lds, (threadIdx.x >> 6) * 4 * ROW_LDS_WORDS);
         for (; (t & ~63u) < 16 * slots; t += stride) {
             const bool run = t < 16 * slots;
@@ -333,18 +358,21 @@ size_t chain_chunks(size_t n) { return (n + CHAIN_CHUNK - 1) / CHAIN_CHUNK; }
 template <class P>
 int launch_fixed(const SignArgs &a, const Chain &ch, hipStream_t st) {
     constexpr int KL = P::K * P::L, PREP = (P::L + 2 * P::K) * (N / 8);
-    // one sponge per 16-lane row where the rows of all messages fit the card
-    // beside the other roles, or on request
-    const bool row = a.row_mu || ch.n <= FIXED_ROW_MAX;
+    // one sponge per wave or 16-lane row where those of all messages fit the
+    // card beside the other roles, or (rows) on request
+    const int lanes = ch.n <= (a.key_idx ? FIXED_WAVE_MAX_RESIDENT : FIXED_WAVE_MAX) ? MU_WAVE : a.row_mu || ch.n <= FIXED_ROW_MAX ? MU_ROW : MU_PAIR;
+    const uint32_t per = 256 / lanes;
     FixedGrid g;
-    g.mu = row ? (ch.n + ROW_ITEMS_PER_BLOCK - 1) / ROW_ITEMS_PER_BLOCK : (ch.n + 127) / 128;
+    g.mu = (ch.n + per - 1) / per;
     g.expand = a.key_idx ? 0 : (uint32_t)(((size_t)ch.n * KL + 255) / 256);  // resident keys are expanded
     g.prep = a.key_idx ? 0 : (uint32_t)(((size_t)ch.n * PREP + 255) / 256);
     const dim3 grid(g.mu + g.expand + g.prep);
-    if (row)
-        hipLaunchKernelGGL((sg_fixed_kernel<P, true>), grid, dim3(256), 0, st, a, ch, g);
+    if (lanes == MU_WAVE)
+        hipLaunchKernelGGL((sg_fixed_kernel<P, MU_WAVE>), grid, dim3(256), 0, st, a, ch, g);
+    else if (lanes == MU_ROW)
+        hipLaunchKernelGGL((sg_fixed_kernel<P, MU_ROW>), grid, dim3(256), 0, st, a, ch, g);
     else
-        hipLaunchKernelGGL((sg_fixed_kernel<P, false>), grid, dim3(256), 0, st, a, ch, g);
+        hipLaunchKernelGGL((sg_fixed_kernel<P, MU_PAIR>), grid, dim3(256), 0, st, a, ch, g);
     return (int)hipGetLastError();
 }
 
@@ -365,15 +393,18 @@ int launch_round(const SignArgs &a, const SlotRef &sr, const Chain &ch, double &
     auto blocks = [](uint32_t units, uint32_t per, uint32_t cap) {
         return dim3(std::max(1u, std::min((units + per - 1) / per, cap)));
     };
-    auto lanes_y = [](uint32_t t) { return t <= Y_ROW_MAX ? 16 * t : t <= Y_PAIR_MAX ? 2 * t : t; };
-    auto lanes_c = [](uint32_t t) { return t <= C_ROW_MAX ? 16 * t : 2 * t; };
-    auto widest = [](auto f, uint32_t from, uint32_t to, uint32_t edge) {
-        return std::max(f(to), edge >= from && edge <= to ? f(edge) : 0u);
+    auto lanes_y = [](uint32_t t) {
+        return t <= Y_WAVE_MAX ? 64 * t : t <= Y_PAIR_MAX ? 2 * t : t;
+    };
+    auto lanes_c = [](uint32_t t) { return t <= C_WAVE_MAX ? 64 * t : t <= C_ROW_MAX ? 16 * t : 2 * t; };
+    auto widest = [](auto f, uint32_t from, uint32_t to, std::initializer_list<uint32_t> edges) {
+        uint32_t most = f(to);
+        for (const uint32_t e : edges) most = std::max(most, e >= from && e <= to ? f(e) : 0u);
+        return most;
     };
     const uint32_t least = std::min(lo * ROUND_MIN_M, most);
-    uint32_t ly = widest(lanes_y, least * P::L, most * P::L, Y_ROW_MAX);
-    ly = std::max(ly, widest(lanes_y, least * P::L, most * P::L, Y_PAIR_MAX));
-    const uint32_t lc = widest(lanes_c, least, most, C_ROW_MAX);
+    const uint32_t ly = widest(lanes_y, least * P::L, most * P::L, {Y_WAVE_MAX, Y_PAIR_MAX});
+    const uint32_t lc = widest(lanes_c, least, most, {C_WAVE_MAX, C_ROW_MAX});
     const dim3 gy = blocks(ly, 256, 4096), gc = blocks(lc, 256, 4096);
     hipLaunchKernelGGL(sg_ry_kernel<P>, gy, dim3(256), 0, st, a, sr, ch);
     hipLaunchKernelGGL(sg_rw_kernel<P>, blocks(slots, ROUND_WAVES, 8192), dim3(64 * ROUND_WAVES), 0, st, a, sr, ch);

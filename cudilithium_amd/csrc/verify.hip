@@ -5,8 +5,8 @@
 //   vf_prep   lane per item: c = SampleInBall(c~).  Small batches leave it to
 //             vf_main, one 16-lane row per item
 //   vf_main   workgroups of two roles, side by side:
-//             mu    tr = H(pk), mu = H(tr || m): a 16-lane row, a lane pair or
-//                   a lane per item by batch size; only vf_final needs it
+//             mu    tr = H(pk), mu = H(tr || m): a wave, a 16-lane row or
+//                   a lane pair per item by batch size; only vf_final needs it
 //             main  one wave per FoldCfg<P>::IPW items: hint decoding, z unpack
 //                   + norm check + NTT, A z^ straight from the sponges
 //                   (fold.hpp), then per row - c^ t1^ 2^d, INTT, caddq,
@@ -27,10 +27,19 @@
 namespace dil {
 
 // Batches up to this size (one row wave per SIMD) are latency-bound: hashes
-// take a 16-lane row each and vf_main samples the challenges itself.  2,500
+// take a 16-lane row or a wave each and vf_main samples the challenges itself.  2,500
 // resident Dilithium3 verifications with messages up to 4 KiB 655 -> 174 us,
 // 16 Dilithium2 verifications 309 -> 141 us against one lane per hash.
 constexpr size_t VERIFY_ROW_MAX = 4096;
+// The smallest of them take a wave per hash, up to the second limit with
+// resident keys, where no ExpandA runs beside the hashes (waves / rows: 16
+// Dilithium2 items 128 / 141 us, 1,000 Dilithium5 138 / 151, 1,500 Dilithium2
+// 205 / 151; resident, messages up to 4 KiB, 1,000 Dilithium3 52 / 72, 2,500
+// Dilithium3 122 / 175, 4,000 Dilithium2 187 / 172).
+constexpr size_t VERIFY_WAVE_MAX = 1024, VERIFY_WAVE_MAX_RESIDENT = 3072;
+static bool wave_hashes(const VerifyArgs &a) {
+    return a.n <= (a.key_idx ? VERIFY_WAVE_MAX_RESIDENT : VERIFY_WAVE_MAX);
+}
 // Beyond, c~' = H(mu || w1') with two lanes per item while those waves fit the
 // card twice, else one.
 constexpr size_t VERIFY_PAIR_MAX = 32768;
@@ -49,10 +58,11 @@ __global__ __launch_bounds__(256) void vf_prep_kernel(VerifyArgs a) {
 
 // ------------------------------------------------------------------ mu role
 
-enum MuForm { MU_ROW, MU_PAIR };
+// lanes per message hash
+enum MuForm { MU_PAIR = 2, MU_ROW = 16, MU_WAVE = 64 };
 template <int FORM>
 constexpr int mu_items(int threads) {
-    return threads / (FORM == MU_ROW ? 16 : 2);
+    return threads / FORM;
 }
 
 // tr = SHAKE256(pk)[0:32] (or the resident key's) and mu = SHAKE256(tr || m)
@@ -109,19 +119,49 @@ __device__ __forceinline__ void mu_row(const VerifyArgs &a, size_t i, const RowL
     row_store_words(s, r, reinterpret_cast<uint32_t *>(a.work + i * a.work_pitch + VL::HASH), 8);
 }
 
-// one workgroup's share of the mu role; lds: ROW_LDS_WORDS * 4 words per wave
-// (row form)
+// the same by a wave; lds: its WAVE_LDS_WORDS words at base
+template <class P>
+__device__ __forceinline__ void mu_wave(const VerifyArgs &a, size_t i, const WaveLane &r, uint32_t *lds,
+                                        uint32_t base) {
+    using Z = Sizes<P>;
+    using VL = VerifyLayout<P>;
+    uint32_t lo, hi;
+    const uint8_t *key = a.key_idx ? a.keys + a.key_idx[i] * a.key_pitch : nullptr;
+    if (!key) {
+        const uint8_t *pk = a.pk + i * a.pk_pitch;
+        shake_wave<SHAKE256_RATE>(lo, hi, r, lds, (uint32_t)Z::PK_BYTES,
+                                  [&](uint32_t w) { return load_word_bytes(pk, 8 * w, Z::PK_BYTES); });
+    } else if (r.w < 4) {
+        const uint64_t v = load_word_bytes(key + KeyLayout<P>::TR, 8 * r.w, SEEDBYTES);
+        lo = (uint32_t)v;
+        hi = (uint32_t)(v >> 32);
+    }
+    // tr's words stay on their lanes: words 0..3 of the next input
+    const uint64_t tr = r.w < 4 ? lo | (uint64_t)hi << 32 : 0ull;
+    const uint8_t *m = a.m.ptr(i);
+    const uint32_t mlen = a.m.len(i);
+    shake_wave<SHAKE256_RATE>(lo, hi, r, lds, SEEDBYTES + mlen, [&](uint32_t w) -> uint64_t {
+        return w < 4 ? tr : load_word_bytes(m, 8 * (w - 4), mlen);
+    });
+    wave_store_words(lo, hi, r, reinterpret_cast<uint32_t *>(a.work + i * a.work_pitch + VL::HASH), 8);
+}
+
+// one workgroup's share of the mu role; lds: ROW_LDS_WORDS * 4 words per wave,
+// 8-byte aligned (row and wave forms)
 template <class P, int FORM>
 __device__ __forceinline__ void mu_role(const VerifyArgs &a, uint32_t block, uint32_t *lds) {
     // serial chains that end the call: highest issue priority
     __builtin_amdgcn_s_setprio(3);
     const uint32_t t = threadIdx.x;
-    const size_t i = (size_t)block * mu_items<FORM>(blockDim.x) + t / (FORM == MU_ROW ? 16 : 2);
+    const size_t i = (size_t)block * mu_items<FORM>(blockDim.x) + t / FORM;
     RowLane r;
     if constexpr (FORM == MU_ROW) r = row_lane_setup(lds, (t >> 6) * 4 * ROW_LDS_WORDS);
-    // whole rows / pairs of lanes; vf_main rejects an index past the store
+    // whole waves / rows / pairs of lanes; vf_main rejects an index past the store
     if (i >= a.n || (a.key_idx && a.key_idx[i] >= a.nkeys)) return;
-    if constexpr (FORM == MU_ROW)
+    if constexpr (FORM == MU_WAVE) {
+        const uint32_t base = (t >> 6) * WAVE_LDS_WORDS;
+        mu_wave<P>(a, i, wave_lane_setup(lds, base), lds, base);
+    } else if constexpr (FORM == MU_ROW)
         mu_row<P>(a, i, r, lds, t >> 6);
     else
         mu_pair<P>(a, i, t & 1);
@@ -220,7 +260,7 @@ struct VfShared {
     uint32_t cp[FoldCfg<P>::IPW][16];  // challenge masks (OWN_C)
     union {
         FoldLds<P> f;                    // its windows double as the transforms' exchange buffer
-        uint32_t mu[4 * ROW_LDS_WORDS];  // mu role
+        __align__(8) uint32_t mu[4 * ROW_LDS_WORDS];  // mu role
         struct {                         // sampling the challenges, before the rest
             uint32_t row[4 * ROW_LDS_WORDS];
             uint32_t chal[4 * CHALLENGE_ROW_WORDS];
@@ -327,7 +367,7 @@ struct VfResShared {
     uint32_t bits[G][P::K * 8];
     int fail[G];
     uint32_t cp[G][16];                  // challenge masks (OWN_C)
-    uint32_t mu[4 * 4 * ROW_LDS_WORDS];  // mu role
+    __align__(8) uint32_t mu[4 * 4 * ROW_LDS_WORDS];  // mu role
     uint32_t chal[16 * CHALLENGE_ROW_WORDS];
 };
 
@@ -416,15 +456,17 @@ __global__ __launch_bounds__(256) void vf_res_kernel(VerifyArgs a, uint32_t mu_b
     }
 }
 
-enum FinalForm { FINAL_ROW, FINAL_PAIR, FINAL_LANE };
+// lanes per hash
+enum FinalForm { FINAL_LANE = 1, FINAL_PAIR = 2, FINAL_ROW = 16, FINAL_WAVE = 64 };
 
-// c~' = SHAKE256(mu || w1')[0:32] against c~, one row / pair / lane per item
+// c~' = SHAKE256(mu || w1')[0:32] against c~, one wave / row / pair / lane per item
 template <class P, int FORM>
 __global__ __launch_bounds__(256) void vf_final_kernel(VerifyArgs a) {
     using Z = Sizes<P>;
     using VL = VerifyLayout<P>;
-    __shared__ uint32_t lds[FORM == FINAL_ROW ? 4 * 4 * ROW_LDS_WORDS : 1];
-    constexpr int PER = FORM == FINAL_ROW ? 16 : FORM == FINAL_PAIR ? 2 : 1;
+    __shared__ __align__(8) uint32_t
+        lds[FORM == FINAL_WAVE ? 4 * WAVE_LDS_WORDS : FORM == FINAL_ROW ? 4 * 4 * ROW_LDS_WORDS : 1];
+    constexpr int PER = FORM;
     const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, i = t / PER;
     RowLane r;
     if constexpr (FORM == FINAL_ROW) r = row_lane_setup(lds, (threadIdx.x >> 6) * 4 * ROW_LDS_WORDS);
@@ -437,7 +479,16 @@ __global__ __launch_bounds__(256) void vf_final_kernel(VerifyArgs a) {
     }
     const uint8_t *sig = a.sig + i * a.sig_pitch;
     const uint32_t *hin = reinterpret_cast<const uint32_t *>(work + VL::HASH);
-    if constexpr (FORM == FINAL_ROW) {
+    if constexpr (FORM == FINAL_WAVE) {
+        const WaveLane wl = wave_lane_setup(lds, (threadIdx.x >> 6) * WAVE_LDS_WORDS);
+        uint32_t lo, hi;
+        shake_wave<SHAKE256_RATE>(lo, hi, wl, lds, Z::CHASH_IN_BYTES,
+                                  [&](uint32_t w) { return hin[2 * w] | (uint64_t)hin[2 * w + 1] << 32; });
+        const bool diff = wl.main && wl.w < 4 &&
+                          (lo | (uint64_t)hi << 32) != load_any<uint64_t>(sig + 8 * wl.w);
+        const bool bad = wave_any(diff);
+        if (lane_id() == 0) *ret = bad ? -1 : 0;
+    } else if constexpr (FORM == FINAL_ROW) {
         uint32_t s[5];
         shake_row<SHAKE256_RATE>(s, r, lds, Z::CHASH_IN_BYTES, [&](uint32_t w) { return hin[2 * w + r.h]; });
         bool diff = false;
@@ -493,6 +544,7 @@ static int launch_vf_res_g(const VerifyArgs &a, bool row, bool own_c, hipStream_
             hipLaunchKernelGGL(kernel, dim3(mu + (unsigned)((a.n + G - 1) / G)), dim3(256), smem, st, a, mu);
             return (int)hipGetLastError();
         };
+        if (wave_hashes(a)) return go(vf_res_kernel<P, G, MU_WAVE, true>, mu_items<MU_WAVE>(256));
         if (own_c) return go(vf_res_kernel<P, G, MU_ROW, true>, mu_items<MU_ROW>(256));
         if (row) return go(vf_res_kernel<P, G, MU_ROW, false>, mu_items<MU_ROW>(256));
         return go(vf_res_kernel<P, G, MU_PAIR, false>, mu_items<MU_PAIR>(256));
@@ -513,9 +565,13 @@ static int launch_vf_res(const VerifyArgs &a, bool row, bool own_c, hipStream_t 
 template <class P>
 static int launch_vf_main(const VerifyArgs &a, bool row, bool own_c, hipStream_t st) {
     constexpr int IPW = FoldCfg<P>::IPW;
-    const uint32_t per = row ? mu_items<MU_ROW>(64) : mu_items<MU_PAIR>(64), mu = (uint32_t)((a.n + per - 1) / per);
+    const bool wave = wave_hashes(a);
+    const uint32_t per = wave ? mu_items<MU_WAVE>(64) : row ? mu_items<MU_ROW>(64) : mu_items<MU_PAIR>(64);
+    const uint32_t mu = (uint32_t)((a.n + per - 1) / per);
     const dim3 grid(mu + (unsigned)((a.n + IPW - 1) / IPW));
-    if (own_c)
+    if (wave)
+        hipLaunchKernelGGL((vf_main_kernel<P, MU_WAVE, true>), grid, dim3(64), 0, st, a, mu);
+    else if (own_c)
         hipLaunchKernelGGL((vf_main_kernel<P, MU_ROW, true>), grid, dim3(64), 0, st, a, mu);
     else if (row)
         hipLaunchKernelGGL((vf_main_kernel<P, MU_ROW, false>), grid, dim3(64), 0, st, a, mu);
@@ -560,7 +616,9 @@ static int verify_impl(const VerifyArgs &a, hipStream_t st, hipEvent_t *ev) {
     if (e) return e;
     if (ev && (e = (int)hipEventRecord(ev[2], st))) return e;
     auto blocks = [&](size_t per) { return dim3((unsigned)((a.n * per + 255) / 256)); };
-    if (small)
+    if (wave_hashes(a))
+        hipLaunchKernelGGL((vf_final_kernel<P, FINAL_WAVE>), blocks(64), dim3(256), 0, st, a);
+    else if (small)
         hipLaunchKernelGGL((vf_final_kernel<P, FINAL_ROW>), blocks(16), dim3(256), 0, st, a);
     else if (a.n <= VERIFY_PAIR_MAX)
         hipLaunchKernelGGL((vf_final_kernel<P, FINAL_PAIR>), blocks(2), dim3(256), 0, st, a);
