@@ -296,4 +296,37 @@ __device__ __forceinline__ void stage_c_wave(const uint32_t *mu, const uint32_t 
     challenge_wave<P::TAU>(lo, hi, masks, r, lds, my);
 }
 
+// LDS words of expand_a_wave's block: 42 and one that the last candidates'
+// second word reads
+constexpr int EXPAND_WAVE_WORDS = 2 * (SHAKE128_RATE / 8) + 2;
+
+// One polynomial of ExpandA by a wave: a[N] from rho (32 bytes) and
+// nonce = k << 8 | l.  The 56 candidates of a block are tested at once, one
+// per lane; an accepted one's place is the number accepted before it.
+__device__ __forceinline__ void expand_a_wave(int32_t *a, const uint8_t *rho, uint32_t nonce, const WaveLane &r,
+                                              uint32_t *lds, uint32_t *block) {
+    constexpr uint32_t CAND = SHAKE128_RATE / 3;
+    const uint32_t lane = (uint32_t)lane_id(), byte = 3 * lane;
+    const uint64_t seed = r.w < 4 ? load_any<uint64_t>(rho + 8 * r.w) : 0ull;
+    uint32_t lo = (uint32_t)seed, hi = (uint32_t)(seed >> 32);
+    if (r.w == 4) lo = (nonce & 0xFFFFu) | (0x1Fu << 16);
+    if (r.w == SHAKE128_RATE / 8 - 1) hi = 0x80000000u;
+    for (uint32_t n = 0; n < N;) {
+        keccak_f1600_wave(lo, hi, r, lds);
+        wave_store_words(lo, hi, r, block, SHAKE128_RATE / 8);
+        wave_lds_sync();
+        uint32_t t = Q;
+        if (lane < CAND) {
+            const uint32_t *q = block + (byte >> 2);
+            t = __builtin_amdgcn_alignbyte(q[1], q[0], byte & 3) & 0x7FFFFFu;
+        }
+        const bool ok = t < (uint32_t)Q;
+        const uint64_t mask = __ballot(ok);
+        const uint32_t at = n + __popcll(mask & ((1ull << lane) - 1ull));
+        if (ok && at < N) a[at] = (int32_t)t;
+        n += __popcll(mask);
+        wave_lds_sync();  // the block is read before the next one overwrites it
+    }
+}
+
 }  // namespace dil

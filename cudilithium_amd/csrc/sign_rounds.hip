@@ -94,7 +94,13 @@ __host__ __device__ inline void plan_round(uint32_t u, uint32_t nslots, uint32_t
 
 struct FixedGrid {
     uint32_t mu, expand, prep;  // workgroups of each role
+    uint32_t expand_wave;       // ExpandA with a wave per entry instead of a lane
 };
+// Up to this many entries of A (with waves for the message hashes too): the
+// chain of a lane's five permutations is 48 us, a wave's 12.  Whole calls with
+// 32-byte messages: 1 Dilithium2 item 92 us (lanes 140), 500 Dilithium2 292
+// (307), 270 Dilithium3 265 (282), 146 Dilithium5 238 (256).
+constexpr size_t EXPAND_WAVE_MAX = 8192;
 
 // lanes per message hash
 enum { MU_PAIR = 2, MU_ROW = 16, MU_WAVE = 64 };
@@ -132,6 +138,18 @@ __global__ __launch_bounds__(256) void sg_fixed_kernel(SignArgs a, Chain ch, Fix
     }
     b -= g.mu;
     if (b < g.expand) {
+        if constexpr (LANES == MU_WAVE) {
+            if (g.expand_wave) {
+                __shared__ __align__(8) uint32_t block[4][EXPAND_WAVE_WORDS];
+                const uint32_t w = threadIdx.x >> 6, t = b * 4 + w, i = t / KL, e = t % KL;
+                if (i >= ch.n) return;  // whole waves
+                const size_t item = ch.first + i;
+                expand_a_wave(reinterpret_cast<int32_t *>(a.rows + item * a.row_pitch + a.off_ints) + e * N,
+                              a.sk + item * a.sk_pitch, e / P::L << 8 | e % P::L,
+                              wave_lane_setup(lds, w * WAVE_LDS_WORDS), lds, block[w]);
+                return;
+            }
+        }
         const size_t t = (size_t)b * 256 + threadIdx.x;
         if (t >= (size_t)ch.n * KL) return;
         const int e = (int)(t % KL);
@@ -364,7 +382,9 @@ int launch_fixed(const SignArgs &a, const Chain &ch, hipStream_t st) {
     const uint32_t per = 256 / lanes;
     FixedGrid g;
     g.mu = (ch.n + per - 1) / per;
-    g.expand = a.key_idx ? 0 : (uint32_t)(((size_t)ch.n * KL + 255) / 256);  // resident keys are expanded
+    const size_t entries = a.key_idx ? 0 : (size_t)ch.n * KL;  // resident keys are expanded
+    g.expand_wave = lanes == MU_WAVE && entries <= EXPAND_WAVE_MAX;
+    g.expand = (uint32_t)(g.expand_wave ? (entries + 3) / 4 : (entries + 255) / 256);
     g.prep = a.key_idx ? 0 : (uint32_t)(((size_t)ch.n * PREP + 255) / 256);
     const dim3 grid(g.mu + g.expand + g.prep);
     if (lanes == MU_WAVE)

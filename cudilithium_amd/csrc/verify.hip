@@ -11,7 +11,8 @@
 //                   + norm check + NTT, A z^ straight from the sponges
 //                   (fold.hpp), then per row - c^ t1^ 2^d, INTT, caddq,
 //                   UseHint, pack w1'.  With resident keys: one workgroup per
-//                   G items, A z^ from the stored A
+//                   G items, A z^ from the stored A.  The smallest batches:
+//                   a workgroup per item and row of A (vf_small)
 //   vf_final  c~' = H(mu || w1'), compare, write the verdict
 // ret is 0 for a valid signature and -1 otherwise (api.cu:454-515).
 #include <hip/hip_runtime.h>
@@ -37,6 +38,11 @@ constexpr size_t VERIFY_ROW_MAX = 4096;
 // 205 / 151; resident, messages up to 4 KiB, 1,000 Dilithium3 52 / 72, 2,500
 // Dilithium3 122 / 175, 4,000 Dilithium2 187 / 172).
 constexpr size_t VERIFY_WAVE_MAX = 1024, VERIFY_WAVE_MAX_RESIDENT = 3072;
+// Without resident keys, vf_small takes calls of up to this many entries of A
+// (vf_small / vf_main, 32-byte messages: 16 Dilithium2 items 52 / 130 us, 512
+// Dilithium2 87 / 132, 270 Dilithium3 98 / 121, 140 Dilithium5 95 / 120; 540
+// Dilithium3 147 / 124, 290 Dilithium5 150 / 122).
+constexpr size_t VERIFY_SMALL_WAVES = 8192;
 static bool wave_hashes(const VerifyArgs &a) {
     return a.n <= (a.key_idx ? VERIFY_WAVE_MAX_RESIDENT : VERIFY_WAVE_MAX);
 }
@@ -351,6 +357,85 @@ __global__ __launch_bounds__(64) void vf_main_kernel(VerifyArgs a, uint32_t mu_b
     }
 }
 
+// The smallest batches: a workgroup per item and row of A, a wave per entry.
+// What ends such a call is the chain of one workgroup, in vf_main's form five
+// lane permutations (9.6 us each) and the transforms of IPW items one after
+// the other; here five wave permutations (2.3 us) and two transforms.  Every
+// workgroup of an item checks and transforms z for itself.
+template <class P>
+struct VfSmallShared {
+    ZetaLds zt;
+    int32_t a[P::L][N], c[N], t1[N];
+    int32_t x[P::L][NTT_XBUF];
+    uint32_t wave[P::L][WAVE_LDS_WORDS + 2];
+    uint32_t block[P::L][EXPAND_WAVE_WORDS];
+    uint32_t chal[CHALLENGE_ROW_WORDS], cp[16], bits[P::K * 8];
+    int fail;
+};
+
+template <class P>
+__global__ __launch_bounds__(64 * P::L) void vf_small_kernel(VerifyArgs a, uint32_t mu_blocks) {
+    using Z = Sizes<P>;
+    using VL = VerifyLayout<P>;
+    __shared__ __align__(16) VfSmallShared<P> sh;
+    if (blockIdx.x < mu_blocks) {
+        static_assert(sizeof(sh.a) >= 4 * P::L * WAVE_LDS_WORDS, "the mu role's waves");
+        return mu_role<P, MU_WAVE>(a, blockIdx.x, reinterpret_cast<uint32_t *>(sh.a));
+    }
+    const uint32_t wave = threadIdx.x >> 6, b = blockIdx.x - mu_blocks, k = b % P::K;
+    const size_t item = b / P::K;
+    const uint8_t *sig = a.sig + item * a.sig_pitch, *pk = a.pk + item * a.pk_pitch;
+    uint8_t *work = a.work + item * a.work_pitch;
+    zeta_lds_load(sh.zt);
+    if (threadIdx.x == 0) sh.fail = 0;
+    __syncthreads();
+
+    int32_t z[4];
+    bool good = load_z_ntt<P>(z, sig, (int)wave, sh.x[wave], sh.zt);
+    if (wave == 1) {
+        good &= decode_hints<P>(sig + Z::SIG_H, sh.bits);
+        uint32_t f[4];
+        int32_t t1[4];
+        wave_fields_A<10>(f, pk + SEEDBYTES + k * POLYT1_BYTES);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t1[r] = (int32_t)(f[r] << D);
+        ntt_wave(t1, sh.x[wave], sh.zt);
+        wave_store_D(sh.t1, t1);
+    }
+    if (!good && lane_id() == 0) sh.fail = 1;
+    const WaveLane r = wave_lane_setup(sh.wave[wave], 0);
+    if (wave == 0) {
+        const uint64_t ct = r.w < 4 ? load_any<uint64_t>(sig + 8 * r.w) : 0ull;
+        const uint32_t lo = r.w == 4 ? 0x1Fu : (uint32_t)ct;
+        const uint32_t hi = r.w == SHAKE256_RATE / 8 - 1 ? 0x80000000u : (uint32_t)(ct >> 32);
+        challenge_wave<P::TAU>(lo, hi, sh.cp, r, sh.wave[wave], sh.chal);
+        wave_lds_sync();
+        int32_t c[4];
+        wave_load_challenge_A(c, sh.cp);
+        ntt_wave(c, sh.x[wave], sh.zt);
+        wave_store_D(sh.c, c);
+    }
+    expand_a_wave(sh.a[wave], pk, k << 8 | wave, r, sh.wave[wave], sh.block[wave]);
+    int32_t av[4];
+    wave_load_D(av, sh.a[wave]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) av[q] = mont_mul(av[q], z[q]);
+    wave_store_D(sh.a[wave], av);
+    __syncthreads();
+    if (k == 0 && threadIdx.x == 0) *reinterpret_cast<int32_t *>(work + VL::FLAG) = sh.fail;
+    if (wave != 0 || sh.fail) return;
+    int32_t w[4] = {0, 0, 0, 0}, c[4], t1[4];
+#pragma unroll
+    for (int l = 0; l < P::L; ++l) {
+        wave_load_D(av, sh.a[l]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] += av[q];
+    }
+    wave_load_D(c, sh.c);
+    wave_load_D(t1, sh.t1);
+    finish_row<P>(work, (int)k, w, c, t1, sh.bits, sh.x[0], sh.zt);
+}
+
 template <class P>
 struct VfMainCfg {
     static constexpr int G = P::MODE == 2 ? 16 : (P::MODE == 3 ? 8 : 4);
@@ -565,6 +650,11 @@ static int launch_vf_res(const VerifyArgs &a, bool row, bool own_c, hipStream_t 
 template <class P>
 static int launch_vf_main(const VerifyArgs &a, bool row, bool own_c, hipStream_t st) {
     constexpr int IPW = FoldCfg<P>::IPW;
+    if (a.n * P::K * P::L <= VERIFY_SMALL_WAVES) {
+        const uint32_t mu = (uint32_t)((a.n + P::L - 1) / P::L);
+        hipLaunchKernelGGL(vf_small_kernel<P>, dim3(mu + (unsigned)a.n * P::K), dim3(64 * P::L), 0, st, a, mu);
+        return (int)hipGetLastError();
+    }
     const bool wave = wave_hashes(a);
     const uint32_t per = wave ? mu_items<MU_WAVE>(64) : row ? mu_items<MU_ROW>(64) : mu_items<MU_PAIR>(64);
     const uint32_t mu = (uint32_t)((a.n + per - 1) / per);

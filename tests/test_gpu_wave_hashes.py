@@ -1,4 +1,4 @@
-"""Hashes with one sponge per wavefront: message lengths around the ends of
+"""Hashes and ExpandA with one sponge per wavefront: message lengths around the ends of
 words and SHAKE256 blocks (the sponge also holds 32 bytes of tr), at unaligned
 offsets, and the batch sizes at which signing and verification change between
 one wave and fewer lanes per hash; bytes and verdicts equal the oracle's."""
@@ -64,3 +64,21 @@ def test_batch_size_edges_match_oracle(n):
     idx = np.arange(n, dtype=np.uint32)[::-1].copy()
     assert np.array_equal(ctx.sign_resident(ks, idx, msgs[::-1]), exp[::-1])
     assert np.array_equal(ks.verify(idx, sig[::-1].copy(), msgs[::-1]), ret[::-1])
+
+
+# slow seeds of tests/test_gpu_expand_fold.py have entries of A with many
+# rejected candidates; n K L around the limit of 8,192 entries
+@pytest.mark.parametrize("mode,n", [(2, 5), (2, 512), (2, 513), (3, 273), (3, 274), (5, 146), (5, 147)])
+def test_entry_per_wave_matches_oracle(mode, n):
+    from cudilithium_amd import api
+    rng = np.random.default_rng(n)
+    msgs = _msgs(rng, rng.integers(0, 150, n))
+    pk, sk = oracle.keypair_counter_batch(mode, n, rand_index=15351 - n // 2)
+    exp, att = oracle.sign_batch(mode, msgs, sk)
+    ctx = api.SignContext(mode, n)
+    assert np.array_equal(ctx.sign(msgs, sk), exp)
+    assert np.array_equal(ctx.attempt_counts(n), att)
+    sig, ret = _verdicts(mode, rng, exp, msgs, pk)
+    sig[0] = 0xFF  # z out of range and hint bytes that break the rules
+    ret[0] = -1
+    assert np.array_equal(api.verify_device(mode, sig, msgs, pk), ret)
