@@ -2,12 +2,12 @@
 
 Headline workload (default): Dilithium3 deterministic signing of 16384
 (key, message) pairs, message lengths log-uniform in [32 B, 4 KiB], keys from
-seeds, inputs resident in HBM, one fixed-stage pass plus one persistent
-rejection-loop launch per step.  A step signs the whole batch.
+seeds, inputs resident in HBM, the fixed stage and the rejection rounds'
+launches per step.  A step signs the whole batch.
 
-Printed on one JSON line: throughput (signatures/s, the persistent engine
-replayed as a HIP graph), the roofline of the dominant kernel (the persistent
-rejection loop, integer-VALU bound), the oracle's CPU rate on a bounded
+Printed on one JSON line: throughput (signatures/s, the default engine
+replayed as a HIP graph), the roofline of its dominant part (the kernels of
+the rejection rounds, integer-VALU bound), the oracle's CPU rate on a bounded
 sample, the per-stage (reference architecture) GPU form on the same inputs,
 a serving summary (resident keys, continuous batching: p50 / p99 latency
 at two offered loads) and the drop-in call's rate with host buffers.
@@ -37,14 +37,14 @@ PEAK_HBM_GBS = 8000.0
 # WRITE_SIZE passes scaled by a 1 GiB copy's readings (read = 2 x FETCH_SIZE,
 # written = WRITE_SIZE); profiles/sign3_16384_hbm_valu_counters.md.
 TRAFFIC_BYTES = {
-    # loop kernel per launch: 2 x FETCH_SIZE + WRITE_SIZE KiB (profiles/sign3_16384_hbm_valu_counters.md)
-    "dilithium3_sign_16384_msg_loguniform_32B-4KiB": (2 * 1641558 + 1548709) * 1024,
-    # vf_mu_pair + vf_prep + vf_main + vf_final per call (profiles/verify5_65536_kernel_stats.md)
+    # the rounds' kernels per call: 2 x FETCH_SIZE + WRITE_SIZE KiB
+    "dilithium3_sign_16384_msg_loguniform_32B-4KiB": (2 * 1691989 + 1260871) * 1024,
+    # vf_prep + vf_main + vf_final per call
     "dilithium5_verify_65536_msg_1KiB_10pct_bitflips":
-        (2 * (119517 + 51717 + 247489 + 46140) + (4096 + 75070 + 65462 + 256)) * 1024,
+        (2 * (5290 + 360000 + 46100) + (4100 + 71600 + 256)) * 1024,
     "ntt_pipeline_65536x256": (2 * 65576 + 65536) * 1024,
     # vf_main alone
-    "dilithium5_verify_65536_msg_1KiB_10pct_bitflips_vf_main": (2 * 247489 + 65462) * 1024,
+    "dilithium5_verify_65536_msg_1KiB_10pct_bitflips_vf_main": (2 * 360000 + 71600) * 1024,
 }
 
 
@@ -95,12 +95,12 @@ def bench_sign(args, mode: int):
     tim = ctx.timings()
     ctx.enable_timing(0)
     sig_eager = d_sig.download((n, sigb), np.uint8)
-    log(f"[bench] persistent: {args.steps} steps in {wall * 1e3:.2f} ms; loop kernel "
+    log(f"[bench] {args.steps} steps in {wall * 1e3:.2f} ms; rejection rounds "
         f"{np.mean([t[1] for t in tim]):.3f} ms, fixed stage {np.mean([t[0] for t in tim]):.3f} ms")
     eager_value = n * args.steps / wall
 
-    # the same call captured as a HIP graph (fixed stage's three branches +
-    # the persistent loop), replayed once per step: the headline figure
+    # the same call captured as a HIP graph (fixed stage and
+    # rounds), replayed once per step: the headline figure
     graph = ctx.graph(d_sig, d_sk, d_msgs)
     d_sig.memset(0)
     for _ in range(max(1, args.warmup)):
@@ -137,7 +137,8 @@ def bench_sign(args, mode: int):
     log(f"[bench] parity vs oracle on {len(idx)} items: {parity}")
 
     # roofline of the rejection loop: algorithmic int32 ops of the attempts the
-    # specification makes, over the loop kernel's event-timed duration
+    # specification makes, over the event-timed duration of the rounds (with two
+    # chains, from the end of the first one's fixed stage on)
     loop_ms = float(np.mean([t[1] for t in tim]))
     ops = float(attempts.sum()) * workmodel.sign_attempt_ops(mode)
     achieved = ops / (loop_ms * 1e-3) / 1e12
@@ -181,7 +182,7 @@ def bench_sign(args, mode: int):
         "dtype": "int32", "config": cfg, "parity": "bit-exact" if parity else "MISMATCH",
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_INT32_TOPS, "unit": "TOP/s",
                      "frac": achieved / PEAK_INT32_TOPS, "traffic": TRAFFIC_BYTES.get(cfg["workload"]),
-                     "kernel": "sg_persistent_kernel", "kernel_ms": loop_ms,
+                     "kernel": "sg_ry / sg_rw / sg_rc / sg_rz / sg_rs / sg_plan", "kernel_ms": loop_ms,
                      "algorithmic_ops": ops},
         "cpu_baseline": cpu, "perstage_gpu_baseline": perstage, "eager_persistent_value": eager_value,
         "speedup_vs_perstage": (value / perstage["value"]) if perstage else None,

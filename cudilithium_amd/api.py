@@ -24,7 +24,7 @@ ENGINE_PERSISTENT, ENGINE_PERSTAGE = 0, 1
 STATUS_ROUND_CAP, STATUS_NO_SECRET = 1, 2
 # message hashing flag of dil_sign_ctx_set_message_hashing / dil_verify_device*_ex
 HASH_LONG_MESSAGES = 1
-# flag of dil_sign_ctx_set_claim: guided claims near the end of the queue
+# flag of dil_sign_ctx_set_claim: accepted, without effect
 CLAIM_GUIDED = 0x10000
 
 

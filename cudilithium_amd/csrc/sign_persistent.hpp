@@ -6,7 +6,7 @@
 //
 //   refill   claim items from a global queue (one atomicAdd per refill) until
 //            the workgroup owns `claim` (at most S) undone items or the queue
-//            is empty; with guided claims fewer near the end of the queue
+//            is empty
 //   assign   S attempt slots round-robin over the owned items: item o gets
 //            slots o, o + U, o + 2U, ... with consecutive nonces, so freed
 //            slots turn into speculative nonces of unfinished items instead of

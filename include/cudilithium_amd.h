@@ -256,9 +256,10 @@ int dil_verify_device_timed(int mode, int32_t *d_ret, const uint8_t *d_sig, size
  * (cudilithium_amd/autotune.py) records them: per kind, mode and batch
  * bucket (0: up to 1,024 items, 1: 4,096, 2: 16,384, 3: more; -1 = all
  * buckets) a value, 0 restoring the compiled default.  Kinds: keys per
- * workgroup of keygen's main kernel and items per workgroup of verify's
- * (2, 4, 8 or 16 where its LDS fits: defaults 16 / 8 / 4 for modes 2 / 3 / 5),
- * wavefronts per workgroup of the standalone NTT (2, 4 or 8; default 4; mode
+ * workgroup of keygen's main kernel (checked and kept, but without effect: a
+ * wave takes a fixed number of keys) and items per workgroup of verify's with
+ * resident keys (2, 4, 8 or 16 where its LDS fits: defaults 16 / 8 / 4 for
+ * modes 2 / 3 / 5), wavefronts per workgroup of the standalone NTT (2, 4 or 8; default 4; mode
  * ignored).  Process-wide; results never depend on them.  DIL_EINVAL for a
  * value the kernels are not built for. */
 #define DIL_TILE_KEYGEN_ITEMS 0
@@ -273,7 +274,10 @@ int dil_get_kernel_tiling(int kind, int mode, size_t n);
 typedef struct dil_sign_ctx dil_sign_ctx;
 int dil_sign_ctx_create(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t nslots);
 int dil_sign_ctx_destroy(dil_sign_ctx *ctx);
-/* Persistent engine tiling: slots per workgroup (0 = automatic, or 1, 8, 16,
+/* Signing runs in device-driven rounds that choose their own launch shapes;
+ * the two tilings below concern the persistent kernel, which runs alone for
+ * calls with fewer slots than half their items and for the phase profile.
+ * Tiling: slots per workgroup (0 = automatic, or 1, 8, 16,
  * 32), register budget as waves per SIMD (0 = automatic, or 2, 3, 4) and
  * workgroup count (0 = nslots / slots_per_block). */
 int dil_sign_ctx_set_tiling(dil_sign_ctx *ctx, int slots_per_block, int occupancy, int blocks);
@@ -281,10 +285,8 @@ int dil_sign_ctx_set_tiling(dil_sign_ctx *ctx, int slots_per_block, int occupanc
  * time (0 = slots per workgroup).  Below that, each owned item gets several
  * slots (consecutive nonces) per round, so small batches finish in fewer
  * rounds at the price of speculative attempts; results are unchanged.
- * OR DIL_CLAIM_GUIDED into items_per_block for guided claims: once the queue
- * holds fewer than items_per_block items per resident workgroup, a workgroup
- * owns at most (remaining items / resident workgroups), so the batch's last
- * items spread over all workgroups (more speculation, shorter tail). */
+ * DIL_CLAIM_GUIDED may be ORed into items_per_block; it has no effect since
+ * the rounds took over the batches whose last items it spread. */
 #define DIL_CLAIM_GUIDED 0x10000
 int dil_sign_ctx_set_claim(dil_sign_ctx *ctx, int items_per_block);
 /* Records HIP events on the call's stream around the fixed stage and the
@@ -330,7 +332,7 @@ int dil_sign_ctx_phase_cycles(dil_sign_ctx *ctx, uint64_t *cycles6, void *stream
  * verify.cu:146-200, and re-unpacks and transforms s1, s2, t0 on every
  * signature, sign.cu:306-403).  A key store holds `capacity` keys of one
  * mode: pk, sk (absent for verify-only keys), tr = H(pk) and the expanded
- * A, s1^, s2^, t0^, t1^ (dil_keystore_row_bytes(mode) each, about 38/60/95
+ * A and t1^ and the int8 limbs of s1, s2, t0 (dil_keystore_row_bytes(mode) each, about 38/60/95
  * KiB for modes 2/3/5).  Results equal the non-resident entry points'. */
 typedef struct dil_keystore dil_keystore;
 size_t dil_keystore_row_bytes(int mode);
@@ -343,7 +345,7 @@ int dil_keystore_mode(const dil_keystore *ks);
 int dil_keystore_has_secret(const dil_keystore *ks, size_t idx);
 /* Installs n keys at [first, first + n) from pk (and sk, or NULL for
  * verify-only keys), host or device memory, and expands them on `stream`.
- * A verify-only load clears the rows' secret-key bytes and s1^, s2^, t0^. */
+ * A verify-only load clears the rows' secret-key bytes and s1, s2, t0. */
 int dil_keystore_load(dil_keystore *ks, size_t first, const uint8_t *pk, size_t pk_pitch,
                       const uint8_t *sk, size_t sk_pitch, size_t n, void *stream);
 /* Generates n keys into [first, first + n) as dil_keypair_device would
