@@ -8,7 +8,8 @@
 //   kg_main   one wave per FoldCfg<P>::IPW keys: NTT(s1), A s1^ straight from
 //             the sponges (fold.hpp), then per row INTT, + s2, caddq,
 //             Power2Round and packing of t1 / t0
-//   kg_tr     tr = SHAKE256(pk)[0:32], a 16-lane row or a lane pair per key
+//   kg_tr     tr = SHAKE256(pk)[0:32], a wave, a 16-lane row or a lane pair
+//             per key
 #include <hip/hip_runtime.h>
 
 #include "fold.hpp"
@@ -210,6 +211,21 @@ __global__ __launch_bounds__(256) void kg_tr_row_kernel(KeygenArgs a) {
         for (int x = 0; x < 4; ++x) store_any<uint32_t>(tr + 8 * x + 4 * r.h, s[x]);
 }
 
+// ... and with a wave per key for the smallest batches
+template <class P>
+__global__ __launch_bounds__(256) void kg_tr_wave_kernel(KeygenArgs a) {
+    using Z = Sizes<P>;
+    __shared__ __align__(8) uint32_t lds[4 * WAVE_LDS_WORDS];
+    const WaveLane r = wave_lane_setup(lds, (threadIdx.x >> 6) * WAVE_LDS_WORDS);
+    const size_t i = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= a.n) return;  // whole waves
+    const uint8_t *pk = a.pk + i * a.pk_pitch;
+    uint32_t lo, hi;
+    shake_wave<SHAKE256_RATE>(lo, hi, r, lds, (uint32_t)Z::PK_BYTES,
+                              [&](uint32_t w) { return load_word_bytes(pk, 8 * w, Z::PK_BYTES); });
+    if (r.main && r.w < 4) store_any<uint64_t>(a.sk + i * a.sk_pitch + Z::SK_TR + 8 * r.w, lo | (uint64_t)hi << 32);
+}
+
 // tr = SHAKE256(pk)[0:32] with two lanes per key (keccak_f1600_pair): the
 // serial absorb of the public key (10 / 15 / 20 permutations) is 2/3 as long
 template <class P>
@@ -234,8 +250,12 @@ constexpr bool kg_fits() {
     return G * (P::L + P::K) * N * 4 + 8 * 1024 <= 160 * 1024;
 }
 
-// 4,096 rows are one wave per SIMD
-constexpr size_t KEYGEN_ROW_MAX = 4096;
+// tr with a wave per key, with a row per key, beyond that with lane pairs.
+// Whole calls, row / wave: 10 Dilithium5 keys 206 / 173 us, 1,000 Dilithium3
+// 199 / 175, 3,000 Dilithium3 236 / 229, 4,000 Dilithium5 393 / 396; pair /
+// row: 6,000 Dilithium3 402 / 372, 8,000 Dilithium5 651 / 613, 10,000
+// Dilithium2 366 / 370.
+constexpr size_t KEYGEN_WAVE_MAX = 3072, KEYGEN_ROW_MAX = 8192;
 
 template <class P>
 static int keygen_impl(const KeygenArgs &a, hipStream_t st) {
@@ -246,7 +266,9 @@ static int keygen_impl(const KeygenArgs &a, hipStream_t st) {
     hipLaunchKernelGGL(kg_eta_kernel<P>, dim3((unsigned)((a.n * NP + 63) / 64)), dim3(64), 0, st, a);
     constexpr int IPW = FoldCfg<P>::IPW;
     hipLaunchKernelGGL(kg_main_kernel<P>, dim3((unsigned)((a.n + IPW - 1) / IPW)), dim3(64), 0, st, a);
-    if (a.n <= KEYGEN_ROW_MAX)
+    if (a.n <= KEYGEN_WAVE_MAX)
+        hipLaunchKernelGGL(kg_tr_wave_kernel<P>, dim3((unsigned)((a.n + 3) / 4)), dim3(256), 0, st, a);
+    else if (a.n <= KEYGEN_ROW_MAX)
         hipLaunchKernelGGL(kg_tr_row_kernel<P>, dim3((unsigned)((a.n + ROW_ITEMS_PER_BLOCK - 1) / ROW_ITEMS_PER_BLOCK)),
                            dim3(256), 0, st, a);
     else

@@ -82,3 +82,11 @@ def test_entry_per_wave_matches_oracle(mode, n):
     sig[0] = 0xFF  # z out of range and hint bytes that break the rules
     ret[0] = -1
     assert np.array_equal(api.verify_device(mode, sig, msgs, pk), ret)
+
+
+@pytest.mark.parametrize("mode,n", [(5, 1), (2, 3072), (3, 3073), (2, 8192), (2, 8193)])
+def test_keys_match_oracle(mode, n):
+    from cudilithium_amd import api
+    pk, sk = api.keypair_device(mode, n=n, rand_index=n)
+    epk, esk = oracle.keypair_counter_batch(mode, n, rand_index=n)
+    assert np.array_equal(pk, epk) and np.array_equal(sk, esk)
