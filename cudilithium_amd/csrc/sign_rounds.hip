@@ -51,9 +51,11 @@ constexpr int ROUND_WAVES = 4;
 constexpr uint32_t ROUND_MAX_M = 32;  // attempts per item and round
 // Messages hashed with a 16-lane row each up to this batch: beyond, the rows'
 // fourfold instruction count costs ExpandA beside them more than the shorter
-// chain gives (3,001 Dilithium5 items with messages up to 4 KiB: fixed stage
-// 394 us with lane pairs, 174 us with rows).
-constexpr uint32_t FIXED_ROW_MAX = 4096;
+// chain gives.  Whole calls, messages up to 4 KiB, rows / lane pairs: 5,000
+// Dilithium3 items 1.19 / 1.36 ms, 6,000 Dilithium2 1.01 / 1.20, 8,000
+// Dilithium3 1.59 / 1.62 (resident 1.46 / 1.61), 8,000 Dilithium5 1.67 / 1.66,
+// 12,000 Dilithium3 2.11 / 2.06; 32-byte messages 6,000 Dilithium3 1.27 / 1.26.
+constexpr size_t FIXED_ROW_MAX = 8192;
 // With a wave each up to these, the second with resident keys, where nothing
 // runs beside the hashes (messages up to 4 KiB, whole call with waves / rows:
 // 1,000 Dilithium3 items 465 / 517 us, 2,000 Dilithium5 691 / 713, 3,001
@@ -378,7 +380,7 @@ int launch_fixed(const SignArgs &a, const Chain &ch, hipStream_t st) {
     constexpr int KL = P::K * P::L, PREP = (P::L + 2 * P::K) * (N / 8);
     // one sponge per wave or 16-lane row where those of all messages fit the
     // card beside the other roles, or (rows) on request
-    const int lanes = ch.n <= (a.key_idx ? FIXED_WAVE_MAX_RESIDENT : FIXED_WAVE_MAX) ? MU_WAVE : a.row_mu || ch.n <= FIXED_ROW_MAX ? MU_ROW : MU_PAIR;
+    const int lanes = ch.n <= (a.key_idx ? FIXED_WAVE_MAX_RESIDENT : FIXED_WAVE_MAX) ? MU_WAVE : a.row_mu || a.n <= FIXED_ROW_MAX ? MU_ROW : MU_PAIR;
     const uint32_t per = 256 / lanes;
     FixedGrid g;
     g.mu = (ch.n + per - 1) / per;

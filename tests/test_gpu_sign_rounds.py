@@ -31,8 +31,8 @@ def test_signatures_and_attempts_match_oracle(mode, n):
         assert ctx.executed_attempts() >= int(att.sum())
 
 
-@pytest.mark.parametrize("n", [12287, 12288, 12801])
-def test_two_chains_match_oracle(n):
+@pytest.mark.parametrize("n", [8192, 8193, 12287, 12288, 12801])
+def test_large_batches_match_oracle(n):
     from cudilithium_amd.api import SignContext
     msgs, sk = _batch(2, n, n)
     exp, att = oracle.sign_batch(2, msgs, sk)
