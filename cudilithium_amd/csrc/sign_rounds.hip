@@ -380,7 +380,8 @@ int launch_fixed(const SignArgs &a, const Chain &ch, hipStream_t st) {
     constexpr int KL = P::K * P::L, PREP = (P::L + 2 * P::K) * (N / 8);
     // one sponge per wave or 16-lane row where those of all messages fit the
     // card beside the other roles, or (rows) on request
-    const int lanes = ch.n <= (a.key_idx ? FIXED_WAVE_MAX_RESIDENT : FIXED_WAVE_MAX) ? MU_WAVE : a.row_mu || a.n <= FIXED_ROW_MAX ? MU_ROW : MU_PAIR;
+    const bool wave = ch.n <= (a.key_idx ? FIXED_WAVE_MAX_RESIDENT : FIXED_WAVE_MAX);
+    const int lanes = wave ? MU_WAVE : a.row_mu || a.n <= FIXED_ROW_MAX ? MU_ROW : MU_PAIR;
     const uint32_t per = 256 / lanes;
     FixedGrid g;
     g.mu = (ch.n + per - 1) / per;
