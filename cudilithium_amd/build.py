@@ -80,20 +80,22 @@ def build(verbose: bool = True, out: str | None = None, extra_flags=()) -> str:
 
 
 def build_cxx_tests() -> None:
-    """The C++ drop-in test programs (tests/cxx/*.cpp), one binary per mode,
-    linked against the in-tree library: the KAT flow, and randomized signing
-    built with -DDILITHIUM_RANDOMIZED_SIGNING."""
+    """The C++ test programs (tests/cxx/*.cpp), linked against the in-tree
+    library: the drop-in's KAT flow and randomized signing (built with
+    -DDILITHIUM_RANDOMIZED_SIGNING), one binary per mode, and the check of the
+    host side without a GPU, which has its own HIP functions."""
     root = os.path.dirname(HERE)
     out_dir = os.path.join(root, "tests", "cxx", "bin")
-    progs = (("kat_dropin", []), ("rnd_dropin", ["-DDILITHIUM_RANDOMIZED_SIGNING"]))
-    for name, extra in progs:
+    progs = [(name, f"{name}_{mode}", [f"-DDILITHIUM_MODE={mode}", *extra])
+             for name, extra in (("kat_dropin", []), ("rnd_dropin", ["-DDILITHIUM_RANDOMIZED_SIGNING"]))
+             for mode in (2, 3, 5)]
+    progs.append(("host_calls", "host_calls", []))
+    for name, binary, defs in progs:
         src = os.path.join(root, "tests", "cxx", f"{name}.cpp")
-        if not os.path.exists(src):
-            continue
-        os.makedirs(out_dir, exist_ok=True)
-        for mode in (2, 3, 5):
-            out = os.path.join(out_dir, f"{name}_{mode}")
-            cmd = [HIPCC, "-std=c++17", "-O2", f"-DDILITHIUM_MODE={mode}", *extra, "-Wno-unused-value",
+        if os.path.exists(src):
+            os.makedirs(out_dir, exist_ok=True)
+            out = os.path.join(out_dir, binary)
+            cmd = [HIPCC, "-std=c++17", "-O2", *defs, "-Wno-unused-value",
                    "-Wno-unused-result", f"-I{os.path.join(root, 'include')}", src, f"-L{HERE}",
                    "-lcudilithium_amd", "-Wl,-rpath,$ORIGIN/../../../cudilithium_amd", "-o", out]
             r = subprocess.run(cmd, capture_output=True, text=True)

@@ -40,6 +40,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 
 #include "hash_row.hpp"
 #include "internal.hpp"
@@ -439,6 +440,36 @@ int launch_round(const SignArgs &a, const SlotRef &sr, const Chain &ch, double &
     return (int)hipGetLastError();
 }
 
+// A second stream forked from the caller's.  join() makes the caller's stream
+// wait for it; a way out that did not join, an error on the way, joins in the
+// destructor, so that buffers which the caller frees after draining its own
+// stream are not in use and a capture is left without a loose branch.
+struct ForkedStream {
+    AuxStreams *aux = nullptr;
+    hipStream_t st = nullptr;
+    std::unique_lock<std::mutex> guard;
+    bool open = false;
+
+    int fork(hipStream_t caller) {
+        st = caller;
+        if (!(aux = aux_streams(st))) return (int)hipErrorOutOfMemory;
+        guard = std::unique_lock<std::mutex>(aux->lock);
+        int e = (int)hipEventRecord(aux->fork, st);
+        if (!e) e = (int)hipStreamWaitEvent(aux->s[0], aux->fork, 0);
+        open = e == 0;
+        return e;
+    }
+    int join() {
+        if (!open) return 0;
+        open = false;
+        int e = (int)hipEventRecord(aux->join[0], aux->s[0]);
+        if (!e) e = (int)hipStreamWaitEvent(st, aux->join[0], 0);
+        if (e) (void)hipStreamSynchronize(aux->s[0]);
+        return e;
+    }
+    ~ForkedStream() { (void)join(); }
+};
+
 template <class P>
 int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRef &lists, const PersistTiling &tiling,
               uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st, hipEvent_t fixed_done) {
@@ -446,15 +477,8 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
     if (e) return e;
     const bool rounds = !phase_sums && a.n <= ROUNDS_MAX_ITEMS_PER_SLOT * nslots;
     const int nchain = rounds && a.n >= TWO_CHAINS_MIN ? 2 : 1;
-    AuxStreams *aux = nullptr;
-    std::unique_lock<std::mutex> guard;
-    if (nchain == 2) {
-        aux = aux_streams(st);
-        if (!aux) return (int)hipErrorOutOfMemory;
-        guard = std::unique_lock<std::mutex>(aux->lock);
-        if ((e = (int)hipEventRecord(aux->fork, st))) return e;
-        if ((e = (int)hipStreamWaitEvent(aux->s[0], aux->fork, 0))) return e;
-    }
+    ForkedStream second;
+    if (nchain == 2 && (e = second.fork(st))) return e;
     Chain ch[2];
     SlotRef csr[2];
     hipStream_t cs[2];
@@ -471,7 +495,7 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
         ch[k].target = (uint32_t)std::min<size_t>(ns, ROUND_TARGET / nchain);
         csr[k] = sr;
         csr[k].base += slot * sr.pitch;
-        cs[k] = k == 0 ? st : aux->s[0];
+        cs[k] = k == 0 ? st : second.aux->s[0];
         u[k] = (double)n;
         first += n;
         slot += ns;
@@ -494,11 +518,7 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
         if ((e = launch_sign_persistent(P::MODE, a, csr[k], ch[k], ch[k].nslots, ch[k].nslots >= 8 ? 8 : 1, 64, 1, ctl,
                                         nullptr, cs[k])))
             return e;
-    if (nchain == 2) {
-        if ((e = (int)hipEventRecord(aux->join[0], aux->s[0]))) return e;
-        return (int)hipStreamWaitEvent(st, aux->join[0], 0);
-    }
-    return 0;
+    return second.join();
 }
 
 }  // namespace

@@ -1,0 +1,190 @@
+// The host side of signing calls without a GPU: this program defines the HIP
+// runtime functions that the library calls (its own definitions take
+// precedence over libamdhip64's), so that it sees every launch, event and
+// allocation and can make any of them fail.  Device pointers are addresses
+// that nothing reads.
+//   host_calls join      errors while a signing call is being enqueued
+// Prints what is wrong and exits with 1, or exits with 0.
+// Run by tests/test_host_sign_calls.py.
+#include <cstdarg>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "cudilithium_amd.h"
+
+namespace {
+
+typedef void *Handle;
+constexpr int FAIL = 999;  // hipErrorUnknown
+
+enum Kind { LAUNCH, RECORD, WAIT, SYNC };
+struct Op {
+    Kind kind;
+    Handle stream, event;
+    bool ok;
+};
+std::vector<Op> ops;
+long fail_at = -1;  // index of the operation that fails
+int last_error = 0;
+
+uintptr_t next_handle = 0x1000, next_address = uintptr_t(1) << 40;
+Handle make_handle() { return reinterpret_cast<Handle>(next_handle += 0x10); }
+
+int op(Kind kind, Handle stream, Handle event) {
+    const bool ok = (long)ops.size() != fail_at;
+    ops.push_back({kind, stream, event, ok});
+    if (!ok) last_error = FAIL;
+    return ok ? 0 : FAIL;
+}
+
+struct Dim3 {
+    uint32_t x, y, z;
+};
+struct Config {
+    Dim3 grid, block;
+    size_t shared;
+    Handle stream;
+} config;
+
+int wrong(const char *fmt, ...) {
+    va_list ap;
+    va_start(ap, fmt);
+    vprintf(fmt, ap);
+    va_end(ap);
+    printf("\n");
+    return 1;
+}
+
+}  // namespace
+
+extern "C" {
+
+int __hipPushCallConfiguration(Dim3 grid, Dim3 block, size_t shared, Handle stream) {
+    config = {grid, block, shared, stream};
+    return 0;
+}
+int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *shared, Handle *stream) {
+    *grid = config.grid;
+    *block = config.block;
+    *shared = config.shared;
+    *stream = config.stream;
+    return 0;
+}
+int hipLaunchKernel(const void *, Dim3, Dim3, void **, size_t, Handle stream) { return op(LAUNCH, stream, nullptr); }
+int hipGetLastError() {
+    const int e = last_error;
+    last_error = 0;
+    return e;
+}
+int hipEventRecord(Handle event, Handle stream) { return op(RECORD, stream, event); }
+int hipStreamWaitEvent(Handle stream, Handle event, unsigned) { return op(WAIT, stream, event); }
+int hipStreamSynchronize(Handle stream) { return op(SYNC, stream, nullptr); }
+
+int hipMalloc(void **p, size_t bytes) {
+    *p = reinterpret_cast<void *>(next_address);
+    next_address += (bytes + 4095) / 4096 * 4096;
+    return 0;
+}
+int hipFree(void *) { return 0; }
+int hipHostMalloc(void **p, size_t bytes, unsigned) {
+    *p = malloc(bytes);
+    return *p ? 0 : 2;
+}
+int hipHostFree(void *p) {
+    free(p);
+    return 0;
+}
+int hipGetDevice(int *dev) {
+    *dev = 0;
+    return 0;
+}
+int hipDeviceGetAttribute(int *v, int, int) {
+    *v = 256;
+    return 0;
+}
+int hipStreamCreateWithFlags(Handle *s, unsigned) {
+    *s = make_handle();
+    return 0;
+}
+int hipEventCreateWithFlags(Handle *e, unsigned) {
+    *e = make_handle();
+    return 0;
+}
+int hipEventCreate(Handle *e) {
+    *e = make_handle();
+    return 0;
+}
+int hipEventDestroy(Handle) { return 0; }
+
+}  // extern "C"
+
+namespace {
+
+uint8_t *device(size_t bytes) {
+    void *p = nullptr;
+    (void)hipMalloc(&p, bytes);
+    return static_cast<uint8_t *>(p);
+}
+
+// one signing call of n items on `st`
+int sign(dil_sign_ctx *ctx, int mode, size_t n, Handle st) {
+    static uint8_t *buf = device(size_t(1) << 32);
+    return dil_sign_device(ctx, buf, dil_signature_bytes(mode), buf, dil_secret_key_bytes(mode), buf,
+                           reinterpret_cast<uint64_t *>(buf), reinterpret_cast<uint32_t *>(buf), n,
+                           DIL_ENGINE_PERSISTENT, st);
+}
+
+// A call of two chains whose k-th operation fails returns an error, and the
+// caller's stream still waits for whatever the second stream was given: the
+// caller may free the buffers once its own stream has drained.
+int join_after_errors() {
+    int bad = 0;
+    for (const int mode : {2, 3, 5}) {
+        const size_t n = 16384;
+        dil_sign_ctx *ctx = nullptr;
+        if (dil_sign_ctx_create(&ctx, mode, n, n)) return wrong("context");
+        const Handle st = make_handle();
+        ops.clear();
+        fail_at = -1;
+        last_error = 0;
+        if (sign(ctx, mode, n, st)) return wrong("mode %d: the call without a failure", mode);
+        const size_t total = ops.size();
+        size_t forked = 0;
+        for (const Op &o : ops) forked += o.kind == LAUNCH && o.stream != st;
+        if (!forked) return wrong("mode %d: nothing runs on a second stream", mode);
+        for (size_t k = 0; k < total; ++k) {
+            ops.clear();
+            fail_at = (long)k;
+            last_error = 0;
+            if (!sign(ctx, mode, n, st)) bad |= wrong("mode %d: operation %zu of %zu failed unnoticed", mode, k, total);
+            // last launch on another stream, and what was waited for after it
+            long last = -1;
+            for (size_t i = 0; i < ops.size(); ++i)
+                if (ops[i].kind == LAUNCH && ops[i].stream != st && ops[i].ok) last = (long)i;
+            if (last < 0) continue;
+            bool joined = false;
+            for (size_t i = (size_t)last + 1; i < ops.size(); ++i) {
+                if (ops[i].ok && ops[i].kind == SYNC && ops[i].stream == ops[last].stream) joined = true;
+                if (!ops[i].ok || ops[i].kind != RECORD || ops[i].stream != ops[last].stream) continue;
+                for (size_t j = i + 1; j < ops.size(); ++j)
+                    joined |= ops[j].ok && ops[j].kind == WAIT && ops[j].stream == st && ops[j].event == ops[i].event;
+            }
+            if (!joined)
+                bad |= wrong("mode %d: operation %zu of %zu failed and the second stream was not joined", mode, k, total);
+        }
+        fail_at = -1;
+        dil_sign_ctx_destroy(ctx);
+    }
+    return bad;
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+    const char *what = argc > 1 ? argv[1] : "";
+    if (!strcmp(what, "join")) return join_after_errors();
+    return 2;
+}
