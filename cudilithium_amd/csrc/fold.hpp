@@ -85,6 +85,7 @@ __device__ __forceinline__ void expand_fold(FoldLds<P> &f, const uint64_t (&rho)
     constexpr int KL = P::K * P::L, ROWS = FoldCfg<P>::IPW * P::K;
     const int lane = lane_id();
     const int i = min(lane / KL, FoldCfg<P>::IPW - 1), k = lane % KL / P::L, l = lane % P::L;
+    wave_lds_sync();  // the transforms that used the windows as their exchange buffer are through
     for (int j = lane; j < ROWS * (FOLD_WIN / 4); j += 64)
         reinterpret_cast<int4 *>(f.win)[j] = make_int4(0, 0, 0, 0);
     Lane64 s[25];

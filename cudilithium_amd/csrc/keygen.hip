@@ -144,6 +144,7 @@ __global__ __launch_bounds__(64) void kg_main_kernel(KeygenArgs a) {
         for (int r = 0; r < 4; ++r) v[r] = P::ETA - (int32_t)f[r];
     };
     zeta_lds_load(sh.zt);
+    wave_lds_sync();
 
 #pragma unroll 1
     for (int t = 0; t < count * P::L; ++t) {

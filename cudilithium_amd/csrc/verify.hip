@@ -290,6 +290,7 @@ __global__ __launch_bounds__(64) void vf_main_kernel(VerifyArgs a, uint32_t mu_b
     const size_t item0 = (size_t)(blockIdx.x - mu_blocks) * IPW;
     auto work_of = [&](size_t item) { return a.work + item * a.work_pitch; };
     zeta_lds_load(sh.zt);
+    wave_lds_sync();
     if constexpr (OWN_C) {
         const RowLane r = row_lane_setup(sh.row, 0);
         const int i = lane >> 4;
