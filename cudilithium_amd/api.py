@@ -100,6 +100,7 @@ def _register():
     R("dil_keystore_keygen", c_int, [c_void_p, c_size_t, c_void_p, c_size_t, ctypes.c_uint64, c_size_t, c_void_p])
     R("dil_keystore_export", c_int, [c_void_p, c_size_t, c_size_t, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p])
     R("dil_sign_ctx_create_resident", c_int, [pp, c_int, c_size_t, c_size_t])
+    R("dil_sign_ctx_create_auto", c_int, [pp, c_int, c_size_t, c_size_t, c_int])
     R("dil_sign_device_resident", c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p,
                                           c_void_p, c_size_t, c_int, c_void_p])
     R("dil_verify_device_resident", c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p,
@@ -334,18 +335,25 @@ class SignContext:
     max_batch signatures of one mode."""
 
     def __init__(self, mode: int, max_batch: int, nslots: int | None = None, resident_only: bool = False):
-        """nslots None: the autotuner's choice for this mode and batch bucket
-        (cudilithium_amd/tuning.json), else one slot per item.  resident_only:
+        """nslots: the attempt slots to allocate, exactly.  None: the autotuner's
+        choice for this mode and batch bucket (cudilithium_amd/tuning.json),
+        else one per item, and beyond it what the rounds of this batch size
+        gain from (dil_sign_ctx_create_auto; up to 1.26 GB).  resident_only:
         rows without per-item expanded arrays (sign_resident only)."""
         from . import autotune
         tuned = autotune.lookup(mode, max_batch)
-        if nslots is None:
+        auto = nslots is None
+        if auto:
             nslots = max(1, int(max_batch * (tuned[0] if tuned else 1.0)))
         self.mode, self.max_batch, self.nslots = mode, max_batch, nslots
         self.pk_bytes, self.sk_bytes, self.sig_bytes = sizes(mode)
         p = c_void_p()
-        create = L().dil_sign_ctx_create_resident if resident_only else L().dil_sign_ctx_create
-        _lib.check(create(ctypes.byref(p), mode, max_batch, nslots), "sign_ctx_create")
+        if auto:
+            r = L().dil_sign_ctx_create_auto(ctypes.byref(p), mode, max_batch, nslots, int(resident_only))
+        else:
+            create = L().dil_sign_ctx_create_resident if resident_only else L().dil_sign_ctx_create
+            r = create(ctypes.byref(p), mode, max_batch, nslots)
+        _lib.check(r, "sign_ctx_create")
         self.handle = p.value
         if tuned and nslots // tuned[1] >= 1:
             self.set_tiling(tuned[1], tuned[2])

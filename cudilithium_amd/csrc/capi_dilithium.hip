@@ -599,7 +599,7 @@ int dil_verify_device(int mode, int32_t *d_ret, const uint8_t *d_sig, size_t sig
 struct dil_sign_ctx {
     int mode = 0;
     size_t max_batch = 0, nslots = 0;
-    size_t round_slots = 0;   // slots allocated: nslots, or more for small batches
+    size_t round_slots = 0;   // slots allocated: nslots, or more when the count was left to the library
     uint8_t *rows = nullptr;  // SignLayout rows (messages stay external)
     size_t row_pitch = 0;
     uint8_t *slots = nullptr;  // TempLayout rows = attempt slots
@@ -704,13 +704,19 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
 }
 
 
-// Attempt slots of a context for small batches: enough that each item gets 32
-// consecutive nonces per round (a round's latency is the same for one or for
-// thousands of attempts), at most 8,192 (about 130 MB).
+// Attempt slots that the rounds gain from, for a context that leaves the count
+// to the library: two per item (ROUND_MIN_M consecutive nonces for each in the
+// first round; 16,384 Dilithium3 items 2.49 ms, 2.69 with one slot per item,
+// 40,000 4.92 and 5.03) up to 65,536, where one fills the card as well (65,536
+// Dilithium3 items 7.6 ms with either), and for small batches up to 32 per item
+// and 8,192 (a round's latency is the same for one or for thousands of
+// attempts; 1,000 Dilithium2 items 0.37 ms, 0.66 with one slot per item).
+// 10 / 14 / 19 KiB a slot: at most 0.7 / 0.94 / 1.26 GB.
 static size_t round_slots_for(size_t max_batch, size_t nslots) {
-    return std::max({nslots, 2 * max_batch, std::min<size_t>(32 * max_batch, 8192)});
+    return std::max({nslots, std::min<size_t>(2 * max_batch, 65536), std::min<size_t>(32 * max_batch, 8192)});
 }
 
+// round_slots >= nslots: allocated if that much memory is free, else nslots
 static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots, size_t round_slots,
                       bool resident_only) {
     if (!out || !valid_mode(mode) || max_batch == 0 || nslots == 0) return DIL_EINVAL;
@@ -729,7 +735,6 @@ static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nsl
         if (r != hipSuccess && e == hipSuccess) e = r;
     };
     chk(hipMalloc((void **)&c->rows, c->row_pitch * max_batch));
-    chk(hipMalloc((void **)&c->slots, c->slot_pitch * round_slots));
     chk(hipMalloc((void **)&c->d_head, 256));
     chk(hipMalloc((void **)&c->d_exec, 4 * nslots));
     chk(hipMalloc((void **)&c->d_done, nslots));
@@ -739,6 +744,14 @@ static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nsl
     chk(hipHostMalloc((void **)&c->h_exec, 4 * nslots, hipHostMallocDefault));
     chk(hipHostMalloc((void **)&c->h_done, nslots, hipHostMallocDefault));
     chk(hipHostMalloc((void **)&c->h_copy, 16 * nslots, hipHostMallocDefault));
+    // last, since it may do with less
+    if (e == hipSuccess && round_slots > nslots &&
+        hipMalloc((void **)&c->slots, c->slot_pitch * round_slots) != hipSuccess) {
+        (void)hipGetLastError();
+        c->slots = nullptr;
+        c->round_slots = nslots;
+    }
+    if (!c->slots) chk(hipMalloc((void **)&c->slots, c->slot_pitch * nslots));
     c->sign_lut.resize(max_batch);
     if (e != hipSuccess) {
         dil_sign_ctx_destroy(c);
@@ -746,10 +759,6 @@ static int ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nsl
     }
     *out = c;
     return 0;
-}
-
-int sign_ctx_create_resident_exact(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots) {
-    return ctx_create(out, mode, max_batch, nslots, nslots, true);
 }
 
 extern "C" {
@@ -772,11 +781,15 @@ int dil_sign_ctx_destroy(dil_sign_ctx *c) {
 }
 
 int dil_sign_ctx_create(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots) {
-    return ctx_create(out, mode, max_batch, nslots, round_slots_for(max_batch, nslots), false);
+    return ctx_create(out, mode, max_batch, nslots, nslots, false);
 }
 
 int dil_sign_ctx_create_resident(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots) {
-    return ctx_create(out, mode, max_batch, nslots, round_slots_for(max_batch, nslots), true);
+    return ctx_create(out, mode, max_batch, nslots, nslots, true);
+}
+
+int dil_sign_ctx_create_auto(dil_sign_ctx **out, int mode, size_t max_batch, size_t nslots, int resident_only) {
+    return ctx_create(out, mode, max_batch, nslots, round_slots_for(max_batch, nslots), resident_only != 0);
 }
 
 int dil_sign_ctx_set_tiling(dil_sign_ctx *c, int slots_per_block, int occupancy, int blocks) {

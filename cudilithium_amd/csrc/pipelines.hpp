@@ -123,8 +123,3 @@ int launch_sign_persistent(int mode, const SignArgs &a, const SlotRef &sr, const
 int default_slots_per_block(size_t nslots);
 
 }  // namespace dil
-
-// dil_sign_ctx_create_resident with exactly nslots attempt slots, for callers
-// that budget the context's memory (the server)
-struct dil_sign_ctx;
-int sign_ctx_create_resident_exact(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t nslots);

@@ -52,7 +52,6 @@
 #include "../../include/cudilithium_amd.h"
 #include "internal.hpp"
 #include "layout.hpp"
-#include "pipelines.hpp"
 #include "params.hpp"
 
 using namespace dil;
@@ -406,7 +405,7 @@ int dil_server_create(dil_server **out, const dil_server_config *cfg) {
         chk((int)hipMalloc((void **)&ln.d_out, out_bytes));
         if (ln.work_pitch) chk((int)hipMalloc((void **)&ln.d_work, b * ln.work_pitch));
         if (ln.op == DIL_OP_SIGN) {
-            chk(sign_ctx_create_resident_exact(&ln.ctx, ln.mode, b, b));
+            chk(dil_sign_ctx_create_resident(&ln.ctx, ln.mode, b, b));
             // long-message lanes hash each message with a 16-lane row
             if (ln.ctx && ln.cls) chk(dil_sign_ctx_set_message_hashing(ln.ctx, DIL_HASH_LONG_MESSAGES));
         }

@@ -40,7 +40,7 @@ namespace dil {
 #define DIL_PERSIST_THREADS 256
 #endif
 constexpr int PERSIST_THREADS = DIL_PERSIST_THREADS;
-constexpr uint32_t PERSIST_MAX_ROUNDS = 20000;
+constexpr int PERSIST_MAX_IDLE_ROUNDS = 20000;  // of one workgroup, without a signature
 // control words (uint32): 0 queue head, 1 status, 2 attempts executed.
 // Optional phase profile: PERSIST_PHASES uint64 cycle sums (assign, y, w, c,
 // z, commit) at a separate pointer, null when not profiling.
@@ -77,7 +77,7 @@ sg_persistent_kernel(SignArgs a, SlotRef sr, Chain chain, uint32_t *ctl, int cla
     __shared__ int own_done[S];
     __shared__ uint32_t slot_own[S], slot_nonce[S];
     __shared__ uint8_t w_unit[S];  // w work units: slot s, paired with s + u when s / u is even
-    __shared__ int n_own, queue_empty, n_units;
+    __shared__ int n_own, queue_empty, n_units, idle;
     const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
     constexpr int NW = PERSIST_THREADS / 64;
     const size_t slot0 = (size_t)blockIdx.x * S;
@@ -87,6 +87,7 @@ sg_persistent_kernel(SignArgs a, SlotRef sr, Chain chain, uint32_t *ctl, int cla
     if (tid == 0) {
         n_own = 0;
         queue_empty = 0;
+        idle = 0;
     }
     __syncthreads();
     // optional phase profile: workgroup cycles per phase, summed over
@@ -106,13 +107,7 @@ sg_persistent_kernel(SignArgs a, SlotRef sr, Chain chain, uint32_t *ctl, int cla
         }
     };
 
-    for (uint32_t round = 0;; ++round) {
-        if (round == PERSIST_MAX_ROUNDS) {
-            // no correct run gets here (each round succeeds per item with
-            // probability >= 1/5); stop instead of spinning and report it
-            if (tid == 0) atomicOr(ctl + 1, SIGN_STATUS_ROUND_CAP);
-            break;
-        }
+    for (;;) {
         if (tid == 0) {
             const int cap = claim > 0 && claim < S ? claim : S;
             int u = n_own;
@@ -150,6 +145,12 @@ sg_persistent_kernel(SignArgs a, SlotRef sr, Chain chain, uint32_t *ctl, int cla
         mark(0);
         const int u = n_own;
         if (u == 0) break;
+        if (idle == PERSIST_MAX_IDLE_ROUNDS) {
+            // no correct run gets here (each round succeeds per item with
+            // probability >= 1/5); stop instead of spinning and report it
+            if (tid == 0) atomicOr(ctl + 1, SIGN_STATUS_ROUND_CAP);
+            break;
+        }
         if (tid == 0) atomicAdd(ctl + 2, (uint32_t)S);  // attempts executed (incl. speculative)
 
         // the Keccak stages (y, c) run few serial permutation chains that the
@@ -231,6 +232,7 @@ sg_persistent_kernel(SignArgs a, SlotRef sr, Chain chain, uint32_t *ctl, int cla
                     own_next[k] = own_next[o];
                     ++k;
                 }
+            idle = k < u ? 0 : idle + 1;
             n_own = k;
         }
         __syncthreads();

@@ -63,13 +63,13 @@ constexpr size_t FIXED_ROW_MAX = 8192;
 // Dilithium5 960 / 938; resident 3,000 Dilithium5 862 / 910).
 constexpr uint32_t FIXED_WAVE_MAX = 2048, FIXED_WAVE_MAX_RESIDENT = 3072;
 // The persistent kernel, which needs no launches between stages, runs what is
-// left after the rounds and calls with fewer slots than half their items (a
-// round then covers a small part of them).  Rounds with enough slots are
-// faster at every size: 17 Dilithium3 items 0.22 ms (persistent 0.79), 1,000
-// Dilithium2 items 0.37 (0.79), 3,001 Dilithium5 0.98 (1.17), 8,000 Dilithium5
-// 1.73 (2.43), 10,000 Dilithium2 1.29 (1.72), 16,384 Dilithium3 2.45 (2.83),
-// 40,000 Dilithium3 5.0 (5.65).
-constexpr size_t ROUNDS_MAX_ITEMS_PER_SLOT = 2;
+// left after the rounds, and alone the calls with so many items per slot that
+// the sequence of rounds would leave most of them.  Rounds / persistent with two
+// slots per item: 17 Dilithium3 items 0.53 / 0.75 ms, 1,000 Dilithium2 0.50 /
+// 0.78, 3,001 Dilithium5 0.97 / 1.18, 10,000 Dilithium2 1.27 / 1.42, 16,384
+// Dilithium3 2.49 / 2.79; with 8 items per slot 1,000 Dilithium2 2.95 / 8.06,
+// 10,000 Dilithium2 4.8 / 7.7; 32: 36 / 52 and 29 / 31; 64: 122 / 67 and 67 / 69.
+constexpr size_t ROUNDS_MAX_ITEMS_PER_SLOT = 32;
 // Two chains from this batch on: 16,384 Dilithium3 items 2.45 ms (one chain
 // 2.60), 40,000 5.03 (5.36), 14,000 2.19 (2.29), 16,384 Dilithium5 2.87
 // (2.84); smaller ones lose as much as they gain (12,288 Dilithium2 1.46 and

@@ -270,13 +270,20 @@ int dil_set_kernel_tiling(int kind, int mode, int bucket, int value);
 int dil_get_kernel_tiling(int kind, int mode, size_t n);
 
 /* Signing context: owns the per-item rows (dil_sign_pool_row_bytes(mode, 0)
- * each), nslots attempt slots and the scheduler tables of either engine. */
+ * each), nslots attempt slots (dil_sign_temp_row_bytes(mode) each, rounded up
+ * to 256) and the scheduler tables of either engine. */
 typedef struct dil_sign_ctx dil_sign_ctx;
 int dil_sign_ctx_create(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t nslots);
+/* The same (resident_only != 0: dil_sign_ctx_create_resident) with more slots
+ * than nslots where signing gains from them and the memory is free: two per
+ * item up to 65,536, and for small batches 32 per item up to 8,192.  At most
+ * 0.7 / 0.94 / 1.26 GB for modes 2 / 3 / 5. */
+int dil_sign_ctx_create_auto(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t nslots,
+                             int resident_only);
 int dil_sign_ctx_destroy(dil_sign_ctx *ctx);
 /* Signing runs in device-driven rounds that choose their own launch shapes;
  * the two tilings below concern the persistent kernel, which runs alone for
- * calls with fewer slots than half their items and for the phase profile.
+ * calls with more than 32 items per slot and for the phase profile.
  * Tiling: slots per workgroup (0 = automatic, or 1, 8, 16,
  * 32), register budget as waves per SIMD (0 = automatic, or 2, 3, 4) and
  * workgroup count (0 = nslots / slots_per_block). */

@@ -4,6 +4,7 @@
 // allocation and can make any of them fail.  Device pointers are addresses
 // that nothing reads.
 //   host_calls join      errors while a signing call is being enqueued
+//   host_calls slots     the attempt slots that a signing context allocates
 // Prints what is wrong and exits with 1, or exits with 0.
 // Run by tests/test_host_sign_calls.py.
 #include <cstdarg>
@@ -29,6 +30,9 @@ struct Op {
 std::vector<Op> ops;
 long fail_at = -1;  // index of the operation that fails
 int last_error = 0;
+
+std::vector<size_t> allocations;  // sizes asked for
+size_t largest = SIZE_MAX;        // larger device allocations fail
 
 uintptr_t next_handle = 0x1000, next_address = uintptr_t(1) << 40;
 Handle make_handle() { return reinterpret_cast<Handle>(next_handle += 0x10); }
@@ -84,6 +88,8 @@ int hipStreamWaitEvent(Handle stream, Handle event, unsigned) { return op(WAIT, 
 int hipStreamSynchronize(Handle stream) { return op(SYNC, stream, nullptr); }
 
 int hipMalloc(void **p, size_t bytes) {
+    allocations.push_back(bytes);
+    if (bytes > largest) return last_error = 2;  // hipErrorOutOfMemory
     *p = reinterpret_cast<void *>(next_address);
     next_address += (bytes + 4095) / 4096 * 4096;
     return 0;
@@ -181,10 +187,57 @@ int join_after_errors() {
     return bad;
 }
 
+// A context allocates the slots that it was asked for; where the count is left
+// to the library, no more than it documents, and no error if that much is not
+// free.
+int slots_allocated() {
+    int bad = 0;
+    struct Case {
+        size_t max_batch, nslots, automatic;
+    };
+    const Case cases[] = {{1, 1, 32},          {17, 17, 544},         {333, 7, 8192},
+                          {1000, 1000, 8192},  {4096, 8192, 8192},    {5000, 2500, 10000},
+                          {16384, 16384, 32768}, {16384, 40000, 40000}, {40000, 40000, 65536}, {65536, 8192, 65536},
+                          {262144, 65536, 65536}};
+    for (const int mode : {2, 3, 5})
+        for (const Case &c : cases)
+            for (int form = 0; form < 5; ++form) {
+                // exact, exact resident, automatic, automatic resident, automatic without memory for more
+                const size_t slot = (dil_sign_temp_row_bytes(mode) + 255) / 256 * 256;
+                const size_t want = form == 2 || form == 3 ? c.automatic : c.nslots;
+                largest = SIZE_MAX;
+                if (form == 4) {
+                    if (c.automatic == c.nslots) continue;
+                    largest = slot * c.automatic - 1;
+                }
+                allocations.clear();
+                dil_sign_ctx *ctx = nullptr;
+                const int e = form == 0   ? dil_sign_ctx_create(&ctx, mode, c.max_batch, c.nslots)
+                              : form == 1 ? dil_sign_ctx_create_resident(&ctx, mode, c.max_batch, c.nslots)
+                                          : dil_sign_ctx_create_auto(&ctx, mode, c.max_batch, c.nslots, form != 2);
+                const size_t rows = allocations.empty() ? 0 : allocations[0];
+                const size_t lists = (c.max_batch + 511) / 512 * 8192 + 8192;
+                if (form == 4 && rows > largest) continue;  // the rows themselves do not fit
+                long found = 0, more = 0;
+                for (size_t i = 1; i < allocations.size(); ++i) {
+                    found += allocations[i] == slot * want;
+                    more += allocations[i] > slot * want && allocations[i] <= largest && allocations[i] != lists;
+                }
+                if (e || found != 1 || more)
+                    bad |= wrong("mode %d, %zu items, %zu slots, form %d: status %d, %ld allocations of %zu slots, %ld larger",
+                                 mode, c.max_batch, c.nslots, form, e, found, want, more);
+                if (form == 4 && hipGetLastError()) bad |= wrong("an error is left behind");
+                if (!e) dil_sign_ctx_destroy(ctx);
+            }
+    largest = SIZE_MAX;
+    return bad;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "join")) return join_after_errors();
+    if (!strcmp(what, "slots")) return slots_allocated();
     return 2;
 }

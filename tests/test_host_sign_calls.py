@@ -18,3 +18,7 @@ def _run(what):
 
 def test_second_chain_is_joined_after_any_error():
     _run("join")
+
+
+def test_contexts_allocate_the_slots_asked_for():
+    _run("slots")
