@@ -596,6 +596,8 @@ int dil_verify_device(int mode, int32_t *d_ret, const uint8_t *d_sig, size_t sig
 
 /* ------------------------------------------------------ signing context */
 
+constexpr size_t CALL_EVENTS = 4;
+
 struct dil_sign_ctx {
     int mode = 0;
     size_t max_batch = 0, nslots = 0;
@@ -611,7 +613,7 @@ struct dil_sign_ctx {
     uint8_t *h_done = nullptr, *d_done = nullptr;
     uint64_t *h_copy = nullptr, *d_copy = nullptr;
     int slots_per_block = 0, blocks = 0, occupancy = 0;
-    // timing: one (start, fixed done, loop done) event triple per timed call
+    // timing: the events (start, fixed stage of either chain of rounds done, loop done) of each timed call
     std::vector<hipEvent_t> ev;
     size_t timing_cap = 0, timed = 0;
     bool resident_only = false;  // rows without the per-item expanded arrays
@@ -673,13 +675,14 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
         const SlotRef slots{c->slots + TempLayout<P>::SLOT, c->slot_pitch, c->slots + TempLayout<P>::SIG,
                             c->slot_pitch};
         int e;
-        hipEvent_t *e3 = timing && c->timed < c->timing_cap ? &c->ev[3 * c->timed] : nullptr;
-        if (e3 && (e = (int)hipEventRecord(e3[0], st))) return e;
+        hipEvent_t *ev = timing && c->timed < c->timing_cap ? &c->ev[CALL_EVENTS * c->timed] : nullptr;
+        if (ev && (e = (int)hipEventRecord(ev[0], st))) return e;
         if (engine == DIL_ENGINE_PERSTAGE) {
             // the per-stage scheduler launches the fixed part itself; the
             // status word is cleared here (the persistent launch clears it)
             if ((e = launch_zero_ctl(c->d_head, nullptr, st))) return e;
-            if (e3 && (e = (int)hipEventRecord(e3[1], st))) return e;
+            for (int k = 1; ev && k < 3; ++k)
+                if ((e = (int)hipEventRecord(ev[k], st))) return e;
             const SlotRef items{c->rows + SignLayout<P>::SLOT, c->row_pitch, d_sig, sig_pitch};
             e = sign_perstage(c->mode, a, items, slots, c->nslots, c->sign_lut.data(), c->h_exec, c->d_exec,
                               c->h_done, c->d_done, c->h_copy, c->d_copy, st);
@@ -690,13 +693,13 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
             // a tiling is for the slots the caller asked for
             const PersistTiling tiling{c->nslots, c->slots_per_block, c->blocks, c->claim};
             e = sign_call(c->mode, a, slots, c->round_slots, lists, tiling, c->d_head, ph, st,
-                          e3 ? e3[1] : nullptr);
+                          ev ? ev + 1 : nullptr);
             if (e == -3) return DIL_ERANGE;
         }
         if (e) return e;
         if (ks && (e = launch_sign_key_check(c->mode, a, c->d_head + 1, st))) return e;
-        if (e3) {
-            if ((e = (int)hipEventRecord(e3[2], st))) return e;
+        if (ev) {
+            if ((e = (int)hipEventRecord(ev[3], st))) return e;
             ++c->timed;
         }
         return 0;
@@ -813,7 +816,7 @@ int dil_sign_ctx_set_claim(dil_sign_ctx *c, int items_per_block) {
 
 int dil_sign_ctx_enable_timing(dil_sign_ctx *c, int max_calls) {
     if (!c || max_calls < 0) return DIL_EINVAL;
-    while (c->ev.size() < 3 * (size_t)max_calls) {
+    while (c->ev.size() < CALL_EVENTS * (size_t)max_calls) {
         hipEvent_t e;
         int r = (int)hipEventCreate(&e);
         if (r) return r;
@@ -828,11 +831,17 @@ int dil_sign_ctx_timed_calls(dil_sign_ctx *c) { return c ? (int)c->timed : 0; }
 
 int dil_sign_ctx_timing(dil_sign_ctx *c, int call, float *fixed_ms, float *loop_ms) {
     if (!c || call < 0 || (size_t)call >= c->timed) return DIL_EINVAL;
-    hipEvent_t *e3 = &c->ev[3 * (size_t)call];
-    int e = (int)hipEventSynchronize(e3[2]);
+    hipEvent_t *ev = &c->ev[CALL_EVENTS * (size_t)call];
+    int e = (int)hipEventSynchronize(ev[3]);
     if (e) return e;
-    if (fixed_ms && (e = (int)hipEventElapsedTime(fixed_ms, e3[0], e3[1]))) return e;
-    if (loop_ms && (e = (int)hipEventElapsedTime(loop_ms, e3[1], e3[2]))) return e;
+    // the stage ends with the later of the chains'
+    float fixed[2], total;
+    for (int k = 0; k < 2; ++k)
+        if ((e = (int)hipEventElapsedTime(&fixed[k], ev[0], ev[1 + k]))) return e;
+    if ((e = (int)hipEventElapsedTime(&total, ev[0], ev[3]))) return e;
+    const float f = std::max(fixed[0], fixed[1]);
+    if (fixed_ms) *fixed_ms = f;
+    if (loop_ms) *loop_ms = total - f;
     return 0;
 }
 

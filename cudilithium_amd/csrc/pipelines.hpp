@@ -93,11 +93,11 @@ int launch_sign_key_check(int mode, const SignArgs &a, uint32_t *status, hipStre
 // kernel, so graph capture records no memset node).
 int launch_zero_ctl(uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st);
 // A whole signing call, over nslots attempt slots: device-driven rounds
-// (sign_rounds.hip), or for large batches the persistent kernel.
+// (sign_rounds.hip), or with many items per slot the persistent kernel.
 // lists: sign_lists_chunks(n) chunks of sign_lists_chunk_bytes() scratch
 // bytes (8-aligned), lists.pitch apart.  phase_sums: null, or the persistent
-// kernel runs and fills them.  fixed_done: null, or an event recorded after
-// the fixed stage.
+// kernel runs and fills them.  fixed_done: null, or two events recorded after
+// the fixed stage of either chain of rounds.
 struct ChunkRef {
     uint8_t *base;
     size_t pitch;
@@ -110,7 +110,7 @@ size_t sign_lists_chunks(size_t n);
 size_t sign_lists_chunk_bytes();
 int sign_call(int mode, const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRef &lists,
               const PersistTiling &tiling, uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st,
-              hipEvent_t fixed_done);
+              hipEvent_t *fixed_done);
 int sign_perstage(int mode, const SignArgs &a, const SlotRef &item_slots, const SlotRef &temp_slots, size_t thr,
                   SignLutEntry *sign_lut, uint32_t *h_exec, uint32_t *d_exec, uint8_t *h_done, uint8_t *d_done,
                   uint64_t *h_copy, uint64_t *d_copy, hipStream_t st);

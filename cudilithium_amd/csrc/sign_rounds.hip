@@ -472,7 +472,7 @@ struct ForkedStream {
 
 template <class P>
 int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRef &lists, const PersistTiling &tiling,
-              uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st, hipEvent_t fixed_done) {
+              uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st, hipEvent_t *fixed_done) {
     int e = launch_zero_ctl(ctl, phase_sums, st);
     if (e) return e;
     const bool rounds = !phase_sums && a.n <= ROUNDS_MAX_ITEMS_PER_SLOT * nslots;
@@ -502,8 +502,9 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
     }
     for (int k = 0; k < nchain; ++k) {
         if ((e = launch_fixed<P>(a, ch[k], cs[k]))) return e;
-        if (k == 0 && fixed_done && (e = (int)hipEventRecord(fixed_done, cs[0]))) return e;
     }
+    for (int k = 0; fixed_done && k < 2; ++k)
+        if ((e = (int)hipEventRecord(fixed_done[k], cs[k < nchain ? k : 0]))) return e;
     if (!rounds) {
         const size_t ns = tiling.nslots ? tiling.nslots : nslots;
         const int spb = tiling.slots_per_block ? tiling.slots_per_block : default_slots_per_block(ns);
@@ -538,7 +539,7 @@ size_t sign_lists_chunk_bytes() { return CHAIN_CHUNK_BYTES; }
 
 int sign_call(int mode, const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRef &lists,
               const PersistTiling &tiling, uint32_t *ctl, unsigned long long *phase_sums, hipStream_t st,
-              hipEvent_t fixed_done) {
+              hipEvent_t *fixed_done) {
     if (a.n == 0) return 0;
     if (nslots == 0) return -3;
     switch (mode) {

@@ -296,10 +296,11 @@ int dil_sign_ctx_set_tiling(dil_sign_ctx *ctx, int slots_per_block, int occupanc
  * the rounds took over the batches whose last items it spread. */
 #define DIL_CLAIM_GUIDED 0x10000
 int dil_sign_ctx_set_claim(dil_sign_ctx *ctx, int items_per_block);
-/* Records HIP events on the call's stream around the fixed stage and the
- * rejection loop of the next max_calls dil_sign_device calls (0 turns timing
- * off and forgets earlier records).  dil_sign_ctx_timing waits for call
- * `call` (0-based) and returns its two durations. */
+/* Records HIP events around the fixed stage and the rejection loop of the next
+ * max_calls dil_sign_device calls (0 turns timing off and forgets earlier
+ * records).  dil_sign_ctx_timing waits for call `call` (0-based) and returns
+ * its two durations; a call that runs as two chains of rounds (12,288 items
+ * and more) ends its fixed stage with the later of the two. */
 int dil_sign_ctx_enable_timing(dil_sign_ctx *ctx, int max_calls);
 int dil_sign_ctx_timed_calls(dil_sign_ctx *ctx);
 int dil_sign_ctx_timing(dil_sign_ctx *ctx, int call, float *fixed_ms, float *loop_ms);

@@ -5,6 +5,7 @@
 // that nothing reads.
 //   host_calls join      errors while a signing call is being enqueued
 //   host_calls slots     the attempt slots that a signing context allocates
+//   host_calls timing    the two durations of a timed call
 // Prints what is wrong and exits with 1, or exits with 0.
 // Run by tests/test_host_sign_calls.py.
 #include <cstdarg>
@@ -30,6 +31,7 @@ struct Op {
 std::vector<Op> ops;
 long fail_at = -1;  // index of the operation that fails
 int last_error = 0;
+Handle caller = nullptr;
 
 std::vector<size_t> allocations;  // sizes asked for
 size_t largest = SIZE_MAX;        // larger device allocations fail
@@ -124,6 +126,22 @@ int hipEventCreate(Handle *e) {
     return 0;
 }
 int hipEventDestroy(Handle) { return 0; }
+int hipEventSynchronize(Handle) { return 0; }
+// An event's time is the number of launches before it on its stream, a launch
+// of the caller's stream taking 1 ms and one of any other 100 ms.
+int hipEventElapsedTime(float *ms, Handle from, Handle to) {
+    auto time = [](Handle event) {
+        for (size_t i = ops.size(); i-- > 0;)
+            if (ops[i].kind == RECORD && ops[i].event == event) {
+                long n = 0;
+                for (size_t j = 0; j < i; ++j) n += ops[j].kind == LAUNCH && ops[j].stream == ops[i].stream;
+                return n * (ops[i].stream == caller ? 1L : 100L);
+            }
+        return -100000L;
+    };
+    *ms = (float)(time(to) - time(from));
+    return 0;
+}
 
 }  // extern "C"
 
@@ -233,11 +251,36 @@ int slots_allocated() {
     return bad;
 }
 
+// The fixed stage of a call ends when it has ended on both streams.
+int timed_calls() {
+    int bad = 0;
+    for (const size_t n : {1000, 16384}) {
+        dil_sign_ctx *ctx = nullptr;
+        if (dil_sign_ctx_create(&ctx, 3, n, n) || dil_sign_ctx_enable_timing(ctx, 1)) return wrong("context");
+        caller = make_handle();
+        ops.clear();
+        if (sign(ctx, 3, n, caller)) return wrong("call");
+        long all = 0, second = 0;
+        for (const Op &o : ops) (o.stream == caller ? all : second) += o.kind == LAUNCH;
+        float fixed = 0, loop = 0;
+        const int e = dil_sign_ctx_timing(ctx, 0, &fixed, &loop);
+        // two launches of the caller's stream (clearing the control words and
+        // the stage), or one of the second stream
+        const float want = second ? 100.f : 2.f;
+        if (e || fixed != want || loop != (float)all - want)
+            bad |= wrong("%zu items: status %d, fixed %g ms, loop %g ms of %ld launches", n, e, fixed, loop, all);
+        if ((n >= 12288) != (second > 0)) bad |= wrong("%zu items: %ld launches on a second stream", n, second);
+        dil_sign_ctx_destroy(ctx);
+    }
+    return bad;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "join")) return join_after_errors();
     if (!strcmp(what, "slots")) return slots_allocated();
+    if (!strcmp(what, "timing")) return timed_calls();
     return 2;
 }

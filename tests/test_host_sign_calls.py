@@ -22,3 +22,7 @@ def test_second_chain_is_joined_after_any_error():
 
 def test_contexts_allocate_the_slots_asked_for():
     _run("slots")
+
+
+def test_fixed_stage_ends_on_both_streams():
+    _run("timing")
