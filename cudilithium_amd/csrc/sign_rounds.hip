@@ -180,12 +180,16 @@ __device__ __forceinline__ Attempt slot_attempt(const Chain &ch, const ChainCtl 
 // Layout of a round's hashes by their number.  A chained permutation of a
 // lone wave takes 8.6 / 5.9 / 3.5 / 2.2 us with one, two, sixteen or 64 lanes
 // per state, and the card runs 9.6 / 7.4 / 2.1 / 0.9 G permutations/s: the
-// wave form while its waves are few, then rows (challenges: 8,192 take 40 us,
-// with pairs 64; there is no such range for the shorter mask chains), pairs
-// and one lane.  17 resident Dilithium3 items 151 us (157 with 2,048 for both
-// limits, 218 without the wave form), 3,001 Dilithium5 919 (938, 977).
+// wave form while its waves are few, then (challenges) rows, pairs and one
+// lane; the mask chains are shorter and have no rows.  17 resident Dilithium3
+// items 151 us (157 with 2,048 for both limits, 218 without the wave form).
+// Challenges, whole calls with 32-byte messages and rounds of that many
+// attempts, waves / rows: 2,500 Dilithium3 1067 / 1098 us, 3,000 Dilithium2
+// 883 / 905, 3,000 Dilithium5 657 / 674; 4,000 Dilithium3 1301 / 1200, 4,096
+// Dilithium2 618 / 578, 4,096 Dilithium5 806 / 754; rows / pairs: one round of
+// 8,192 40 / 64 us.
 constexpr uint32_t Y_WAVE_MAX = 4096, Y_PAIR_MAX = 32768;
-constexpr uint32_t C_WAVE_MAX = 4096, C_ROW_MAX = 8192;
+constexpr uint32_t C_WAVE_MAX = 3072, C_ROW_MAX = 8192;
 constexpr uint32_t ROW_LDS = 4 * 4 * ROW_LDS_WORDS;
 static_assert(ROW_LDS >= 4 * WAVE_LDS_WORDS, "the row form's LDS also serves the wave form");
 

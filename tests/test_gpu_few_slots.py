@@ -29,3 +29,10 @@ def test_few_slots_match_oracle(mode, n, nslots):
 def test_no_limit_on_the_rounds_that_a_long_queue_takes():
     # 20,000 rounds without a signature are an error; with signatures they are not
     assert _check(2, 6000, 1) > 20000
+
+
+@pytest.mark.parametrize("mode", [2, 3, 5])
+@pytest.mark.parametrize("n", [1536, 1537])
+def test_challenge_forms_change_at_3072_attempts(mode, n):
+    # two attempts for each item in the first round: 3,072 with a wave each, 3,074 with a row
+    _check(mode, n, 2 * n)
