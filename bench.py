@@ -7,7 +7,8 @@ launches per step.  A step signs the whole batch.
 
 Printed on one JSON line: throughput (signatures/s, the default engine
 replayed as a HIP graph), the roofline of its dominant part (the kernels of
-the rejection rounds, integer-VALU bound), the oracle's CPU rate on a bounded
+the rejection rounds, integer-VALU bound; the least instructions of its work
+against the card's issue rate), the oracle's CPU rate on a bounded
 sample, the per-stage (reference architecture) GPU form on the same inputs,
 a serving summary (resident keys, continuous batching: p50 / p99 latency
 at two offered loads) and the drop-in call's rate with host buffers.
@@ -73,8 +74,7 @@ def bench_sign(args, mode: int):
     d_sk = DeviceBuffer.from_array(sk)
     d_msgs = api.DeviceMessages(msgs)
     d_sig = DeviceBuffer(n * sigb)
-    ctx = api.SignContext(mode, n, args.slots or None)  # autotuned tiling unless overridden
-    nslots = ctx.nslots
+    ctx = api.SignContext(mode, n, args.slots or None)
     if args.spb or args.occupancy:
         ctx.set_tiling(args.spb, args.occupancy)
     if args.claim:
@@ -113,19 +113,9 @@ def bench_sign(args, mode: int):
     wall = time.perf_counter() - t0
     sig = d_sig.download((n, sigb), np.uint8)
     attempts = ctx.attempt_counts(n)
+    executed = ctx.executed_attempts()
     graph_matches_eager = bool(np.array_equal(sig, sig_eager))
     log(f"[bench] graph replay: {args.steps} steps in {wall * 1e3:.2f} ms; bytes equal eager: {graph_matches_eager}")
-
-    # phase profile of one more call, outside the timed region
-    ctx.profile_phases(True)
-    ctx.sign_device(d_sig, d_sk, d_msgs, api.ENGINE_PERSISTENT)
-    phases = ctx.phase_cycles()
-    executed = ctx.executed_attempts()
-    ctx.profile_phases(False)
-    tot = sum(phases.values()) or 1
-    phase_share = {k: round(v / tot, 4) for k, v in phases.items()}
-    log(f"[bench] loop phase shares (workgroup cycles): {phase_share}; executed attempts "
-        f"{ctx.executed_attempts()}")
 
     # parity on a sample (outside the timed region)
     import oracle
@@ -136,12 +126,14 @@ def bench_sign(args, mode: int):
         and graph_matches_eager
     log(f"[bench] parity vs oracle on {len(idx)} items: {parity}")
 
-    # roofline of the rejection loop: algorithmic int32 ops of the attempts the
-    # specification makes, over the event-timed duration of the rounds (with two
-    # chains, from the end of the first one's fixed stage on)
+    # roofline of the rejection loop: the instructions that the attempts of the
+    # specification take at least, over the event-timed duration of the rounds
     loop_ms = float(np.mean([t[1] for t in tim]))
-    ops = float(attempts.sum()) * workmodel.sign_attempt_ops(mode)
-    achieved = ops / (loop_ms * 1e-3) / 1e12
+    needed = float(attempts.sum())
+    ops = needed * workmodel.sign_attempt_ops(mode)
+    instr = needed * workmodel.sign_attempt_instr(mode)
+    whole = instr + sum(workmodel.sign_fixed_instr(mode, len(m)) for m in msgs)
+    achieved = instr / (loop_ms * 1e-3) / 1e12
     value = n * args.steps / wall
 
     perstage = None
@@ -161,7 +153,7 @@ def bench_sign(args, mode: int):
             ps_sig = d_sig.download((n, sigb), np.uint8)
             del ps
             r = {"value": n / ps_wall, "unit": "signs/s", "exec_threshold": thr,
-                 "ms_per_step": ps_wall * 1e3, "bit_exact_vs_persistent": bool(np.array_equal(ps_sig, sig))}
+                 "ms_per_step": ps_wall * 1e3, "bit_exact_vs_rounds": bool(np.array_equal(ps_sig, sig))}
             log(f"[bench] per-stage form, exec_threshold {thr}: {ps_wall * 1e3:.2f} ms per batch")
             if perstage is None:
                 perstage = r
@@ -173,27 +165,25 @@ def bench_sign(args, mode: int):
         cpu = cpu_baseline_sign(mode, msgs, sk, args.cpu_seconds)
 
     cfg = {"workload": f"dilithium{mode}_sign_{n}_msg_loguniform_32B-4KiB",
-           "batch": n, "mode": mode, "engine": "persistent+graph", "slots": nslots,
-           "slots_per_block": ctx.slots_per_block or "auto", "occupancy": ctx.occupancy or "auto",
-           "claim": (ctx.claim & 0xFFFF) or "slots", "guided_claims": bool(ctx.claim & api.CLAIM_GUIDED),
-           "mean_attempts": float(attempts.mean()), "loop_phase_shares": phase_share}
+           "batch": n, "mode": mode, "engine": "rounds+graph", "slots": ctx.slots,
+           "mean_attempts": float(attempts.mean())}
     return {
         "metric": METRIC, "value": value, "unit": "signs/s", "ms_per_step": wall / args.steps * 1e3,
         "dtype": "int32", "config": cfg, "parity": "bit-exact" if parity else "MISMATCH",
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_INT32_TOPS, "unit": "TOP/s",
                      "frac": achieved / PEAK_INT32_TOPS, "traffic": TRAFFIC_BYTES.get(cfg["workload"]),
                      "kernel": "sg_ry / sg_rw / sg_rc / sg_rz / sg_rs / sg_plan", "kernel_ms": loop_ms,
-                     "algorithmic_ops": ops},
-        "cpu_baseline": cpu, "perstage_gpu_baseline": perstage, "eager_persistent_value": eager_value,
+                     "least_instructions": instr, "algorithmic_ops": ops,
+                     "algorithmic_frac": ops / (loop_ms * 1e-3) / 1e12 / PEAK_INT32_TOPS},
+        "cpu_baseline": cpu, "perstage_gpu_baseline": perstage, "eager_value": eager_value,
         "speedup_vs_perstage": (value / perstage["value"]) if perstage else None,
         "speedup_vs_perstage_at_exec_threshold_batch":
             (value / perstage["at_exec_threshold_batch"]["value"]) if perstage else None,
         "step": {"fixed_ms": float(np.mean([t[0] for t in tim])), "loop_ms": loop_ms,
                  "graph_ms_per_step": wall / args.steps * 1e3,
-                 "whole_step_frac": (ops + n * float(np.mean([workmodel.sign_fixed_ops(mode, len(m)) for m in msgs])))
-                 / (wall / args.steps) / 1e12 / PEAK_INT32_TOPS,
-                 "executed_attempts": int(executed), "needed_attempts": int(attempts.sum()),
-                 "speculation_ratio": executed / float(attempts.sum())},
+                 "whole_step_frac": whole / (wall / args.steps) / 1e12 / PEAK_INT32_TOPS,
+                 "executed_attempts": int(executed), "needed_attempts": int(needed),
+                 "speculation_ratio": executed / needed},
     }
 
 
@@ -379,9 +369,10 @@ def bench_verify(args, mode: int = 5):
     parity = bool(np.array_equal(ret, oret)) and bool(np.array_equal(ret, want)) and bool(np.array_equal(ret, ret_eager))
     value = n * args.steps / wall
     kops = {k: n * v for k, v in workmodel.verify_kernel_ops(mode, 1024).items()}
+    kins = {k: n * v for k, v in workmodel.verify_kernel_ops(mode, 1024, workmodel.INSTR_KECCAK).items()}
     main_ms = float(kms[1])
-    achieved = kops["vf_main"] / (main_ms * 1e-3) / 1e12
-    pipe = sum(kops.values()) / (wall / args.steps) / 1e12
+    achieved = kins["vf_main"] / (main_ms * 1e-3) / 1e12
+    pipe = sum(kins.values()) / (wall / args.steps) / 1e12
     log(f"[bench] verify5: graph {wall / args.steps * 1e3:.3f} ms per batch; kernels vf_prep / vf_main / vf_final "
         f"{kms[0]:.3f} / {kms[1]:.3f} / {kms[2]:.3f} ms")
     return {"metric": METRIC, "value": value, "unit": "verifies/s", "ms_per_step": wall / args.steps * 1e3,
@@ -393,7 +384,9 @@ def bench_verify(args, mode: int = 5):
             "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_INT32_TOPS, "unit": "TOP/s",
                          "frac": achieved / PEAK_INT32_TOPS,
                          "traffic": TRAFFIC_BYTES.get(f"dilithium{mode}_verify_{n}_msg_1KiB_10pct_bitflips_vf_main"),
-                         "kernel": "vf_main_kernel", "kernel_ms": main_ms, "algorithmic_ops": kops["vf_main"],
+                         "kernel": "vf_main_kernel", "kernel_ms": main_ms, "least_instructions": kins["vf_main"],
+                         "algorithmic_ops": kops["vf_main"],
+                         "algorithmic_frac": kops["vf_main"] / (main_ms * 1e-3) / 1e12 / PEAK_INT32_TOPS,
                          "pipeline_frac": pipe / PEAK_INT32_TOPS},
             "cpu_baseline": None}
 
@@ -748,11 +741,11 @@ def main():
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--workload", default="sign3")
     ap.add_argument("--batch", type=int, default=0)
-    ap.add_argument("--slots", type=int, default=0, help="attempt slots (default: batch)")
-    ap.add_argument("--spb", type=int, default=0, help="slots per workgroup (0 = autotuned)")
-    ap.add_argument("--occupancy", type=int, default=0, help="waves per SIMD of the loop kernel (0 = autotuned)")
-    ap.add_argument("--claim", type=int, default=0, help="items per workgroup of the loop kernel (0 = its slots)")
-    ap.add_argument("--claim-guided", action="store_true", help="guided claims near the end of the queue")
+    ap.add_argument("--slots", type=int, default=0, help="attempt slots, exactly (default: the library's choice)")
+    ap.add_argument("--spb", type=int, default=0, help="persistent kernel: slots per workgroup (0 = autotuned)")
+    ap.add_argument("--occupancy", type=int, default=0, help="accepted, without effect")
+    ap.add_argument("--claim", type=int, default=0, help="persistent kernel: items per workgroup (0 = its slots)")
+    ap.add_argument("--claim-guided", action="store_true", help="accepted, without effect")
     ap.add_argument("--check", type=int, default=128, help="items checked against the oracle")
     ap.add_argument("--cpu-seconds", type=float, default=8.0)
     ap.add_argument("--no-cpu", action="store_true")

@@ -100,6 +100,7 @@ def _register():
     R("dil_keystore_keygen", c_int, [c_void_p, c_size_t, c_void_p, c_size_t, ctypes.c_uint64, c_size_t, c_void_p])
     R("dil_keystore_export", c_int, [c_void_p, c_size_t, c_size_t, c_void_p, c_size_t, c_void_p, c_size_t, c_void_p])
     R("dil_sign_ctx_create_resident", c_int, [pp, c_int, c_size_t, c_size_t])
+    R("dil_sign_ctx_slots", c_size_t, [c_void_p])
     R("dil_sign_ctx_create_auto", c_int, [pp, c_int, c_size_t, c_size_t, c_int])
     R("dil_sign_device_resident", c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p,
                                           c_void_p, c_size_t, c_int, c_void_p])
@@ -364,6 +365,11 @@ class SignContext:
     slots_per_block = 0
     occupancy = 0
     claim = 0
+
+    @property
+    def slots(self) -> int:
+        """The attempt slots held: nslots, or more if the count was left open."""
+        return int(L().dil_sign_ctx_slots(self.handle))
 
     def set_tiling(self, slots_per_block: int = 0, occupancy: int = 0, blocks: int = 0) -> None:
         _lib.check(L().dil_sign_ctx_set_tiling(self.handle, slots_per_block, occupancy, blocks), "set_tiling")

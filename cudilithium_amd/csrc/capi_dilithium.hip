@@ -795,6 +795,8 @@ int dil_sign_ctx_create_auto(dil_sign_ctx **out, int mode, size_t max_batch, siz
     return ctx_create(out, mode, max_batch, nslots, round_slots_for(max_batch, nslots), resident_only != 0);
 }
 
+size_t dil_sign_ctx_slots(const dil_sign_ctx *c) { return c ? c->round_slots : 0; }
+
 int dil_sign_ctx_set_tiling(dil_sign_ctx *c, int slots_per_block, int occupancy, int blocks) {
     if (!c) return DIL_EINVAL;
     if (slots_per_block != 0 && slots_per_block != 1 && slots_per_block != 8 && slots_per_block != 16 &&

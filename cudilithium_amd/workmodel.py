@@ -7,6 +7,11 @@ depend on the implementation (the figures roofline.achieved uses).
                         then one add and one sub)
     OPS_MONT   = 5      per pointwise Montgomery product or INTT scaling
 
+    INSTR_KECCAK = 4320 the least instructions per lane of a permutation: gfx950's
+                        three-input v_bitop3 joins theta's and chi's operations
+                        (24 rounds x 180); the denominator of a fraction of the
+                        card's issue rate, which counted operations can exceed
+
 Keccak permutation counts follow the specification's squeeze policy:
 ExpandA 5 SHAKE128 blocks, ExpandMask 5 SHAKE256 blocks, ExpandS 2 blocks,
 and a hash of inlen bytes costs floor(inlen / rate) + out_blocks.
@@ -14,6 +19,7 @@ and a hash of inlen bytes costs floor(inlen / rate) + out_blocks.
 from __future__ import annotations
 
 OPS_KECCAK = 6240
+INSTR_KECCAK = 4320
 OPS_BFLY = 7
 OPS_MONT = 5
 N = 256
@@ -44,12 +50,25 @@ def sign_attempt_counts(mode: int):
     return perms, fwd, inv, pw
 
 
-def _ops(perms, fwd, inv, pw):
-    return perms * OPS_KECCAK + fwd * FWD_NTT_OPS + inv * INV_NTT_OPS + pw * POINTWISE_OPS
+def _ops(perms, fwd, inv, pw, keccak=OPS_KECCAK):
+    return perms * keccak + fwd * FWD_NTT_OPS + inv * INV_NTT_OPS + pw * POINTWISE_OPS
 
 
 def sign_attempt_ops(mode: int) -> int:
     return _ops(*sign_attempt_counts(mode))
+
+
+def sign_attempt_instr(mode: int) -> int:
+    """Least vector instructions of an attempt here: c s1, c s2 and c t0 run on
+    the matrix cores, which leaves the hashes, NTT(y), A y^ and w's INTT."""
+    k, l, _, _ = PARAMS[mode]
+    return _ops(sign_attempt_counts(mode)[0], l, k, k * l, INSTR_KECCAK)
+
+
+def sign_fixed_instr(mode: int, mlen: int) -> int:
+    """The hashes of sign_fixed_ops: the secret key is used as it is unpacked."""
+    k, l, _, _ = PARAMS[mode]
+    return (_hash_perms(32 + mlen) + 1 + 5 * k * l) * INSTR_KECCAK
 
 
 def sign_fixed_ops(mode: int, mlen: int) -> int:
@@ -59,23 +78,23 @@ def sign_fixed_ops(mode: int, mlen: int) -> int:
     return _ops(perms, l + 2 * k, 0, 0)
 
 
-def verify_ops(mode: int, mlen: int) -> int:
+def verify_ops(mode: int, mlen: int, keccak: int = OPS_KECCAK) -> int:
     """tr, mu, ExpandA, SampleInBall, c~'; NTT of z, c, t1; A z; c t1; INTT
     (verify.cu:28-325)."""
     k, l, w1b, pkb = PARAMS[mode]
     perms = _hash_perms(pkb) + _hash_perms(32 + mlen) + 5 * k * l + 1 + _hash_perms(64 + k * w1b)
-    return _ops(perms, l + 1 + k, k, k * l + k)
+    return _ops(perms, l + 1 + k, k, k * l + k, keccak)
 
 
-def verify_kernel_ops(mode: int, mlen: int) -> dict:
-    """verify_ops split by the engine's three launches: vf_prep (tr, mu,
-    SampleInBall), vf_main (ExpandA, NTT of z / c / t1, A z - c t1, INTT) and
-    vf_final (c~' = H(mu || w1'))."""
+def verify_kernel_ops(mode: int, mlen: int, keccak: int = OPS_KECCAK) -> dict:
+    """verify_ops split by the engine's three launches, as they run for batches
+    above 4,096 items: vf_prep (SampleInBall), vf_main (tr, mu, ExpandA, NTT of
+    z / c / t1, A z - c t1, INTT) and vf_final (c~' = H(mu || w1'))."""
     k, l, w1b, pkb = PARAMS[mode]
-    prep = _ops(_hash_perms(pkb) + _hash_perms(32 + mlen) + 1, 0, 0, 0)
-    main = _ops(5 * k * l, l + 1 + k, k, k * l + k)
-    final = _ops(_hash_perms(64 + k * w1b), 0, 0, 0)
-    assert prep + main + final == verify_ops(mode, mlen)
+    prep = _ops(1, 0, 0, 0, keccak)
+    main = _ops(_hash_perms(pkb) + _hash_perms(32 + mlen) + 5 * k * l, l + 1 + k, k, k * l + k, keccak)
+    final = _ops(_hash_perms(64 + k * w1b), 0, 0, 0, keccak)
+    assert prep + main + final == verify_ops(mode, mlen, keccak)
     return {"vf_prep": prep, "vf_main": main, "vf_final": final}
 
 

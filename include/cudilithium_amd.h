@@ -280,6 +280,8 @@ int dil_sign_ctx_create(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t n
  * 0.7 / 0.94 / 1.26 GB for modes 2 / 3 / 5. */
 int dil_sign_ctx_create_auto(dil_sign_ctx **ctx, int mode, size_t max_batch, size_t nslots,
                              int resident_only);
+/* The slots that the context holds. */
+size_t dil_sign_ctx_slots(const dil_sign_ctx *ctx);
 int dil_sign_ctx_destroy(dil_sign_ctx *ctx);
 /* Signing runs in device-driven rounds that choose their own launch shapes;
  * the two tilings below concern the persistent kernel, which runs alone for

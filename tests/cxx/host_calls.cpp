@@ -244,6 +244,7 @@ int slots_allocated() {
                 if (e || found != 1 || more)
                     bad |= wrong("mode %d, %zu items, %zu slots, form %d: status %d, %ld allocations of %zu slots, %ld larger",
                                  mode, c.max_batch, c.nslots, form, e, found, want, more);
+                if (!e && dil_sign_ctx_slots(ctx) != want) bad |= wrong("the context reports other slots");
                 if (form == 4 && hipGetLastError()) bad |= wrong("an error is left behind");
                 if (!e) dil_sign_ctx_destroy(ctx);
             }
