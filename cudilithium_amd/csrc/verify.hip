@@ -607,10 +607,10 @@ __global__ __launch_bounds__(256) void vf_final_kernel(VerifyArgs a) {
     }
 }
 
+// The values a tiling may choose; they stayed as they were when the kernel's
+// LDS shrank, so a recorded or refused value stays so.
 template <class P, int G>
 constexpr bool vf_fits() {
-    // the values a tiling may choose: what the kernel's LDS allowed when the
-    // streaming form shared this tiling
     return G * (P::L + P::K + 1) * N * 4 + 8 * 1024 <= 160 * 1024;
 }
 
@@ -619,7 +619,8 @@ static int launch_vf_res_g(const VerifyArgs &a, bool row, bool own_c, hipStream_
     if constexpr (!vf_fits<P, G>()) {
         return -1;
     } else {
-        const size_t smem = sizeof(VfResShared<P, G>);
+        constexpr size_t smem = sizeof(VfResShared<P, G>);
+        static_assert(smem <= 160 * 1024, "the LDS of a CU");
         auto go = [&](auto kernel, uint32_t per) {
             if (smem > 64 * 1024) {
                 const hipError_t attr = hipFuncSetAttribute((const void *)kernel,
