@@ -448,7 +448,7 @@ class SignContext:
         return d_sig.download((n, self.sig_bytes), np.uint8)
 
     def graph(self, d_sig: DeviceBuffer, d_sk: DeviceBuffer, msgs: DeviceMessages) -> "Graph":
-        """The persistent-engine call sign_device(d_sig, d_sk, msgs) captured
+        """The call sign_device(d_sig, d_sk, msgs) captured
         as a HIP graph (replayed by Graph.launch)."""
         p = c_void_p()
         _lib.check(L().dil_sign_graph_create(ctypes.byref(p), self.handle, d_sig.ptr, self.sig_bytes, d_sk.ptr,
@@ -539,7 +539,7 @@ def keypair_graph(mode: int, d_pk: DeviceBuffer, d_sk: DeviceBuffer, n: int, d_w
 
 class KeyStore:
     """dil_keystore: `capacity` resident keys of one mode with their expanded
-    A, s1^, s2^, t0^, t1^ and tr."""
+    A, t1^, int8 s1, s2, t0 and tr."""
 
     def __init__(self, mode: int, capacity: int):
         p = c_void_p()

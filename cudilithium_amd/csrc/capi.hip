@@ -43,13 +43,14 @@ int create_queue_stream(hipStream_t *st) {
     return (int)hipExtStreamCreateWithCUMask(st, (uint32_t)mask.size(), mask.data());
 }
 
-AuxStreams *aux_streams(hipStream_t caller) {
+AuxStream *aux_stream(hipStream_t caller) {
     // per device: one set per caller stream (up to kAuxSets, then shared by
     // hash), so that callers on different streams fork onto different
-    // auxiliary streams and their fixed stages run concurrently on the GPU
+    // auxiliary streams and their second chains of signing rounds run
+    // concurrently on the GPU
     constexpr size_t kAuxSets = 16;
     struct PerDevice {
-        std::vector<std::pair<hipStream_t, AuxStreams *>> sets;
+        std::vector<std::pair<hipStream_t, AuxStream *>> sets;
     };
     static PerDevice per_dev[64];
     static std::mutex mu;
@@ -60,14 +61,12 @@ AuxStreams *aux_streams(hipStream_t caller) {
     for (auto &e : v)
         if (e.first == caller) return e.second;
     if (v.size() >= kAuxSets) return v[std::hash<void *>()(reinterpret_cast<void *>(caller)) % v.size()].second;
-    AuxStreams *a = new AuxStreams();
+    AuxStream *a = new AuxStream();
     // plain streams: with a hardware queue per auxiliary stream as well, ten
     // concurrent callers ran their signing calls 4x slower (too many queues)
-    bool ok = hipStreamCreateWithFlags(&a->s[0], hipStreamNonBlocking) == hipSuccess &&
-              hipStreamCreateWithFlags(&a->s[1], hipStreamNonBlocking) == hipSuccess &&
+    bool ok = hipStreamCreateWithFlags(&a->s, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreateWithFlags(&a->fork, hipEventDisableTiming) == hipSuccess &&
-              hipEventCreateWithFlags(&a->join[0], hipEventDisableTiming) == hipSuccess &&
-              hipEventCreateWithFlags(&a->join[1], hipEventDisableTiming) == hipSuccess;
+              hipEventCreateWithFlags(&a->join, hipEventDisableTiming) == hipSuccess;
     if (!ok) return nullptr;  // (a partly created set is not reused)
     v.emplace_back(caller, a);
     return a;

@@ -612,17 +612,17 @@ struct dil_sign_ctx {
     uint32_t *h_exec = nullptr, *d_exec = nullptr;
     uint8_t *h_done = nullptr, *d_done = nullptr;
     uint64_t *h_copy = nullptr, *d_copy = nullptr;
-    int slots_per_block = 0, blocks = 0, occupancy = 0;
+    int slots_per_block = 0, blocks = 0;  // of the persistent kernel
     // timing: the events (start, fixed stage of either chain of rounds done, loop done) of each timed call
     std::vector<hipEvent_t> ev;
     size_t timing_cap = 0, timed = 0;
     bool resident_only = false;  // rows without the per-item expanded arrays
-    int claim = 0;               // items owned per workgroup (0 = slots per workgroup)
+    int claim = 0;               // persistent kernel: items owned per workgroup (0 = its slots)
     bool profile = false;        // phase sums into d_head words 16..27
     bool row_mu = false;         // long messages: mu / rhoprime with one sponge per 16-lane row
 };
 
-// Resident keys: KeyLayout rows (pk, sk, tr, A, s1^, s2^, t0^, t1^).
+// Resident keys: KeyLayout rows (pk, sk, tr, A, int8 s2 / s1 / t0 limbs, t1^).
 struct dil_keystore {
     int mode = 0;
     size_t capacity = 0, pitch = 0;
@@ -679,7 +679,7 @@ static int sign_enqueue(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const
         if (ev && (e = (int)hipEventRecord(ev[0], st))) return e;
         if (engine == DIL_ENGINE_PERSTAGE) {
             // the per-stage scheduler launches the fixed part itself; the
-            // status word is cleared here (the persistent launch clears it)
+            // status word is cleared here (sign_call clears it otherwise)
             if ((e = launch_zero_ctl(c->d_head, nullptr, st))) return e;
             for (int k = 1; ev && k < 3; ++k)
                 if ((e = (int)hipEventRecord(ev[k], st))) return e;
@@ -805,7 +805,6 @@ int dil_sign_ctx_set_tiling(dil_sign_ctx *c, int slots_per_block, int occupancy,
     if (occupancy != 0 && (occupancy < 2 || occupancy > 4)) return DIL_EINVAL;
     if (slots_per_block > 0 && c->nslots / slots_per_block == 0) return DIL_ERANGE;
     c->slots_per_block = slots_per_block;
-    c->occupancy = occupancy;
     c->blocks = blocks < 0 ? 0 : blocks;
     return 0;
 }
@@ -905,8 +904,8 @@ int dil_sign_device(dil_sign_ctx *c, uint8_t *d_sig, size_t sig_pitch, const uin
 // A captured pipeline: every launch of one keygen / sign / verify call with
 // its arguments fixed, replayed by one hipGraphLaunch.  Capture runs on a
 // private stream in thread-local mode, so other threads' HIP calls do not
-// interfere; the fixed sign stage's fork/join over the auxiliary streams
-// becomes parallel branches of the graph.  No memset nodes are recorded
+// interfere; the second chain of signing rounds becomes a parallel branch of
+// the graph.  No memset nodes are recorded
 // (control words are cleared by a kernel).
 struct dil_graph {
     hipGraph_t graph = nullptr;

@@ -20,19 +20,18 @@ int device_cu_count();
 // blocks per CU.
 int default_grid_blocks(size_t units, int per_block, int blocks_per_cu = 8);
 
-// Two auxiliary streams (default priority, non-blocking) and fork/join
-// events of the current device for work forked from the caller's stream
-// `caller`, created on first use and kept until the process ends.  Each
+// An auxiliary stream (default priority, non-blocking) and fork/join events of
+// the current device for work forked from the caller's stream `caller`, created on first use and kept until the process ends.  Each
 // caller stream gets a set of its own (up to a cap, then sets are shared),
 // so forks from different streams do not queue behind each other.  A caller
 // holds `lock` while it enqueues a fork/join so that host threads sharing a
 // set cannot interleave their event records.
-struct AuxStreams {
-    hipStream_t s[2];
-    hipEvent_t fork, join[2];
+struct AuxStream {
+    hipStream_t s;
+    hipEvent_t fork, join;
     std::mutex lock;
 };
-AuxStreams *aux_streams(hipStream_t caller);
+AuxStream *aux_stream(hipStream_t caller);
 
 // Kernel tilings chosen at run time (set by the autotuner's cache through
 // dil_set_kernel_tiling): per (kind, mode, batch bucket) a value, 0 for the

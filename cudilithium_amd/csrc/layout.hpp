@@ -87,7 +87,7 @@ struct VerifyLayout {
     static constexpr size_t PK = align256(Z::SIG_BYTES);
     static constexpr size_t HASH = PK + align256(Z::PK_BYTES);  // mu | w1' packed
     static constexpr size_t CP = HASH + align256(Z::CHASH_IN_BYTES);  // challenge masks (64 B)
-    static constexpr size_t HINT = CP + 256;                          // K x 256 bits
+    static constexpr size_t HINT = CP + 256;                          // unused; the row's size is part of the interface
     static constexpr size_t FLAG = HINT + 256;                        // int32 status
     static constexpr size_t M = FLAG + 256;
     static size_t row(size_t mlen) { return M + align256(mlen); }

@@ -206,9 +206,6 @@ __device__ __forceinline__ void intt_wave(int32_t (&v)[4], int32_t *x, const Zet
 }
 
 // Converts between layouts through the exchange buffer (no arithmetic).
-__device__ __forceinline__ void layout_D_to_A(int32_t (&v)[4], int32_t *x) {
-    transpose(v, x, lane_id(), idx_D, idx_A);
-}
 __device__ __forceinline__ void layout_A_to_D(int32_t (&v)[4], int32_t *x) {
     transpose(v, x, lane_id(), idx_A, idx_D);
 }

@@ -54,8 +54,8 @@ struct VerifyArgs {
     const uint8_t *keys;
     size_t key_pitch;
     uint32_t nkeys;
-    // Long messages: tr and mu with one sponge per 16-lane row whatever the
-    // batch size.
+    // Long messages: tr and mu with one sponge per 16-lane row at least,
+    // whatever the batch size.
     int row_mu;
 };
 
@@ -72,7 +72,7 @@ struct Chain;
 
 int launch_keygen(int mode, const KeygenArgs &a, hipStream_t st);
 // Expands keys [0, n) of a key store (KeyLayout rows from `keys`): tr, A and
-// t1^ from the public key, and s1^, s2^, t0^ when with_sk.
+// t1^ from the public key, and the int8 limbs of s2, s1, t0 when with_sk.
 int launch_key_expand(int mode, uint8_t *keys, size_t key_pitch, size_t n, int with_sk, hipStream_t st);
 // ev: null, or four events recorded around vf_prep / vf_main / vf_final
 int launch_verify(int mode, const VerifyArgs &a, hipStream_t st, hipEvent_t *ev = nullptr);

@@ -9,8 +9,8 @@
 //   launch   when its group has waiting requests, take them in FIFO order,
 //            up to max_batch and the lane's message area, stage the inputs
 //            into the pinned buffer, copy them in one transfer, enqueue the
-//            group's pipeline (persistent sign with resident keys / resident
-//            verify / keygen) on the lane's stream, copy the outputs back in
+//            group's pipeline (sign with resident keys / resident verify /
+//            keygen) on the lane's stream, copy the outputs back in
 //            one transfer and record an event
 //   harvest  wait for the event (the thread sleeps until it signals), scatter the
 //            outputs into the requests (signature bytes, verdict, pk || sk),

@@ -7,7 +7,7 @@
 // round, full rounds written in place and tail rounds issued with several
 // consecutive nonces per item into temporary rows, the smallest successful
 // nonce per item winning (api.cu:218-441).  It is the baseline the
-// persistent engine (sign_persistent.hip) is measured against.
+// device-driven rounds (sign_rounds.hip) are measured against.
 #include <hip/hip_runtime.h>
 
 #include <vector>

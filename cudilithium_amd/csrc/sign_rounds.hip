@@ -449,26 +449,26 @@ int launch_round(const SignArgs &a, const SlotRef &sr, const Chain &ch, double &
 // destructor, so that buffers which the caller frees after draining its own
 // stream are not in use and a capture is left without a loose branch.
 struct ForkedStream {
-    AuxStreams *aux = nullptr;
+    AuxStream *aux = nullptr;
     hipStream_t st = nullptr;
     std::unique_lock<std::mutex> guard;
     bool open = false;
 
     int fork(hipStream_t caller) {
         st = caller;
-        if (!(aux = aux_streams(st))) return (int)hipErrorOutOfMemory;
+        if (!(aux = aux_stream(st))) return (int)hipErrorOutOfMemory;
         guard = std::unique_lock<std::mutex>(aux->lock);
         int e = (int)hipEventRecord(aux->fork, st);
-        if (!e) e = (int)hipStreamWaitEvent(aux->s[0], aux->fork, 0);
+        if (!e) e = (int)hipStreamWaitEvent(aux->s, aux->fork, 0);
         open = e == 0;
         return e;
     }
     int join() {
         if (!open) return 0;
         open = false;
-        int e = (int)hipEventRecord(aux->join[0], aux->s[0]);
-        if (!e) e = (int)hipStreamWaitEvent(st, aux->join[0], 0);
-        if (e) (void)hipStreamSynchronize(aux->s[0]);
+        int e = (int)hipEventRecord(aux->join, aux->s);
+        if (!e) e = (int)hipStreamWaitEvent(st, aux->join, 0);
+        if (e) (void)hipStreamSynchronize(aux->s);
         return e;
     }
     ~ForkedStream() { (void)join(); }
@@ -499,7 +499,7 @@ int sign_impl(const SignArgs &a, const SlotRef &sr, size_t nslots, const ChunkRe
         ch[k].target = (uint32_t)std::min<size_t>(ns, ROUND_TARGET / nchain);
         csr[k] = sr;
         csr[k].base += slot * sr.pitch;
-        cs[k] = k == 0 ? st : second.aux->s[0];
+        cs[k] = k == 0 ? st : second.aux->s;
         u[k] = (double)n;
         first += n;
         slot += ns;

@@ -1,15 +1,15 @@
-// Device-side stages of deterministic signing, shared by the per-stage
-// (one launch per stage, host-driven rejection rounds) form and the
-// persistent work-queue engine.
+// Device-side stages of deterministic signing, shared by the device-driven
+// rounds, the per-stage form (host-driven rejection rounds) and the persistent
+// kernel; hash_row.hpp has the hashes with more lanes each.
 //
 // Fixed part per item (api.cu:117-182):
-//   mu = SHAKE256(tr || m), rhoprime = SHAKE256(key || mu)   lane per item
-//   A = ExpandA(rho)                                         lane per entry
+//   mu = SHAKE256(tr || m), rhoprime = SHAKE256(key || mu)   lane pair, row or wave per item
+//   A = ExpandA(rho)                                         lane or wave per entry
 //   s2 | s1 and the limbs of t0 as int8 (unpack of sk)        lane per 8 coefficients
 // One attempt (item, nonce) in a "slot" (sign.cu:463-1196):
-//   y    lane per (slot, l)   raw ExpandMask squeeze of rhoprime || L*nonce+l
+//   y    per (slot, l)        raw ExpandMask squeeze of rhoprime || L*nonce+l
 //   w    wave per slot        NTT(y), A y^, INTT, caddq -> w; pack w1
-//   c    lane per slot        c~ = SHAKE256(mu || w1), c = SampleInBall(c~)
+//   c    per slot             c~ = SHAKE256(mu || w1), c = SampleInBall(c~)
 //   z    wave per slot        c s2, c s1, c t0 on the matrix cores
 //                             (ringmul.hpp), the norm checks, z = y + c s1,
 //                             MakeHint, pack z and h
@@ -48,8 +48,8 @@ struct SignArgs {
     // rnd + i * rnd_pitch instead of SHAKE256(key || mu) (api.cu:143-148).
     const uint8_t *rnd;
     size_t rnd_pitch;
-    // Long messages: mu / rhoprime with one sponge per 16-lane row
-    // (sg_mu_row_kernel) instead of one lane per item.
+    // Long messages: mu / rhoprime with one sponge per 16-lane row at least,
+    // whatever the batch size.
     int row_mu;
 };
 

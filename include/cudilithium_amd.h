@@ -83,7 +83,7 @@ typedef struct {
 #define DIL_POOL_SIGN_TEMP 2
 #define DIL_POOL_VERIFY 3
 
-#define DIL_ENGINE_PERSISTENT 0 /* device work queue, one persistent launch */
+#define DIL_ENGINE_PERSISTENT 0 /* rounds driven by the device, no host wait */
 #define DIL_ENGINE_PERSTAGE 1   /* one launch per stage, host-driven rounds */
 
 /* Minimum pitch of each pool row this library needs.  Each is at most the
@@ -118,11 +118,10 @@ int dil_crypto_sign_keypair(int mode, uint8_t *pk, uint8_t *sk, uint8_t *d_keypa
  * signatures of batch messages of mlen bytes (host, stride m_pitch) under
  * host secret keys; signatures to host `sig` with stride sig_pitch;
  * *siglen = CRYPTO_BYTES.  Per item the result is the attempt with the first
- * successful nonce, as in the reference.  This entry point runs the
- * persistent work-queue engine.  Attempt slots: the exec_threshold temp
- * rows when batch_size <= exec_threshold; otherwise up to batch_size slots,
- * each with its state in a sign-pool row and its candidate signature in the
- * temp pool read as one array.  batch_size <= 65536. */
+ * successful nonce, as in the reference.  This entry point runs
+ * device-driven rounds.  Attempt slots: the exec_threshold temp rows when
+ * batch_size <= exec_threshold; otherwise batch_size slots, each with its
+ * state in a sign-pool row.  batch_size <= 65536. */
 int dil_crypto_sign_signature(int mode, uint8_t *sig, size_t sig_pitch, size_t *siglen,
                               const uint8_t *m, size_t m_pitch, size_t mlen, const uint8_t *sk,
                               uint8_t *d_sign_mem_pool, size_t d_sign_mem_pool_pitch,
@@ -142,7 +141,7 @@ int dil_crypto_sign_signature_perstage(int mode, uint8_t *sig, size_t sig_pitch,
  * (api.cu:143-148): per item, rhoprime is 64 bytes drawn from the random
  * source (one draw of 64 * batch_size bytes, item i taking bytes
  * [64 i, 64 i + 64)) instead of SHAKE256(key || mu); otherwise the same
- * contract as dil_crypto_sign_signature (persistent engine).  Returns the
+ * contract as dil_crypto_sign_signature.  Returns the
  * random source's error, if it reports one, before any GPU work. */
 int dil_crypto_sign_signature_randomized(int mode, uint8_t *sig, size_t sig_pitch, size_t *siglen,
                                          const uint8_t *m, size_t m_pitch, size_t mlen,
@@ -218,12 +217,13 @@ int dil_verify_device(int mode, int32_t *d_ret, const uint8_t *d_sig, size_t sig
                       const uint8_t *d_pk, size_t pk_pitch, const uint8_t *d_msg,
                       const uint64_t *d_moff, const uint32_t *d_mlen, size_t n, uint8_t *d_work,
                       size_t work_pitch, void *stream);
-/* Message hashing of the verify / sign calls below: by default one lane
- * absorbs a message serially (one SHAKE256 permutation per 136 bytes, the
- * throughput form).  DIL_HASH_LONG_MESSAGES gives each message a 16-lane
- * row of ten active lanes instead, which shortens the serial chain about
- * 2.5 times at more instructions per message: for batches whose latency
- * is set by long messages.  Results are identical. */
+/* Message hashing of the verify / sign calls below: a message is absorbed
+ * serially (one SHAKE256 permutation per 136 bytes) by a wave in the smallest
+ * batches, a 16-lane row up to 4,096 items (signing 8,192) and a pair of lanes
+ * beyond, the throughput form.  DIL_HASH_LONG_MESSAGES keeps the row for the
+ * largest batches too, whose chain is 1.7 times as short as the pair's at more
+ * instructions per message: for batches whose latency is set by long messages.
+ * Results are identical. */
 #define DIL_HASH_LONG_MESSAGES 1
 int dil_verify_device_ex(int mode, int32_t *d_ret, const uint8_t *d_sig, size_t sig_pitch,
                          const uint8_t *d_pk, size_t pk_pitch, const uint8_t *d_msg,
@@ -258,8 +258,8 @@ int dil_verify_device_timed(int mode, int32_t *d_ret, const uint8_t *d_sig, size
  * buckets) a value, 0 restoring the compiled default.  Kinds: keys per
  * workgroup of keygen's main kernel (checked and kept, but without effect: a
  * wave takes a fixed number of keys) and items per workgroup of verify's with
- * resident keys (2, 4, 8 or 16 where its LDS fits: defaults 16 / 8 / 4 for
- * modes 2 / 3 / 5), wavefronts per workgroup of the standalone NTT (2, 4 or 8; default 4; mode
+ * resident keys (2, 4, 8 or, mode 2, 16; defaults 16 / 8 / 4 for modes 2 / 3 /
+ * 5), wavefronts per workgroup of the standalone NTT (2, 4 or 8; default 4; mode
  * ignored).  Process-wide; results never depend on them.  DIL_EINVAL for a
  * value the kernels are not built for. */
 #define DIL_TILE_KEYGEN_ITEMS 0
@@ -286,11 +286,11 @@ int dil_sign_ctx_destroy(dil_sign_ctx *ctx);
 /* Signing runs in device-driven rounds that choose their own launch shapes;
  * the two tilings below concern the persistent kernel, which runs alone for
  * calls with more than 32 items per slot and for the phase profile.
- * Tiling: slots per workgroup (0 = automatic, or 1, 8, 16,
- * 32), register budget as waves per SIMD (0 = automatic, or 2, 3, 4) and
- * workgroup count (0 = nslots / slots_per_block). */
+ * Tiling: slots per workgroup (0 = automatic, or 1, 8, 16, 32), workgroup count
+ * (0 = nslots / slots_per_block) and occupancy (0, 2, 3 or 4), which has no
+ * effect: the kernel is built for one register budget. */
 int dil_sign_ctx_set_tiling(dil_sign_ctx *ctx, int slots_per_block, int occupancy, int blocks);
-/* Persistent engine: at most items_per_block items owned by a workgroup at a
+/* Persistent kernel: at most items_per_block items owned by a workgroup at a
  * time (0 = slots per workgroup).  Below that, each owned item gets several
  * slots (consecutive nonces) per round, so small batches finish in fewer
  * rounds at the price of speculative attempts; results are unchanged.
@@ -308,26 +308,26 @@ int dil_sign_ctx_timed_calls(dil_sign_ctx *ctx);
 int dil_sign_ctx_timing(dil_sign_ctx *ctx, int call, float *fixed_ms, float *loop_ms);
 /* Deterministic signatures of n messages (per-item lengths) under n secret
  * keys, all in device memory; engine DIL_ENGINE_PERSISTENT or
- * DIL_ENGINE_PERSTAGE (n <= 65536).  Asynchronous for the persistent engine;
+ * DIL_ENGINE_PERSTAGE (n <= 65536).  Asynchronous for the first;
  * the per-stage engine synchronises `stream` once per rejection round. */
 int dil_sign_device(dil_sign_ctx *ctx, uint8_t *d_sig, size_t sig_pitch, const uint8_t *d_sk,
                     size_t sk_pitch, const uint8_t *d_msg, const uint64_t *d_moff,
                     const uint32_t *d_mlen, size_t n, int engine, void *stream);
-/* After a persistent-engine call: per item, the number of attempts the
+/* After a DIL_ENGINE_PERSISTENT call: per item, the number of attempts the
  * sequential specification makes (winning nonce + 1), copied to host and
  * synchronised on `stream`. */
 int dil_sign_ctx_attempt_counts(dil_sign_ctx *ctx, uint32_t *h_counts, size_t n, void *stream);
 /* Status of the last call (synchronises `stream`): 0, or a combination of
- * DIL_SIGN_STATUS_ROUND_CAP (a persistent workgroup stopped at its round
- * limit; never expected; the batch's signatures are then incomplete) and
+ * DIL_SIGN_STATUS_ROUND_CAP (a persistent workgroup ran 20,000 rounds
+ * without a signature; never expected; the batch's signatures are then incomplete) and
  * DIL_SIGN_STATUS_NO_SECRET (resident signing: an item's key is verify-only). */
 #define DIL_SIGN_STATUS_ROUND_CAP 1
 #define DIL_SIGN_STATUS_NO_SECRET 2
 int dil_sign_ctx_status(dil_sign_ctx *ctx, int *status, void *stream);
-/* Attempts the last persistent-engine call executed, speculative ones
+/* Attempts the last DIL_ENGINE_PERSISTENT call executed, speculative ones
  * included (synchronises `stream`). */
 int dil_sign_ctx_executed_attempts(dil_sign_ctx *ctx, uint64_t *count, void *stream);
-/* Phase profile of the persistent engine (for tuning): when enabled, each
+/* Phase profile of the persistent kernel: when enabled, calls run it alone, each
  * workgroup sums shader-clock cycles spent in its six phases (assign, y, w,
  * c, z, commit) and the sums over workgroups of the last call are returned by
  * dil_sign_ctx_phase_cycles (synchronises `stream`).  Off by default. */
@@ -411,8 +411,8 @@ int dil_sign_device_randomized(dil_sign_ctx *ctx, const dil_keystore *ks, const 
  * graph; dil_graph_launch replays it on `stream` (one hipGraphLaunch).
  * Buffers named at creation must stay allocated while the graph exists;
  * replays of graphs sharing buffers (the same sign context, work rows or
- * outputs) must not overlap in time.  Sign graphs use the persistent
- * engine with the context's tiling at creation. */
+ * outputs) must not overlap in time.  Sign graphs use
+ * DIL_ENGINE_PERSISTENT with the context's settings at creation. */
 typedef struct dil_graph dil_graph;
 int dil_sign_graph_create(dil_graph **graph, dil_sign_ctx *ctx, uint8_t *d_sig, size_t sig_pitch,
                           const uint8_t *d_sk, size_t sk_pitch, const uint8_t *d_msg,
