@@ -115,7 +115,6 @@ struct Lane {
     dil_sign_ctx *ctx = nullptr;  // sign lanes
     std::vector<dil_request *> reqs;
     uint32_t batch_id = 0;
-    bool backlog = false;  // requests of the group were still waiting after fill()
     std::condition_variable *cv = nullptr;  // woken when its queue gets work
 };
 
@@ -208,7 +207,6 @@ bool dil_server::fill(Lane &ln) {
         dq.pop_front();
     }
     npending -= ln.reqs.size();
-    ln.backlog = !dq.empty();
     ln.batch_id = next_batch++;
     ++batches;
     by_op[ln.op] += ln.reqs.size();
@@ -250,18 +248,6 @@ int dil_server::enqueue(Lane &ln) {
     const uint32_t *d_mlen = reinterpret_cast<const uint32_t *>(ln.d_in + L.mlen);
     const uint8_t *d_msg = ln.d_in + L.msgs, *d_pay = ln.d_in + L.payload;
     if (ln.op == DIL_OP_SIGN) {
-        // small batches: fewer slots per workgroup.  Without a backlog the
-        // batch is spread over all workgroups, so that each item gets
-        // spb / claim nonces per round and finishes in fewer rounds (latency);
-        // with one, every slot is a distinct item's attempt (throughput).
-        int spb = n >= 8192 ? 32 : (n >= 2048 ? 16 : 8);
-        if ((size_t)spb > cfg.max_batch) spb = 1;
-        if ((e = dil_sign_ctx_set_tiling(ln.ctx, spb, 0, 0))) return e;
-        const size_t blocks = cfg.max_batch / (size_t)spb;
-        const int claim = ln.backlog ? spb
-                                     : (int)std::min<size_t>((size_t)spb,
-                                                             std::max<size_t>(1, (n + blocks - 1) / blocks));
-        if ((e = dil_sign_ctx_set_claim(ln.ctx, claim))) return e;
         e = dil_sign_device_resident(ln.ctx, ks[ms], d_idx, ln.d_out, sigb, d_msg, d_moff, d_mlen, n,
                                      DIL_ENGINE_PERSISTENT, ln.st);
     } else if (ln.op == DIL_OP_VERIFY) {
