@@ -27,7 +27,8 @@
 // A chained permutation takes 2.2 us on MI355X while a SIMD has one such wave
 // (row form 3.5, lane pair 5.9, lane 8.6); 1,024 / 2,048 / 3,072 / 4,096 states
 // on the card take 2.6 / 3.2 / 4.1 / 5.0 us, where the row form takes 3.5 to
-// 3.9 us up to 4,096: the wave form is for up to about 2,048 states.
+// 3.9 us up to 4,096: the wave form is for up to 2,000 states, or 3,000 where the
+// work around the hash gains from whole waves too.
 //
 // All 64 lanes must execute every call.  The round constants and rotation
 // offsets are those of keccak.hpp.
